@@ -6,6 +6,8 @@
 // shuffles and a fixed-order combine of its 4 waves; a single block then sums the
 // per-block partials in a fixed order.  No floating-point atomics, so the result is
 // bitwise reproducible for a given n and launch shape.
+#include <algorithm>
+#include <map>
 #include <mutex>
 
 #include "field.hpp"
@@ -240,66 +242,124 @@ __global__ __launch_bounds__(kTPB) void k_bin_finish(uint32_t nbins, const uint3
 
 // Transverse structure factor at a list of mesh wave-vectors k:
 //   out[g][k] = sum_{i in g} (S_a(i) ua_i + i S_b(i) ub_i) exp(-2 pi i sum_d k_d x_d(i) / N_d).
-// The spins of each group are cut into chunks of kSqChunk; a block stages one chunk's
-// (c_i, mesh position) in LDS and each thread accumulates one k over it in FP64; a second
-// pass adds the chunks of each group in order.  Phase: frac(sum_d k_d x_d / N_d) in FP64,
-// then sincospi(2 frac).
-constexpr uint32_t kSqChunk = 512;
+// The phase splits over the axes, so the sum is taken in two passes: along one axis d (chosen
+// by set_sq) the spins of each mesh plane x_d = const are summed first, once per distinct pair
+// of the other two wave-vector components (a "projection" p), then out[g][k] is the sum of the
+// planes' values at p(k) times exp(-2 pi i k_d x_d / N_d).  A line of wave-vectors (q, 0, 0),
+// which spin-wave runs sample, has one projection with no phase: n complex additions instead
+// of n nk phase evaluations.  The planes are cut into chunks of at most kSqChunk spins, one
+// block each (4 spins a thread, kept in registers over the projections); partial sums are
+// combined in a fixed order.  Phases: (k x mod N) / N exactly in FP64 (products below 2^53),
+// then sincospi.
+// Bound by latency (262,144 spins read 1 MB of rows and 2 MB of spins).  64^3 spins, 33
+// wave-vectors (q, 0, 0), trace durations: 90 + 125 us for the two passes with one sincospi per
+// (spin, k) and one thread per k in the second; 5.1 + 3.8 us here.
+constexpr uint32_t kSqChunk = 1024;
+constexpr uint32_t kSqTile = 32;  // projections a block takes per pass over its registers
 
 struct SqArgs {
-    uint32_t n, nk, axis;
-    double inv[3];             // 1 / N_d
-    const uint4* spin;         // {device row, x, y, z} per listed spin
-    const double2* w;          // (ua, ub)
+    uint32_t n, nk, np, axis;
+    double nu, nv, nd;         // mesh extents along the two projected axes and the plane axis
+    const uint32_t* row;       // device row per listed spin
+    const uint2* uv;           // mesh coordinates along the two projected axes
+    const double2* w;          // (ua, ub) or null
     const uint32_t* cs;        // chunk starts [nch + 1]
-    const uint32_t* kp;        // [nk][3]
+    const uint32_t* cx;        // plane coordinate of each chunk
+    const uint32_t* cg;        // first chunk of each group [ngroups + 1]
+    const uint2* proj;         // [np] wave-vector components along the projected axes
+    const uint2* kp;           // [nk] {projection, component along the plane axis}
 };
+
+// k x / N modulo 1, k and x below N
+__device__ __forceinline__ double sq_turns(double k, double x, double N) {
+    const double t = k * x;
+    double r = t - floor(t / N) * N;
+    if (r < 0.0) r += N;
+    if (r >= N) r -= N;
+    return r / N;
+}
 
 template <class SpinT>
 __global__ __launch_bounds__(kTPB) void k_sq_partial(SqArgs a, const SpinT* __restrict__ S, double* __restrict__ part) {
-    __shared__ double sre[kSqChunk], sim[kSqChunk], px[kSqChunk], py[kSqChunk], pz[kSqChunk];
+    constexpr uint32_t SPT = kSqChunk / kTPB, NW = kTPB / 64;
+    __shared__ double2 lds[kSqTile][NW];
     const uint32_t ch = blockIdx.x, b = a.cs[ch], e = a.cs[ch + 1];
     const uint32_t ca = a.axis == 0 ? 1u : 0u, cb = a.axis == 2 ? 1u : 2u;
-    for (uint32_t q = b + threadIdx.x; q < e; q += kTPB) {
-        const uint4 sp = a.spin[q];
-        const double2 w = a.w[q];
-        const uint32_t l = q - b;
-        sre[l] = (double)S[(size_t)ca * a.n + sp.x] * w.x;
-        sim[l] = (double)S[(size_t)cb * a.n + sp.x] * w.y;
-        px[l] = (double)sp.y * a.inv[0];
-        py[l] = (double)sp.z * a.inv[1];
-        pz[l] = (double)sp.w * a.inv[2];
+    double re[SPT], im[SPT];
+    uint2 x[SPT];
+#pragma unroll
+    for (uint32_t j = 0; j < SPT; ++j) {
+        const uint32_t q = b + j * kTPB + threadIdx.x;
+        re[j] = im[j] = 0.0;
+        x[j] = make_uint2(0u, 0u);
+        if (q < e) {
+            const uint32_t i = a.row[q];
+            const double2 w = a.w ? a.w[q] : make_double2(1.0, 1.0);
+            re[j] = (double)S[(size_t)ca * a.n + i] * w.x;
+            im[j] = (double)S[(size_t)cb * a.n + i] * w.y;
+            x[j] = a.uv[q];
+        }
     }
-    __syncthreads();
-    const uint32_t k = blockIdx.y * kTPB + threadIdx.x;
-    if (k >= a.nk) return;
-    const double kx = a.kp[3 * k], ky = a.kp[3 * k + 1], kz = a.kp[3 * k + 2];
-    double re = 0.0, im = 0.0;
-    for (uint32_t l = 0; l < e - b; ++l) {
-        double t = kx * px[l] + ky * py[l] + kz * pz[l];
-        t -= floor(t);
-        double sn, cn;
-        sincospi(2.0 * t, &sn, &cn);
-        // (c_re + i c_im)(cos - i sin)
-        re += sre[l] * cn + sim[l] * sn;
-        im += sim[l] * cn - sre[l] * sn;
+    for (uint32_t p0 = blockIdx.y * kSqTile; p0 < a.np; p0 += gridDim.y * kSqTile) {
+        const uint32_t p1 = p0 + kSqTile < a.np ? p0 + kSqTile : a.np;
+        for (uint32_t p = p0; p < p1; ++p) {
+            const uint2 k = a.proj[p];
+            double sr = 0.0, si = 0.0;
+            if ((k.x | k.y) == 0u) {
+#pragma unroll
+                for (uint32_t j = 0; j < SPT; ++j) {
+                    sr += re[j];
+                    si += im[j];
+                }
+            } else {
+#pragma unroll
+                for (uint32_t j = 0; j < SPT; ++j) {
+                    const double t = sq_turns(k.x, x[j].x, a.nu) + sq_turns(k.y, x[j].y, a.nv);
+                    double sn, cn;
+                    sincospi(2.0 * (t - floor(t)), &sn, &cn);
+                    // (c_re + i c_im)(cos - i sin)
+                    sr += re[j] * cn + im[j] * sn;
+                    si += im[j] * cn - re[j] * sn;
+                }
+            }
+            sr = wave_sum(sr);
+            si = wave_sum(si);
+            if ((threadIdx.x & 63u) == 0) lds[p - p0][threadIdx.x >> 6] = make_double2(sr, si);
+        }
+        __syncthreads();
+        if (threadIdx.x < p1 - p0) {
+            double2 v = lds[threadIdx.x][0];
+            for (uint32_t w = 1; w < NW; ++w) {
+                v.x += lds[threadIdx.x][w].x;
+                v.y += lds[threadIdx.x][w].y;
+            }
+            reinterpret_cast<double2*>(part)[(size_t)ch * a.np + p0 + threadIdx.x] = v;
+        }
+        __syncthreads();
     }
-    part[((size_t)ch * a.nk + k) * 2] = re;
-    part[((size_t)ch * a.nk + k) * 2 + 1] = im;
 }
 
-__global__ __launch_bounds__(kTPB) void k_sq_finish(uint32_t ngroups, uint32_t nk, const uint32_t* __restrict__ cg,
-                                                    const double* __restrict__ part, double* __restrict__ out) {
-    const uint32_t v = blockIdx.x * kTPB + threadIdx.x;
-    if (v >= ngroups * nk) return;
-    const uint32_t g = v / nk, k = v % nk;
+// One wave per (group, wave-vector): its lanes take the group's chunks in a stride.
+__global__ __launch_bounds__(kTPB) void k_sq_finish(SqArgs a, uint32_t ngroups, const double* __restrict__ part,
+                                                     double* __restrict__ out) {
+    const uint32_t v = blockIdx.x * (kTPB / 64) + (threadIdx.x >> 6), lane = threadIdx.x & 63u;
+    if (v >= ngroups * a.nk) return;
+    const uint32_t g = v / a.nk;
+    const uint2 k = a.kp[v % a.nk];
     double re = 0.0, im = 0.0;
-    for (uint32_t ch = cg[g]; ch < cg[g + 1]; ++ch) {
-        re += part[((size_t)ch * nk + k) * 2];
-        im += part[((size_t)ch * nk + k) * 2 + 1];
+    for (uint32_t ch = a.cg[g] + lane; ch < a.cg[g + 1]; ch += 64u) {
+        const double2 c = reinterpret_cast<const double2*>(part)[(size_t)ch * a.np + k.x];
+        double sn, cn;
+        sincospi(2.0 * sq_turns(k.y, a.cx[ch], a.nd), &sn, &cn);
+        re += c.x * cn + c.y * sn;
+        im += c.y * cn - c.x * sn;
     }
-    out[(size_t)v * 2] = re;
-    out[(size_t)v * 2 + 1] = im;
+    re = wave_sum(re);
+    im = wave_sum(im);
+    if (lane == 0) {
+        out[(size_t)v * 2] = re;
+        out[(size_t)v * 2 + 1] = im;
+    }
 }
 
 // ---------------------------------------------------------------- host launchers
@@ -535,72 +595,113 @@ int reduce_bins(llg_ctx* c, double* dev_out) {
 int set_sq(llg_ctx* c, const uint32_t grid[3], const uint32_t* mesh, uint32_t nk, const uint32_t* kpts, int axis,
            const double* ua, const double* ub, uint32_t ngroups, const uint32_t* group) {
     const uint32_t n = c->n;
-    std::vector<uint32_t> cnt(ngroups + 1, 0);
-    for (uint32_t i = 0; i < n; ++i) {
-        const uint32_t g = group ? group[i] : 0u;
-        if (g < ngroups) ++cnt[g + 1];
+    // The plane axis: the one with the least work, (spins x projections) in the first pass and
+    // (planes x wave-vectors) in the second.  Projections: the distinct pairs of the other two
+    // wave-vector components.
+    const int ax[3][3] = {{0, 1, 2}, {1, 0, 2}, {2, 0, 1}};  // plane axis, projected axes
+    int d = 0;
+    std::vector<uint2> kp(nk), proj;
+    double best = 0.0;
+    for (int t = 0; t < 3; ++t) {
+        std::map<std::pair<uint32_t, uint32_t>, uint32_t> seen;
+        std::vector<uint2> kq(nk), pr;
+        for (uint32_t k = 0; k < nk; ++k) {
+            const uint32_t* q = kpts + 3 * (size_t)k;
+            const auto it = seen.emplace(std::make_pair(q[ax[t][1]], q[ax[t][2]]), (uint32_t)pr.size());
+            if (it.second) pr.push_back(make_uint2(q[ax[t][1]], q[ax[t][2]]));
+            kq[k] = make_uint2(it.first->second, q[ax[t][0]]);
+        }
+        const double planes = (double)std::min<uint64_t>(n, (uint64_t)ngroups * grid[ax[t][0]]) + (double)n / kSqChunk;
+        const double cost = (double)n * pr.size() + planes * ((double)nk + (double)kTPB * pr.size());
+        if (t == 0 || cost < best) {
+            best = cost;
+            d = t;
+            kp.swap(kq);
+            proj.swap(pr);
+        }
     }
-    for (uint32_t g = 0; g < ngroups; ++g) cnt[g + 1] += cnt[g];
-    std::vector<uint4> sp(std::max<uint32_t>(1, cnt[ngroups]));
-    std::vector<double2> w(sp.size());
-    std::vector<uint32_t> fill(cnt.begin(), cnt.end() - 1);
-    for (uint32_t d = 0; d < n; ++d) {
-        const uint32_t i = c->perm.to_ref(d);
-        const uint32_t g = group ? group[i] : 0u;
-        if (g >= ngroups) continue;
-        const uint32_t q = fill[g]++;
-        sp[q] = make_uint4(d, mesh[3 * (size_t)i], mesh[3 * (size_t)i + 1], mesh[3 * (size_t)i + 2]);
-        w[q] = make_double2(ua ? ua[i] : 1.0, ub ? ub[i] : 1.0);
+    // listed spins by (group, plane), ascending device row within a plane
+    std::vector<std::pair<uint64_t, uint32_t>> list;
+    list.reserve(n);
+    for (uint32_t r = 0; r < n; ++r) {
+        const uint32_t i = c->perm.to_ref(r), g = group ? group[i] : 0u;
+        if (g < ngroups) list.emplace_back(((uint64_t)g << 32) | mesh[3 * (size_t)i + ax[d][0]], r);
     }
-    std::vector<uint32_t> cs(1, 0), cg(ngroups + 1, 0);
-    for (uint32_t g = 0; g < ngroups; ++g) {
-        cg[g] = (uint32_t)cs.size() - 1;
-        for (uint32_t q = cnt[g]; q < cnt[g + 1]; q += kSqChunk) cs.push_back(std::min(cnt[g + 1], q + kSqChunk));
+    if (!std::is_sorted(list.begin(), list.end())) std::sort(list.begin(), list.end());
+    const bool weighted = ua || ub;
+    std::vector<uint32_t> row(std::max<size_t>(1, list.size()));
+    std::vector<uint2> uv(row.size());
+    std::vector<double2> w(weighted ? row.size() : 0);
+    std::vector<uint32_t> cs(1, 0), cx, cg(ngroups + 1, 0);
+    for (size_t q = 0; q < list.size(); ++q) {
+        const uint32_t r = list[q].second, i = c->perm.to_ref(r);
+        row[q] = r;
+        uv[q] = make_uint2(mesh[3 * (size_t)i + ax[d][1]], mesh[3 * (size_t)i + ax[d][2]]);
+        if (weighted) w[q] = make_double2(ua ? ua[i] : 1.0, ub ? ub[i] : 1.0);
+        if (q + 1 == list.size() || list[q + 1].first != list[q].first || q + 1 - cs.back() == kSqChunk) {
+            cs.push_back((uint32_t)q + 1);
+            cx.push_back((uint32_t)list[q].first);
+            cg[(list[q].first >> 32) + 1] = (uint32_t)cx.size();  // end of the group's chunks so far
+        }
     }
-    cg[ngroups] = (uint32_t)cs.size() - 1;
-    const uint32_t nch = (uint32_t)cs.size() - 1;
-    auto up = [&](DevBuf& d, const void* h, size_t bytes) -> int {
-        SLLG_TRY(d.alloc(std::max<size_t>(bytes, 8)));
-        if (bytes) SLLG_HIP(hipMemcpyAsync(d.p, h, bytes, hipMemcpyHostToDevice, c->stream));
+    for (uint32_t g = 0; g < ngroups; ++g) cg[g + 1] = std::max(cg[g + 1], cg[g]);  // groups without spins
+    const uint32_t nch = (uint32_t)cx.size();
+    auto up = [&](DevBuf& b, const void* h, size_t bytes) -> int {
+        SLLG_TRY(b.alloc(std::max<size_t>(bytes, 8)));
+        if (bytes) SLLG_HIP(hipMemcpyAsync(b.p, h, bytes, hipMemcpyHostToDevice, c->stream));
         return 0;
     };
-    SLLG_TRY(up(c->sq_spin, sp.data(), sp.size() * sizeof(uint4)));
-    SLLG_TRY(up(c->sq_w, w.data(), w.size() * sizeof(double2)));
+    SLLG_TRY(up(c->sq_row, row.data(), row.size() * 4));
+    SLLG_TRY(up(c->sq_uv, uv.data(), uv.size() * sizeof(uint2)));
+    if (weighted)
+        SLLG_TRY(up(c->sq_w, w.data(), w.size() * sizeof(double2)));
+    else
+        c->sq_w.release();
     SLLG_TRY(up(c->sq_cs, cs.data(), cs.size() * 4));
+    SLLG_TRY(up(c->sq_cx, cx.data(), cx.size() * 4));
     SLLG_TRY(up(c->sq_cg, cg.data(), cg.size() * 4));
-    SLLG_TRY(up(c->sq_k, kpts, (size_t)nk * 3 * 4));
-    SLLG_TRY(c->sq_part.alloc(std::max<size_t>(1, (size_t)nch * nk) * 2 * sizeof(double)));
+    SLLG_TRY(up(c->sq_proj, proj.data(), proj.size() * sizeof(uint2)));
+    SLLG_TRY(up(c->sq_k, kp.data(), kp.size() * sizeof(uint2)));
+    SLLG_TRY(c->sq_part.alloc(std::max<size_t>(1, (size_t)nch * proj.size()) * 2 * sizeof(double)));
     SLLG_HIP(hipStreamSynchronize(c->stream));
     c->sq_nk = nk;
+    c->sq_np = (uint32_t)proj.size();
     c->sq_ngroups = ngroups;
     c->sq_nch = nch;
     c->sq_axis = axis;
-    for (int d = 0; d < 3; ++d) c->sq_grid[d] = grid[d];
+    for (int a = 0; a < 3; ++a) c->sq_grid[a] = grid[ax[d][a]];
     return 0;
 }
 
 int sample_sq(llg_ctx* c, double* dev_out) {
     SLLG_TRY(sync_spins(c));
     if (c->sq_nk == 0 || c->sq_ngroups == 0) return 0;
+    SqArgs a{};
+    a.n = c->n;
+    a.nk = c->sq_nk;
+    a.np = c->sq_np;
+    a.axis = (uint32_t)c->sq_axis;
+    a.nd = (double)c->sq_grid[0];
+    a.nu = (double)c->sq_grid[1];
+    a.nv = (double)c->sq_grid[2];
+    a.row = c->sq_row.as<uint32_t>();
+    a.uv = c->sq_uv.as<uint2>();
+    a.w = c->sq_w.as<double2>();
+    a.cs = c->sq_cs.as<uint32_t>();
+    a.cx = c->sq_cx.as<uint32_t>();
+    a.cg = c->sq_cg.as<uint32_t>();
+    a.proj = c->sq_proj.as<uint2>();
+    a.kp = c->sq_k.as<uint2>();
     if (c->sq_nch) {
-        SqArgs a{};
-        a.n = c->n;
-        a.nk = c->sq_nk;
-        a.axis = (uint32_t)c->sq_axis;
-        for (int d = 0; d < 3; ++d) a.inv[d] = 1.0 / (double)c->sq_grid[d];
-        a.spin = c->sq_spin.as<uint4>();
-        a.w = c->sq_w.as<double2>();
-        a.cs = c->sq_cs.as<uint32_t>();
-        a.kp = c->sq_k.as<uint32_t>();
-        const dim3 grid(c->sq_nch, blocks_for(c->sq_nk, kTPB));
+        const dim3 grid(c->sq_nch, std::min(blocks_for(a.np, kSqTile), 65535u));
         if (c->prec == LLG_FP64_PLAIN)
             k_sq_partial<double><<<grid, kTPB, 0, c->stream>>>(a, c->S.as<double>(), c->sq_part.as<double>());
         else
             k_sq_partial<float><<<grid, kTPB, 0, c->stream>>>(a, c->S.as<float>(), c->sq_part.as<double>());
         SLLG_HIP(hipGetLastError());
     }
-    k_sq_finish<<<blocks_for(c->sq_ngroups * c->sq_nk, kTPB), kTPB, 0, c->stream>>>(
-        c->sq_ngroups, c->sq_nk, c->sq_cg.as<uint32_t>(), c->sq_part.as<double>(), dev_out);
+    k_sq_finish<<<blocks_for((size_t)c->sq_ngroups * c->sq_nk, kTPB / 64), kTPB, 0, c->stream>>>(
+        a, c->sq_ngroups, c->sq_part.as<double>(), dev_out);
     SLLG_HIP(hipGetLastError());
     return 0;
 }
