@@ -192,10 +192,7 @@ int step_plain(llg_ctx* c, uint64_t t) {
 }
 
 int step_fused(llg_ctx* c, uint64_t t) {
-    if (c->dip && t % c->dip_refresh == 0) {
-        SLLG_TRY(sync_spins(c));
-        SLLG_TIMED("dipolar_refresh", dipolar_refresh(c, c->S.p, c->DEM.p));
-    }
+    if (c->dip && t % c->dip_refresh == 0) SLLG_TIMED("dipolar_refresh", dipolar_refresh_spins(c));
     StepSched s{t, nullptr};
     SLLG_TRY(take_noise(c, &s.xi));
     if (c->scheme == LLG_HEUN) {

@@ -33,6 +33,7 @@
 #include <mutex>
 #include <vector>
 
+#include "conv.hpp"
 #include "kernels.hpp"
 
 namespace sllg {
@@ -69,6 +70,9 @@ struct DipolarPlan {
     bool yz = false, yz_dense = false;  // yz_dense: the map below is the identity
     DevBuf map;       // [species][x][y][z] over the physical extents: device spin or ~0
     DevBuf twy, twz;  // exp(-2 pi i m / Gy), m < Gy / 2; exp(-2 pi i m / Gz), m < Gz
+    // FP32, mirror-symmetric kernel, small mesh: the register-transform convolution (k_conv.hip)
+    // in place of everything above
+    std::unique_ptr<ConvPlan> conv;
     ~DipolarPlan() {
         if (have_fwd) hipfftDestroy(fwd);
         if (have_inv) hipfftDestroy(inv);
@@ -909,6 +913,11 @@ int dipolar_create(llg_ctx* c, const llg_dipolar& d, const uint32_t* spin_specie
     }
     p->P = (size_t)p->G[0] * p->G[1] * p->G[2];
     p->Ph = (size_t)p->G[0] * p->G[1] * (p->G[2] / 2 + 1);
+    if (conv_applies(c, d, fx)) {
+        p->general = fx != nullptr;
+        p->conv.reset(new ConvPlan());
+        return conv_create(c, *p->conv, d, spin_species, fx, dip_terms);
+    }
     if (fx) return fftexch_create(c, p, d, spin_species, *fx, dip_terms);
     const uint32_t n = c->n;
     // grid point of each spin, indexed in the handle's device order; one spin per point (two
@@ -1052,9 +1061,9 @@ int dipolar_set_stream(llg_ctx* c) {
 
 bool dipolar_is_exchange(const llg_ctx* c) { return c->dplan && c->dplan->general; }
 
-// The FP32 half-grid plane path runs only kernels of this file (no hipFFT plans, no memsets),
-// so a stream capture of a refresh replays exactly.
-bool dipolar_capturable(const llg_ctx* c) { return c->dplan && !c->dplan->f64 && c->dplan->yz; }
+// The FP32 register-transform and half-grid plane paths run only this library's kernels (no
+// hipFFT plans, no memsets), so a stream capture of a refresh replays exactly.
+bool dipolar_capturable(const llg_ctx* c) { return c->dplan && !c->dplan->f64 && (c->dplan->conv || c->dplan->yz); }
 
 void dipolar_destroy(llg_ctx* c) {
     delete c->dplan;
@@ -1064,6 +1073,7 @@ void dipolar_destroy(llg_ctx* c) {
 uint64_t dipolar_bytes(const llg_ctx* c) {
     const DipolarPlan* p = c->dplan;
     if (!p) return 0;
+    if (p->conv) return p->conv->bytes();
     uint64_t b = p->lin.bytes + p->mu.bytes + p->grid.bytes + p->spec.bytes + p->hgrid.bytes + p->sp.bytes +
                  p->Nkc.bytes + p->hspec.bytes + p->tw.bytes + p->map.bytes + p->twy.bytes + p->twz.bytes +
                  (p->Nk ? p->Nk->bytes : 0) +
@@ -1077,6 +1087,7 @@ uint64_t dipolar_bytes(const llg_ctx* c) {
 int dipolar_refresh(llg_ctx* c, const void* S, void* out) {
     DipolarPlan* p = c->dplan;
     if (!p) SLLG_FAIL(LLG_E_STATE, "dipolar plan missing");
+    if (p->conv) return conv_apply(c, *p->conv, (const float*)S, false, (float*)out);
     const uint32_t n = c->n;
     const dim3 gn(blocks_for(n, kTPB)), gk(blocks_for(p->Ph, kTPB)), b(kTPB);
     if (p->general) {
@@ -1165,6 +1176,15 @@ int dipolar_refresh(llg_ctx* c, const void* S, void* out) {
     }
     SLLG_HIP(hipGetLastError());
     return 0;
+}
+
+// FP32: refresh at the current spins.  The register-transform path reads them from their AoS3
+// copy when only that is current; the others from the SoA spins, rebuilt first.
+int dipolar_refresh_spins(llg_ctx* c) {
+    const DipolarPlan* p = c->dplan;
+    if (p && p->conv && !c->s_soa_valid) return conv_apply(c, *p->conv, c->S3.as<float>(), true, c->DEM.as<float>());
+    SLLG_TRY(sync_spins(c));
+    return dipolar_refresh(c, c->S.p, c->DEM.p);
 }
 
 }  // namespace sllg

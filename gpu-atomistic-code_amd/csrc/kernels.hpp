@@ -86,6 +86,7 @@ uint64_t dipolar_bytes(const llg_ctx* c);  // plan buffers and FFT work areas (a
 bool dipolar_is_exchange(const llg_ctx* c);  // the plan is an FFT-exchange plan
 bool dipolar_capturable(const llg_ctx* c);   // a refresh is this library's kernels only (no hipFFT plan)
 int dipolar_refresh(llg_ctx* c, const void* S, void* out);  // spins of the path's precision -> out (3n)
+int dipolar_refresh_spins(llg_ctx* c);  // FP32: DEM at the current spins, in whichever copy they are
 
 // Encodings (encode.cpp)
 int build_exchange_fp64(llg_ctx* c, const llg_exchange& e);
