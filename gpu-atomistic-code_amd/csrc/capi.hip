@@ -5,8 +5,7 @@
 //         (cullg::llgGPU, src/cuda.cu:43-258)
 //   RK4 / RK5: [dipolar refresh] -> noise -> stages -> combine
 //         (cullg::llgGPURK4 / llgGPURK5, src/cudaRK4.cu:38-233, src/cudaRK5.cu:38-273)
-// The FP64 plain path launches the reference's kernel sequence (SpMV, stage, SpMV,
-// stage); the FP32 path launches one fused kernel per field evaluation.
+// Both paths launch one kernel per field evaluation.
 #include <algorithm>
 #include <cmath>
 #include <cstring>
@@ -164,28 +163,21 @@ int take_noise(llg_ctx* c, const double** dev_xi) {
 }
 
 int step_plain(llg_ctx* c, uint64_t t) {
-    double* S = c->S.as<double>();
-    double* Y = c->Y.as<double>();
-    double* H = c->H.as<double>();
-    if (c->dip && t % c->dip_refresh == 0) SLLG_TIMED("dipolar_refresh", dipolar_refresh(c, S, c->DEM.p));
+    if (c->dip && t % c->dip_refresh == 0) SLLG_TIMED("dipolar_refresh", dipolar_refresh(c, c->S.p, c->DEM.p));
     const double* xi = nullptr;
     SLLG_TRY(take_noise(c, &xi));
-    if (c->noise_mode == LLG_NOISE_COUNTER && c->T > 0.0) SLLG_TIMED("plain_noise", plain_noise(c, t));
     if (c->scheme == LLG_HEUN) {
-        SLLG_TIMED("plain_spmv", plain_spmv(c, S, H));
-        SLLG_TIMED("plain_heun1", plain_heun1(c));
-        if (c->dip && c->dip_every_stage) SLLG_TIMED("dipolar_refresh", dipolar_refresh(c, Y, c->DEM.p));
-        SLLG_TIMED("plain_spmv", plain_spmv(c, Y, H));
-        SLLG_TIMED("plain_heun2", plain_heun2(c));
+        SLLG_TIMED("plain_predictor", plain_heun_pred(c, t));
+        if (c->dip && c->dip_every_stage) SLLG_TIMED("dipolar_refresh", dipolar_refresh(c, c->Y.p, c->DEM.p));
+        SLLG_TIMED("plain_corrector", plain_heun_corr(c, t));
         c->det_valid = true;
     } else {
         const int ns = c->scheme == LLG_RK4 ? 4 : 6;
         for (int m = 0; m < ns; ++m) {
-            if (m > 0 && c->dip && c->dip_every_stage) SLLG_TIMED("dipolar_refresh", dipolar_refresh(c, Y, c->DEM.p));
-            SLLG_TIMED("plain_spmv", plain_spmv(c, m == 0 ? S : Y, H));
-            SLLG_TIMED("plain_rk_stage", plain_rk_stage(c, m));
+            if (m > 0 && c->dip && c->dip_every_stage)
+                SLLG_TIMED("dipolar_refresh", dipolar_refresh(c, plain_rk_input(c, m), c->DEM.p));
+            SLLG_TIMED("plain_rk_stage", plain_rk_stage(c, t, m));
         }
-        SLLG_TIMED("plain_rk_combine", plain_rk_comb(c));
         c->det_valid = false;
     }
     return 0;
@@ -396,7 +388,7 @@ static int create_impl(const llg_desc* d, const std::shared_ptr<ExchStore>& shar
         SLLG_HIP(hipMemcpy(c->p_k1udir.p, kd.data(), 3 * (size_t)n * 8, hipMemcpyHostToDevice));
         if (c->scheme != LLG_HEUN) {
             SLLG_TRY(plain_rk_init_tables());
-            for (int m = 0; m < 6; ++m) SLLG_TRY(c->K[m].alloc(v3));
+            for (int m = 0; m < (c->scheme == LLG_RK4 ? 3 : 5); ++m) SLLG_TRY(c->K[m].alloc(v3));
         }
         if (!proto) SLLG_TRY(build_exchange_fp64(c, d->exch));
     } else {
@@ -776,19 +768,21 @@ int llg_get_info(llg_ctx* c, llg_info* info) {
                          (c->noise_mode == LLG_NOISE_INJECTED && c->T > 0 ? 24 : 0);
     if (c->prec == LLG_FP64_PLAIN) {
         const double params = 5 * 8.0 + 3 * 8.0;  // sigma, llgpf, lambda, k1u (+kc) and k1udir
-        const double noise = c->T > 0 ? 3 * 8.0 : 0.0;
-        const double spmv = M + 3 * P + (c->dip ? 3 * P : 0);
+        const double noise = c->T > 0 && c->noise_mode == LLG_NOISE_COUNTER ? 3 * 8.0 : 0.0;  // injected: in `extra`
+        const double read = M + 3 * P + params + noise + extra;  // couplings, spins, parameters, noise, fields
         if (c->scheme == LLG_HEUN) {
-            const double h1 = 3 * P + 3 * P + params + noise + 6 * P + (c->stag_set ? 3 * P : 0);
-            const double h2 = 3 * P * 3 + params + noise + 6 * P + (c->stag_set ? 3 * P : 0);
-            info->bytes_per_spin_update = 2 * spmv + h1 + h2 + (c->T > 0 && c->noise_mode == LLG_NOISE_COUNTER ? noise : 0);
-            info->dominant_kernel_bytes_per_spin = spmv;
-            std::snprintf(info->dominant_kernel, sizeof info->dominant_kernel, "k_plain_spmv");
+            // predictor writes Y and f(S) (and the draw); corrector reads S and f(S), writes S and DET
+            info->dominant_kernel_bytes_per_spin = read + 12 * P;
+            info->bytes_per_spin_update = read + 6 * P + info->dominant_kernel_bytes_per_spin;
+            std::snprintf(info->dominant_kernel, sizeof info->dominant_kernel, "k_plain_corr");
         } else {
+            // stage m reads its input (S for m = 0), S and the earlier k it needs, writes k_m and
+            // the next input; the last writes S
             const int ns = c->scheme == LLG_RK4 ? 4 : 6;
-            info->bytes_per_spin_update = ns * (spmv + 6 * P + params + noise + 3 * P) + 6 * P + ns * 3 * P;
-            info->dominant_kernel_bytes_per_spin = spmv;
-            std::snprintf(info->dominant_kernel, sizeof info->dominant_kernel, "k_plain_spmv");
+            const double ks = c->scheme == LLG_RK4 ? 3 : 10 + 3;  // k_j read over the step
+            info->bytes_per_spin_update = ns * read + ((ns - 1) + ks + (ns - 1) * 2 + 1) * 3 * P;
+            info->dominant_kernel_bytes_per_spin = read + (c->scheme == LLG_RK4 ? 4 : 7) * 3 * P;
+            std::snprintf(info->dominant_kernel, sizeof info->dominant_kernel, "k_plain_rk");
         }
     } else {
         if (c->scheme == LLG_HEUN) {

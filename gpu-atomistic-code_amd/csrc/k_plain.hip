@@ -1,15 +1,19 @@
-// k_plain.hip - FP64 plain path: the reference GPU step structure (separate SpMV and
-// integrator passes, FP64 couplings per nnz, per-spin parameter arrays) written for
-// gfx950 with SoA state.  Built with -ffp-contract=off; every operation follows the
+// k_plain.hip - FP64 plain path: FP64 couplings, state and per-spin parameter arrays (SoA),
+// one kernel per field evaluation.  Built with -ffp-contract=off; every operation follows the
 // order of the FP64 oracle so that both give the same bits.
 //
-//   k_plain_spmv     <- cufields::CSpMV_CSR / _OffDiag / CSpMV_DIA / _OffDiag (src/cufields.cu:97-246)
-//   k_plain_noise    <- curandGenerateNormal (src/cuda.cu:148), replaced by Philox4x32-10 + Box-Muller
-//   k_plain_heun1    <- cuint::CHeun1 (src/cuint.cu:60-163)
-//   k_plain_heun2    <- cuint::CHeun2 (src/cuint.cu:165-242)
-//   k_plain_rk_stage <- cuintRK4::CdetRK4k1..k4 (src/cuintRK4.cu:62-434), cuintRK5::CdetRK5k1..k6
-//                       (src/cuintRK5.cu:79-628), with textbook stage inputs
-//   k_plain_rk_comb  <- CdetSnp1 (src/cuintRK4.cu:436-456, src/cuintRK5.cu:630-651)
+//   plain_exchange   <- cufields::CSpMV_CSR / _OffDiag / CSpMV_DIA / _OffDiag (src/cufields.cu:97-246)
+//   normals3_f64     <- curandGenerateNormal (src/cuda.cu:148), replaced by Philox4x32-10 + Box-Muller
+//   k_plain_pred     <- exchange at S, noise, cuint::CHeun1 (src/cuint.cu:60-163)
+//   k_plain_corr     <- exchange at Y, cuint::CHeun2 (src/cuint.cu:165-242)
+//   k_plain_rk       <- exchange, cuintRK4::CdetRK4k1..k4 (src/cuintRK4.cu:62-434),
+//                       cuintRK5::CdetRK5k1..k6 (src/cuintRK5.cu:79-628) with textbook stage
+//                       inputs, and CdetSnp1 (src/cuintRK4.cu:436-456, src/cuintRK5.cu:630-651)
+//
+// The reference launches a kernel for the noise, for each SpMV and for each integrator pass,
+// with the field in memory between them.  Here a row's field stays in registers: a Heun step
+// is two launches instead of five and moves 72 bytes a spin less (the field written and read
+// twice, less the draw's); small systems are bound by the launches (PLAIN_FUSED).
 #include "field.hpp"
 #include "kernels.hpp"
 #include "philox.hpp"
@@ -27,47 +31,46 @@ struct PlainArgs {
     const double* k1udir;  // SoA 3n
     const double* kc;      // per spin or null
     const double* stg;     // 3n or null
-    const double* xi;      // 3n or null (T == 0)
+    const double* dem;     // dipolar field, 3n or null
+    double* xi;            // 3n or null (T == 0)
+    int draw;              // the kernel draws xi of step t (counter noise) and stores it
+    Perm perm;             // device row -> reference spin index, which keys the noise
+    uint64_t seed, stream, t;
     AnisG<double> an;
+    Exch<double> ex;
 };
 
+// Exchange sum of row i at spins S (CSR order), plus the dipolar field and the four-spin term:
+// H of the reference's SpMV pass.
 template <int NC>
-__global__ __launch_bounds__(kTPB) void k_plain_spmv(Exch<double> e, const double* __restrict__ S,
-                                                     const double* __restrict__ dem, double* __restrict__ H) {
-    const uint32_t i = blockIdx.x * kTPB + threadIdx.x;
+__device__ __forceinline__ void plain_exchange(const Exch<double>& e, uint32_t i, const double* __restrict__ S,
+                                               const double* __restrict__ dem, double hx[3]) {
     const uint32_t n = e.n;
-    if (i >= n) return;
     double dot[3];
     exch_row_ref<NC, double, double, double>(e, i, S, dot);
-    double hx[3];
     for (int a = 0; a < 3; ++a) hx[a] = (dem ? dem[(size_t)a * n + i] : 0.0) + dot[a];
     if (e.fs_xadj) {  // CH += four-spin field (src/cuda.cu:143-146)
         double h4[3];
         fourspin_row<double, double, double>(e, i, S, h4);
         for (int a = 0; a < 3; ++a) hx[a] = hx[a] + h4[a];
     }
-    for (int a = 0; a < 3; ++a) H[(size_t)a * n + i] = hx[a];
-}
-
-__global__ __launch_bounds__(kTPB) void k_plain_noise(uint32_t n, uint64_t seed, uint64_t stream, uint64_t t,
-                                                      double* __restrict__ xi) {
-    const uint32_t i = blockIdx.x * kTPB + threadIdx.x;
-    if (i >= n) return;
-    double z[3];
-    normals3_f64(seed, stream, i, t, z);
-    xi[i] = z[0];
-    xi[(size_t)n + i] = z[1];
-    xi[2 * (size_t)n + i] = z[2];
 }
 
 // Field at spin i (own spin s, exchange+demag hex): h = ((hex + stg) + th) + B, then local terms
 // (th = 0 when noise is false: the deterministic field).
 __device__ __forceinline__ void plain_field(const PlainArgs& a, uint32_t i, const double s[3], const double hex[3],
-                                            double th[3], double h[3], bool noise = true) {
+                                            double th[3], double h[3], bool noise = true, bool draw = false) {
     const uint32_t n = a.n;
     if (noise && a.xi) {
+        double z[3];
+        if (draw) {
+            normals3_f64(a.seed, a.stream, a.perm.to_ref(i), a.t, z);
+            for (int c = 0; c < 3; ++c) a.xi[(size_t)c * n + i] = z[c];  // for the later passes of the step
+        } else {
+            for (int c = 0; c < 3; ++c) z[c] = a.xi[(size_t)c * n + i];
+        }
         const double TP = sqrt(a.T) * a.sigma[i];
-        for (int c = 0; c < 3; ++c) th[c] = a.xi[(size_t)c * n + i] * TP;
+        for (int c = 0; c < 3; ++c) th[c] = z[c] * TP;
     } else {
         th[0] = th[1] = th[2] = 0.0;
     }
@@ -79,16 +82,16 @@ __device__ __forceinline__ void plain_field(const PlainArgs& a, uint32_t i, cons
     local_terms<double>(a.k1u[i], d, a.kc ? a.kc[i] : 0.0, a.an, s, h);
 }
 
-__global__ __launch_bounds__(kTPB) void k_plain_heun1(PlainArgs a, const double* __restrict__ H,
-                                                      const double* __restrict__ S, double* __restrict__ Y,
-                                                      double* __restrict__ FN) {
+template <int NC>
+__global__ __launch_bounds__(kTPB) void k_plain_pred(PlainArgs a, const double* __restrict__ S, double* __restrict__ Y,
+                                                     double* __restrict__ FN) {
     const uint32_t i = blockIdx.x * kTPB + threadIdx.x;
     const uint32_t n = a.n;
     if (i >= n) return;
+    double hex[3], th[3], h[3], f[3];
+    plain_exchange<NC>(a.ex, i, S, a.dem, hex);
     const double s[3] = {S[i], S[(size_t)n + i], S[2 * (size_t)n + i]};
-    const double hex[3] = {H[i], H[(size_t)n + i], H[2 * (size_t)n + i]};
-    double th[3], h[3], f[3];
-    plain_field(a, i, s, hex, th, h);
+    plain_field(a, i, s, hex, th, h, true, a.draw);
     llg_rhs<double>(a.llgpf[i], a.lambda[i], s, h, f);
     double es[3], mods = 0.0;
     for (int c = 0; c < 3; ++c) {
@@ -100,15 +103,15 @@ __global__ __launch_bounds__(kTPB) void k_plain_heun1(PlainArgs a, const double*
     for (int c = 0; c < 3; ++c) Y[(size_t)c * n + i] = es[c] / nrm;
 }
 
-__global__ __launch_bounds__(kTPB) void k_plain_heun2(PlainArgs a, const double* __restrict__ H,
-                                                      const double* __restrict__ Y, double* __restrict__ S,
-                                                      const double* __restrict__ FN, double* __restrict__ DET) {
+template <int NC>
+__global__ __launch_bounds__(kTPB) void k_plain_corr(PlainArgs a, const double* __restrict__ Y, double* __restrict__ S,
+                                                     const double* __restrict__ FN, double* __restrict__ DET) {
     const uint32_t i = blockIdx.x * kTPB + threadIdx.x;
     const uint32_t n = a.n;
     if (i >= n) return;
+    double hex[3], th[3], h[3], f[3];
+    plain_exchange<NC>(a.ex, i, Y, a.dem, hex);
     const double s[3] = {Y[i], Y[(size_t)n + i], Y[2 * (size_t)n + i]};
-    const double hex[3] = {H[i], H[(size_t)n + i], H[2 * (size_t)n + i]};
-    double th[3], h[3], f[3];
     plain_field(a, i, s, hex, th, h);
     llg_rhs<double>(a.llgpf[i], a.lambda[i], s, h, f);
     double ps[3] = {S[i], S[(size_t)n + i], S[2 * (size_t)n + i]};
@@ -124,97 +127,83 @@ __global__ __launch_bounds__(kTPB) void k_plain_heun2(PlainArgs a, const double*
     }
 }
 
-// RK stage m: k_m = rdt f(Y_m) into K[m]; then the next stage input in place of Y:
+// RK stage m: k_m = rdt f(Y_m) into K[m]; then the next stage input:
 // RK4: Y = S + a_m k_m (a = 1/2, 1/2, 1); Cash-Karp: Y = (((S + b_{m+1,0} k_0) + ...) + b_{m+1,m} k_m).
+// The last stage combines instead: S = N(S + sum_m w_m k_m).  Stage inputs alternate between
+// two buffers, since neighbouring rows still read the input of this stage.
 struct RkTab {
     double b[6][5];
-    int nb[6];
 };
 __constant__ RkTab c_rk5;
 
-template <int SCHEME, int M>
-__global__ __launch_bounds__(kTPB) void k_plain_rk_stage(PlainArgs a, const double* __restrict__ H,
-                                                         double* __restrict__ Y, const double* __restrict__ S,
-                                                         double* __restrict__ K0, double* __restrict__ K1,
-                                                         double* __restrict__ K2, double* __restrict__ K3,
-                                                         double* __restrict__ K4, double* __restrict__ K5) {
+struct RkBufs {
+    const double* in;
+    double* out;
+    double* S;
+    double* K[5];
+};
+
+template <int NC, int SCHEME>
+__global__ __launch_bounds__(kTPB) void k_plain_rk(PlainArgs a, RkBufs r, int m) {
     const uint32_t i = blockIdx.x * kTPB + threadIdx.x;
     const uint32_t n = a.n;
     if (i >= n) return;
-    const double* src = (M == 0) ? S : Y;
-    const double s[3] = {src[i], src[(size_t)n + i], src[2 * (size_t)n + i]};
-    const double hex[3] = {H[i], H[(size_t)n + i], H[2 * (size_t)n + i]};
-    double th[3], h[3], f[3];
-    plain_field(a, i, s, hex, th, h);
+    double hex[3], th[3], h[3], f[3], ls[3];
+    plain_exchange<NC>(a.ex, i, r.in, a.dem, hex);
+    const double s[3] = {r.in[i], r.in[(size_t)n + i], r.in[2 * (size_t)n + i]};
+    plain_field(a, i, s, hex, th, h, true, a.draw && m == 0);
     llg_rhs<double>(a.llgpf[i], a.lambda[i], s, h, f);
-    double* Ks[6] = {K0, K1, K2, K3, K4, K5};
-    double k[3];
-    for (int c = 0; c < 3; ++c) {
-        k[c] = a.rdt * f[c];
-        Ks[M][(size_t)c * n + i] = k[c];
-    }
-    if constexpr (SCHEME == LLG_RK4) {
-        if constexpr (M < 3) {
-            const double am = (M == 2) ? 1.0 : 0.5;
-            for (int c = 0; c < 3; ++c) Y[(size_t)c * n + i] = S[(size_t)c * n + i] + am * k[c];
-        }
-    } else {
-        if constexpr (M < 5) {
-            for (int c = 0; c < 3; ++c) {
-                double v = S[(size_t)c * n + i];
-                for (int j = 0; j <= M; ++j) {
-                    const double kj = (j == M) ? k[c] : Ks[j][(size_t)c * n + i];
-                    v = v + c_rk5.b[M + 1][j] * kj;
-                }
-                Y[(size_t)c * n + i] = v;
-            }
-        }
-    }
-}
-
-template <int SCHEME>
-__global__ __launch_bounds__(kTPB) void k_plain_rk_comb(uint32_t n, double* __restrict__ S,
-                                                        const double* __restrict__ K0, const double* __restrict__ K1,
-                                                        const double* __restrict__ K2, const double* __restrict__ K3,
-                                                        const double* __restrict__ K4, const double* __restrict__ K5) {
-    const uint32_t i = blockIdx.x * kTPB + threadIdx.x;
-    if (i >= n) return;
-    double ls[3], mods = 0.0;
+    constexpr int last = SCHEME == LLG_RK4 ? 3 : 5;
+    double mods = 0.0;
     for (int c = 0; c < 3; ++c) {
         const size_t o = (size_t)c * n + i;
-        if constexpr (SCHEME == LLG_RK4) {
+        const double k = a.rdt * f[c];
+        if (m < last) {
+            r.K[m][o] = k;
+            if constexpr (SCHEME == LLG_RK4) {
+                const double am = (m == 2) ? 1.0 : 0.5;
+                r.out[o] = r.S[o] + am * k;
+            } else {
+                double v = r.S[o];
+                for (int j = 0; j < m; ++j) v = v + c_rk5.b[m + 1][j] * r.K[j][o];
+                r.out[o] = v + c_rk5.b[m + 1][m] * k;
+            }
+        } else if constexpr (SCHEME == LLG_RK4) {
             const double onesixth = 1.0 / 6.0, onethird = 1.0 / 3.0;
-            ls[c] = S[o] + K0[o] * onesixth + K1[o] * onethird + K2[o] * onethird + K3[o] * onesixth;
+            ls[c] = r.S[o] + r.K[0][o] * onesixth + r.K[1][o] * onethird + r.K[2][o] * onethird + k * onesixth;
+            mods += ls[c] * ls[c];
         } else {
-            double v = S[o];
-            v = v + K0[o] * (37.0 / 378.0);
-            v = v + K2[o] * (250.0 / 621.0);
-            v = v + K3[o] * (125.0 / 594.0);
-            v = v + K5[o] * (512.0 / 1771.0);
-            ls[c] = v;
+            double v = r.S[o];
+            v = v + r.K[0][o] * (37.0 / 378.0);
+            v = v + r.K[2][o] * (250.0 / 621.0);
+            v = v + r.K[3][o] * (125.0 / 594.0);
+            ls[c] = v + k * (512.0 / 1771.0);
+            mods += ls[c] * ls[c];
         }
-        mods += ls[c] * ls[c];
     }
-    const double nrm = sqrt(mods);
-    for (int c = 0; c < 3; ++c) S[(size_t)c * n + i] = ls[c] / nrm;
+    if (m == last) {
+        const double nrm = sqrt(mods);
+        for (int c = 0; c < 3; ++c) r.S[(size_t)c * n + i] = ls[c] / nrm;
+    }
 }
 
 // Deterministic field (no thermal part) at spins Sp, FP64 plain layout.
-__global__ __launch_bounds__(kTPB) void k_plain_detfield(PlainArgs a, const double* __restrict__ H,
-                                                         const double* __restrict__ Sp, double* __restrict__ out) {
+template <int NC>
+__global__ __launch_bounds__(kTPB) void k_plain_detfield(PlainArgs a, const double* __restrict__ Sp,
+                                                         double* __restrict__ out) {
     const uint32_t i = blockIdx.x * kTPB + threadIdx.x;
     const uint32_t n = a.n;
     if (i >= n) return;
+    double hex[3], th[3], h[3];
+    plain_exchange<NC>(a.ex, i, Sp, a.dem, hex);
     const double s[3] = {Sp[i], Sp[(size_t)n + i], Sp[2 * (size_t)n + i]};
-    const double hex[3] = {H[i], H[(size_t)n + i], H[2 * (size_t)n + i]};
-    double th[3], h[3];
     plain_field(a, i, s, hex, th, h, false);
     for (int c = 0; c < 3; ++c) out[(size_t)c * n + i] = h[c];
 }
 
 // ---------------------------------------------------------------- host launchers
 
-static PlainArgs plain_args(const llg_ctx* c, bool with_noise) {
+static PlainArgs plain_args(const llg_ctx* c, bool with_noise, uint64_t t) {
     PlainArgs a;
     a.n = c->n;
     a.rdt = c->rdt;
@@ -227,42 +216,44 @@ static PlainArgs plain_args(const llg_ctx* c, bool with_noise) {
     a.k1udir = c->p_k1udir.as<double>();
     a.kc = c->p_kc.as<double>();
     a.stg = c->stag_set ? c->STG.as<double>() : nullptr;
+    a.dem = c->dip ? c->DEM.as<double>() : nullptr;
     a.xi = (with_noise && c->T > 0.0) ? c->XI.as<double>() : nullptr;
+    a.draw = c->noise_mode == LLG_NOISE_COUNTER;
+    a.perm = c->perm;
+    a.seed = c->seed;
+    a.stream = c->stream_id;
+    a.t = t;
     a.an = c->an64;
+    a.ex = c->ex64;
     return a;
 }
 
-int plain_spmv(llg_ctx* c, const double* S, double* H) {
+#define SLLG_PLAIN_NC(NC_VAL, MACRO)      \
+    do {                                  \
+        if ((NC_VAL) == 1) { MACRO(1); }  \
+        else if ((NC_VAL) == 3) { MACRO(3); } \
+        else { MACRO(9); }                \
+    } while (0)
+
+// Predictor of step t: the exchange at S, the step's noise (drawn here in counter mode), Y and f(S).
+int plain_heun_pred(llg_ctx* c, uint64_t t) {
+    const PlainArgs a = plain_args(c, true, t);
     const dim3 g(blocks_for(c->n, kTPB)), b(kTPB);
-    const double* dem = c->dip ? c->DEM.as<double>() : nullptr;
-    switch (c->ex64.ncomp) {
-        case 1: k_plain_spmv<1><<<g, b, 0, c->stream>>>(c->ex64, S, dem, H); break;
-        case 3: k_plain_spmv<3><<<g, b, 0, c->stream>>>(c->ex64, S, dem, H); break;
-        default: k_plain_spmv<9><<<g, b, 0, c->stream>>>(c->ex64, S, dem, H); break;
-    }
+#define SLLG_L(N) k_plain_pred<N><<<g, b, 0, c->stream>>>(a, c->S.as<double>(), c->Y.as<double>(), c->FN.as<double>())
+    SLLG_PLAIN_NC(a.ex.ncomp, SLLG_L);
+#undef SLLG_L
     SLLG_HIP(hipGetLastError());
     return 0;
 }
 
-int plain_noise(llg_ctx* c, uint64_t t) {
-    k_plain_noise<<<blocks_for(c->n, kTPB), kTPB, 0, c->stream>>>(c->n, c->seed, c->stream_id, t, c->XI.as<double>());
-    SLLG_HIP(hipGetLastError());
-    return 0;
-}
-
-int plain_heun1(llg_ctx* c) {
-    PlainArgs a = plain_args(c, true);
-    k_plain_heun1<<<blocks_for(c->n, kTPB), kTPB, 0, c->stream>>>(a, c->H.as<double>(), c->S.as<double>(),
-                                                                  c->Y.as<double>(), c->FN.as<double>());
-    SLLG_HIP(hipGetLastError());
-    return 0;
-}
-
-int plain_heun2(llg_ctx* c) {
-    PlainArgs a = plain_args(c, true);
-    k_plain_heun2<<<blocks_for(c->n, kTPB), kTPB, 0, c->stream>>>(a, c->H.as<double>(), c->Y.as<double>(),
-                                                                  c->S.as<double>(), c->FN.as<double>(),
-                                                                  c->DET.as<double>());
+int plain_heun_corr(llg_ctx* c, uint64_t t) {
+    const PlainArgs a = plain_args(c, true, t);
+    const dim3 g(blocks_for(c->n, kTPB)), b(kTPB);
+#define SLLG_L(N)                                                                                      \
+    k_plain_corr<N><<<g, b, 0, c->stream>>>(a, c->Y.as<double>(), c->S.as<double>(), c->FN.as<double>(), \
+                                            c->DET.as<double>())
+    SLLG_PLAIN_NC(a.ex.ncomp, SLLG_L);
+#undef SLLG_L
     SLLG_HIP(hipGetLastError());
     return 0;
 }
@@ -284,54 +275,35 @@ int plain_rk_init_tables() {
     return 0;
 }
 
-int plain_rk_stage(llg_ctx* c, int m) {
-    PlainArgs a = plain_args(c, true);
-    const dim3 g(blocks_for(c->n, kTPB)), b(kTPB);
-    double* K[6];
-    for (int k = 0; k < 6; ++k) K[k] = c->K[k].as<double>();
-    const double* H = c->H.as<double>();
-    double* Y = c->Y.as<double>();
-    const double* S = c->S.as<double>();
-#define SLLG_RK_CASE(SCH, MM) \
-    k_plain_rk_stage<SCH, MM><<<g, b, 0, c->stream>>>(a, H, Y, S, K[0], K[1], K[2], K[3], K[4], K[5])
-    if (c->scheme == LLG_RK4) {
-        switch (m) {
-            case 0: SLLG_RK_CASE(LLG_RK4, 0); break;
-            case 1: SLLG_RK_CASE(LLG_RK4, 1); break;
-            case 2: SLLG_RK_CASE(LLG_RK4, 2); break;
-            default: SLLG_RK_CASE(LLG_RK4, 3); break;
-        }
-    } else {
-        switch (m) {
-            case 0: SLLG_RK_CASE(LLG_RK5, 0); break;
-            case 1: SLLG_RK_CASE(LLG_RK5, 1); break;
-            case 2: SLLG_RK_CASE(LLG_RK5, 2); break;
-            case 3: SLLG_RK_CASE(LLG_RK5, 3); break;
-            case 4: SLLG_RK_CASE(LLG_RK5, 4); break;
-            default: SLLG_RK_CASE(LLG_RK5, 5); break;
-        }
-    }
-#undef SLLG_RK_CASE
-    SLLG_HIP(hipGetLastError());
-    return 0;
+// Stage m of a Runge-Kutta step: its input is S (m = 0), then Y and H in turn.
+double* plain_rk_input(const llg_ctx* c, int m) {
+    return m == 0 ? c->S.as<double>() : ((m & 1) ? c->Y.as<double>() : c->H.as<double>());
 }
 
-int plain_rk_comb(llg_ctx* c) {
+int plain_rk_stage(llg_ctx* c, uint64_t t, int m) {
+    const PlainArgs a = plain_args(c, true, t);
     const dim3 g(blocks_for(c->n, kTPB)), b(kTPB);
-    double* K[6];
-    for (int k = 0; k < 6; ++k) K[k] = c->K[k].as<double>();
-    if (c->scheme == LLG_RK4)
-        k_plain_rk_comb<LLG_RK4><<<g, b, 0, c->stream>>>(c->n, c->S.as<double>(), K[0], K[1], K[2], K[3], K[4], K[5]);
-    else
-        k_plain_rk_comb<LLG_RK5><<<g, b, 0, c->stream>>>(c->n, c->S.as<double>(), K[0], K[1], K[2], K[3], K[4], K[5]);
+    RkBufs r;
+    r.in = plain_rk_input(c, m);
+    r.out = plain_rk_input(c, m + 1);
+    r.S = c->S.as<double>();
+    for (int k = 0; k < 5; ++k) r.K[k] = c->K[k].as<double>();
+#define SLLG_L(N)                                                                      \
+    do {                                                                               \
+        if (c->scheme == LLG_RK4) k_plain_rk<N, LLG_RK4><<<g, b, 0, c->stream>>>(a, r, m); \
+        else k_plain_rk<N, LLG_RK5><<<g, b, 0, c->stream>>>(a, r, m);                  \
+    } while (0)
+    SLLG_PLAIN_NC(a.ex.ncomp, SLLG_L);
+#undef SLLG_L
     SLLG_HIP(hipGetLastError());
     return 0;
 }
 
 int plain_detfield(llg_ctx* c, const double* Sp, double* out) {
-    SLLG_TRY(plain_spmv(c, Sp, c->H.as<double>()));
-    PlainArgs a = plain_args(c, false);
-    k_plain_detfield<<<blocks_for(c->n, kTPB), kTPB, 0, c->stream>>>(a, c->H.as<double>(), Sp, out);
+    const PlainArgs a = plain_args(c, false, 0);
+#define SLLG_L(N) k_plain_detfield<N><<<blocks_for(c->n, kTPB), kTPB, 0, c->stream>>>(a, Sp, out)
+    SLLG_PLAIN_NC(a.ex.ncomp, SLLG_L);
+#undef SLLG_L
     SLLG_HIP(hipGetLastError());
     return 0;
 }

@@ -5,13 +5,11 @@
 namespace sllg {
 
 // FP64 plain path (k_plain.hip)
-int plain_spmv(llg_ctx* c, const double* S, double* H);
-int plain_noise(llg_ctx* c, uint64_t t);
-int plain_heun1(llg_ctx* c);
-int plain_heun2(llg_ctx* c);
+int plain_heun_pred(llg_ctx* c, uint64_t t);
+int plain_heun_corr(llg_ctx* c, uint64_t t);
 int plain_rk_init_tables();
-int plain_rk_stage(llg_ctx* c, int m);
-int plain_rk_comb(llg_ctx* c);
+double* plain_rk_input(const llg_ctx* c, int m);  // spins RK stage m is evaluated at
+int plain_rk_stage(llg_ctx* c, uint64_t t, int m);
 int plain_detfield(llg_ctx* c, const double* Sp, double* out);
 int stag_scale(llg_ctx* c, double r);  // STG = r * STG0 (FP64 H0 kept on the device)
 
