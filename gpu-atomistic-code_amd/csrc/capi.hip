@@ -74,6 +74,30 @@ struct Scope {
 
 size_t prec_bytes(const llg_ctx* c) { return c->prec == LLG_FP64_PLAIN ? sizeof(double) : sizeof(float); }
 
+// One component between the reference spin order in FP64 (host side) and the device order in
+// the path's precision.
+template <class T>
+__global__ __launch_bounds__(kTPB) void k_from_ref(uint32_t n, Perm perm, const double* __restrict__ ref,
+                                                   T* __restrict__ dev) {
+    const uint32_t i = blockIdx.x * kTPB + threadIdx.x;
+    if (i < n) dev[perm.to_dev(i)] = (T)ref[i];
+}
+template <class T>
+__global__ __launch_bounds__(kTPB) void k_to_ref(uint32_t n, Perm perm, const T* __restrict__ dev,
+                                                 double* __restrict__ ref) {
+    const uint32_t i = blockIdx.x * kTPB + threadIdx.x;
+    if (i < n) ref[i] = (double)dev[perm.to_dev(i)];
+}
+
+// From this size on order and precision are converted on the device, one component at a time
+// (fcc 64^3: FP32 spins set in 1.9 ms and fetched in 1.9 instead of 3.3 and 2.5 with the host
+// loop, an FP64 field fetched in 2.0 instead of 8.8); below it three kernels and copies take
+// longer than the loop (10^3 spins: 58 us against 28).
+constexpr uint32_t kIoDevice = 65536;
+// n doubles of device memory that are free between steps: the FP32 path's A, the FP64 path's H
+// (both only carry values within a step).
+double* io_scratch(const llg_ctx* c) { return c->prec == LLG_FP64_PLAIN ? c->H.as<double>() : c->A.as<double>(); }
+
 // Upload a host SoA double[3n] (reference spin order) into a state buffer of the path's
 // precision, in the device order.
 int upload_state(llg_ctx* c, DevBuf& dst, const double* x, const double* y, const double* z) {
@@ -84,16 +108,32 @@ int upload_state(llg_ctx* c, DevBuf& dst, const double* x, const double* y, cons
         c->s_soa_valid = true;
     }
     if (&dst == &c->Y) c->y_soa_valid = true;
-    if (c->prec == LLG_FP64_PLAIN) {
-        for (int a = 0; a < 3; ++a)
-            SLLG_HIP(hipMemcpyAsync(dst.as<double>() + (size_t)a * n, src[a], n * 8, hipMemcpyHostToDevice, c->stream));
-    } else {
-        std::vector<float> t(3 * (size_t)n);
+    const bool f64 = c->prec == LLG_FP64_PLAIN, direct = f64 && !c->permuted();
+    if (!direct && n < kIoDevice) {
+        std::vector<double> t64(f64 ? 3 * (size_t)n : 0);
+        std::vector<float> t32(f64 ? 0 : 3 * (size_t)n);
         for (uint32_t i = 0; i < n; ++i) {
-            const uint32_t d = c->perm.to_dev(i);
-            for (int a = 0; a < 3; ++a) t[(size_t)a * n + d] = (float)src[a][i];
+            const size_t d = c->perm.to_dev(i);
+            for (int a = 0; a < 3; ++a) {
+                if (f64) t64[(size_t)a * n + d] = src[a][i];
+                else t32[(size_t)a * n + d] = (float)src[a][i];
+            }
         }
-        SLLG_HIP(hipMemcpyAsync(dst.p, t.data(), t.size() * 4, hipMemcpyHostToDevice, c->stream));
+        SLLG_HIP(hipMemcpyAsync(dst.p, f64 ? (const void*)t64.data() : (const void*)t32.data(),
+                                3 * (size_t)n * (f64 ? 8 : 4), hipMemcpyHostToDevice, c->stream));
+        SLLG_HIP(hipStreamSynchronize(c->stream));
+        return 0;
+    }
+    double* const tmp = io_scratch(c);
+    for (int a = 0; a < 3; ++a) {
+        double* const to = direct ? dst.as<double>() + (size_t)a * n : tmp;
+        SLLG_HIP(hipMemcpyAsync(to, src[a], (size_t)n * 8, hipMemcpyHostToDevice, c->stream));
+        if (direct) continue;
+        if (f64)
+            k_from_ref<double><<<blocks_for(n, kTPB), kTPB, 0, c->stream>>>(n, c->perm, tmp, dst.as<double>() + (size_t)a * n);
+        else
+            k_from_ref<float><<<blocks_for(n, kTPB), kTPB, 0, c->stream>>>(n, c->perm, tmp, dst.as<float>() + (size_t)a * n);
+        SLLG_HIP(hipGetLastError());
     }
     SLLG_HIP(hipStreamSynchronize(c->stream));
     return 0;
@@ -104,23 +144,34 @@ int upload_state(llg_ctx* c, DevBuf& dst, const double* x, const double* y, cons
 int download_state(llg_ctx* c, const void* src_dev, bool src_f64, double* x, double* y, double* z) {
     const uint32_t n = c->n;
     double* dst[3] = {x, y, z};
-    if (src_f64 && !c->permuted()) {
-        const double* s = (const double*)src_dev;
-        for (int a = 0; a < 3; ++a)
-            SLLG_HIP(hipMemcpyAsync(dst[a], s + (size_t)a * n, n * 8, hipMemcpyDeviceToHost, c->stream));
+    const bool direct = src_f64 && !c->permuted();
+    if (!direct && n < kIoDevice) {
+        const size_t eb = src_f64 ? 8 : 4;
+        std::vector<unsigned char> raw(3 * (size_t)n * eb);
+        SLLG_HIP(hipMemcpyAsync(raw.data(), src_dev, raw.size(), hipMemcpyDeviceToHost, c->stream));
         SLLG_HIP(hipStreamSynchronize(c->stream));
+        const double* r64 = reinterpret_cast<const double*>(raw.data());
+        const float* r32 = reinterpret_cast<const float*>(raw.data());
+        for (uint32_t i = 0; i < n; ++i) {
+            const size_t d = c->perm.to_dev(i);
+            for (int a = 0; a < 3; ++a) dst[a][i] = src_f64 ? r64[(size_t)a * n + d] : (double)r32[(size_t)a * n + d];
+        }
         return 0;
     }
-    const size_t eb = src_f64 ? 8 : 4;
-    std::vector<unsigned char> raw(3 * (size_t)n * eb);
-    SLLG_HIP(hipMemcpyAsync(raw.data(), src_dev, raw.size(), hipMemcpyDeviceToHost, c->stream));
-    SLLG_HIP(hipStreamSynchronize(c->stream));
-    const double* r64 = reinterpret_cast<const double*>(raw.data());
-    const float* r32 = reinterpret_cast<const float*>(raw.data());
-    for (uint32_t i = 0; i < n; ++i) {
-        const size_t d = c->perm.to_dev(i);
-        for (int a = 0; a < 3; ++a) dst[a][i] = src_f64 ? r64[(size_t)a * n + d] : (double)r32[(size_t)a * n + d];
+    double* const tmp = io_scratch(c);
+    for (int a = 0; a < 3; ++a) {
+        const double* const s64 = (const double*)src_dev + (size_t)a * n;
+        const float* const s32 = (const float*)src_dev + (size_t)a * n;
+        if (!direct) {
+            if (src_f64)
+                k_to_ref<double><<<blocks_for(n, kTPB), kTPB, 0, c->stream>>>(n, c->perm, s64, tmp);
+            else
+                k_to_ref<float><<<blocks_for(n, kTPB), kTPB, 0, c->stream>>>(n, c->perm, s32, tmp);
+            SLLG_HIP(hipGetLastError());
+        }
+        SLLG_HIP(hipMemcpyAsync(dst[a], direct ? s64 : tmp, (size_t)n * 8, hipMemcpyDeviceToHost, c->stream));
     }
+    SLLG_HIP(hipStreamSynchronize(c->stream));
     return 0;
 }
 
@@ -368,14 +419,16 @@ static int create_impl(const llg_desc* d, const std::shared_ptr<ExchStore>& shar
         SLLG_TRY(c->H.alloc(v3));
         SLLG_TRY(c->FN.alloc(v3));
         SLLG_TRY(c->DET.alloc(v3));
+        if (!proto) SLLG_TRY(build_exchange_fp64(c, d->exch));
         // per-spin parameter arrays, as the reference uploads them (src/cuda_util.cu:282-556)
         std::vector<double> sg(n), lp(n), lm(n), k1(n), kd(3 * (size_t)n), kc(n);
         bool any_kc = false;
         for (uint32_t i = 0; i < n; ++i) {
             const Species<double>& q = c->sp64[spec[i]];
-            sg[i] = q.sigma; lp[i] = q.llgpf; lm[i] = q.lambda; k1[i] = q.k1u; kc[i] = q.kc;
+            const uint32_t d = c->xs->perm.to_dev(i);
+            sg[d] = q.sigma; lp[d] = q.llgpf; lm[d] = q.lambda; k1[d] = q.k1u; kc[d] = q.kc;
             any_kc = any_kc || q.kc != 0.0;
-            for (int a = 0; a < 3; ++a) kd[(size_t)a * n + i] = q.k1dir[a];
+            for (int a = 0; a < 3; ++a) kd[(size_t)a * n + d] = q.k1dir[a];
         }
         DevBuf* bufs[5] = {&c->p_sigma, &c->p_llgpf, &c->p_lambda, &c->p_k1u, &c->p_kc};
         std::vector<double>* srcs[5] = {&sg, &lp, &lm, &k1, &kc};
@@ -390,7 +443,6 @@ static int create_impl(const llg_desc* d, const std::shared_ptr<ExchStore>& shar
             SLLG_TRY(plain_rk_init_tables());
             for (int m = 0; m < (c->scheme == LLG_RK4 ? 3 : 5); ++m) SLLG_TRY(c->K[m].alloc(v3));
         }
-        if (!proto) SLLG_TRY(build_exchange_fp64(c, d->exch));
     } else {
         SLLG_TRY(c->A.alloc(v3));
         if (c->scheme == LLG_RK4) SLLG_TRY(c->K[0].alloc(v3));
@@ -753,7 +805,8 @@ int llg_get_info(llg_ctx* c, llg_info* info) {
     // coupling bytes per row per field evaluation (M)
     double M = 0.0;
     if (c->prec == LLG_FP64_PLAIN) {
-        if (h.fmt == LLG_EXCH_CSR) M = 4.0 + (double)h.nnz / n * (4.0 + 8.0 * nc);
+        if (c->ex64.fmt == FMT_UNI) M = (double)c->ex64.nent * 4.0 / n;
+        else if (h.fmt == LLG_EXCH_CSR) M = 4.0 + (double)h.nnz / n * (4.0 + 8.0 * nc);
         else if (h.fmt == LLG_EXCH_DIA) M = (double)h.ndiag * 8.0 * nc;
         else if (h.fmt == LLG_EXCH_STENCIL && h.per_row) M = (double)h.sk * 8.0 * nc;
     } else {

@@ -53,7 +53,8 @@ enum ExchFmt : int {
     FMT_SELL_LINE = 6,   // FP32: slices that are periodic 64-cell lines, lane-uniform scalar coupling stream
     FMT_SELL_LINE16 = 7,      // FP32: slices of four periodic 16-cell lines, same stream (rotations within 16 lanes)
     FMT_SELL_LINE_OPEN = 8,   // FP32: open 64-cell lines (zero-filling shifts instead of rotations)
-    FMT_SELL_LINE16_OPEN = 9  // FP32: four open 16-cell lines per slice
+    FMT_SELL_LINE16_OPEN = 9, // FP32: four open 16-cell lines per slice
+    FMT_UNI = 10              // FP64 plain: CSR rows as lane-uniform records of 64-row slices
 };
 
 constexpr bool is_line_fmt(int f) {
@@ -61,6 +62,20 @@ constexpr bool is_line_fmt(int f) {
 }
 constexpr int line_len(int f) { return (f == FMT_SELL_LINE || f == FMT_SELL_LINE_OPEN) ? 64 : 16; }
 constexpr bool line_open(int f) { return f == FMT_SELL_LINE_OPEN || f == FMT_SELL_LINE16_OPEN; }
+
+// Records of the lane-uniform CSR (FMT_UNI), in blocks of kUniBlock stored field by field so
+// that a wave reads a block with wide scalar loads:
+//   [0, 4)       d0: byte offset of the neighbour's component 0 from the row's own, for the lanes
+//                whose bit of the mask is clear
+//   [4, 8)       d1: the same for the others
+//   [8, 16)      masks (low, high word)
+//   [16, ..)     couplings [record][component], FP64
+// kUniNone as an offset stands for "no entry": the load falls outside the spins and reads zero.
+constexpr uint32_t kUniBlock = 4;
+constexpr uint32_t kUniNone = 0x80000000u;
+constexpr uint32_t uni_words(int nc) { return kUniBlock * (4 + 2 * (uint32_t)nc); }
+// Spins a record can address: three components of 8 bytes within kUniNone.
+constexpr uint64_t kUniMaxSpins = kUniNone / 24;
 
 // Per-species constants, precision R.
 template <class R> struct Species {
@@ -97,9 +112,9 @@ template <class V> struct Exch {
     const uint32_t* scount = nullptr; // [na]
     // sliced ELL
     // [nslices] {first entry / 64, entries per row}; slices with identical packed entries
-    // point at one stored copy
+    // point at one stored copy (lane-uniform records: {first word, blocks})
     const uint2* slice = nullptr;
-    const uint32_t* ent = nullptr;        // packed entries or columns, [..][64]
+    const uint32_t* ent = nullptr;        // packed entries or columns, [..][64]; record words
     const V* dict = nullptr;              // [ndict][ncomp] (SELL_PACK) or raw values
     uint32_t ndict = 0;
     uint64_t nent = 0;                    // total entries (SELL_RAW value stride)

@@ -1,8 +1,9 @@
 // encode.hip - host-side validation of the exchange given in the descriptor and its
 // upload in the layout each path reads.
 //
-// FP64 plain path: the reference layouts as given (CSR u32 + FP64 [ncomp][nnz];
-// DIA [ncomp][ndiag][n]; periodic stencil).
+// FP64 plain path: CSR as lane-uniform records of 64-row slices where the couplings repeat
+// from row to row, else sliced (u32 columns + FP64 values); DIA [ncomp][ndiag][n] and the
+// periodic stencil as given.
 //
 // FP32 path: CSR becomes sliced ELL with 64-row slices (one wavefront) so that every
 // load of the coupling stream is a contiguous wave access (1 KB per uint4 load).  When the
@@ -129,6 +130,133 @@ void release_host(HostExch& h) {
 
 }  // namespace
 
+namespace {
+
+// CSR rows as lane-uniform records (FMT_UNI).  Entry q of the 64 rows of a slice falls into a
+// few classes of equal (row offset, couplings): one away from the lattice's boundaries, a
+// second where a row's neighbour wraps around a periodic one.  A record holds one coupling and
+// two offsets with the lanes that take the second, so a slice is about as many records as its
+// rows have entries, each read once a wave, where the CSR reads 12 bytes or more a row and
+// entry; rows without an entry q (open boundaries) take the offset "none".  Every row meets its
+// own entries in CSR order, and the others load zeros, so the sums are the CSR's bit for bit.
+// Slices with equal records are stored once.  False (nothing kept) when the records would be
+// more than twice the entries of a row, as for couplings that differ from row to row, when the
+// offsets do not fit, or when the caller wants every slice stored.
+bool build_uniform(llg_ctx* c, const HostExch& h, const Perm& P, std::vector<uint2>& table,
+                   std::vector<uint32_t>& words, uint32_t& stored) {
+    const uint32_t n = c->n, nc = (uint32_t)h.ncomp, nsl = (n + kSlice - 1) / kSlice, BW = uni_words((int)nc);
+    if (n > kUniMaxSpins || (c->flags & LLG_FLAG_NO_SLICE_SHARING)) return false;
+    struct Rec {
+        uint32_t d0, d1;
+        uint64_t mask;
+        uint32_t entry;  // an entry with the record's couplings
+    };
+    auto same = [&](uint32_t p, uint32_t q) {
+        for (uint32_t k = 0; k < nc; ++k)
+            if (std::memcmp(&h.vals[(size_t)k * h.nnz + p], &h.vals[(size_t)k * h.nnz + q], 8)) return false;
+        return true;
+    };
+    const uint32_t sh = P.na > 1 && !(P.na & (P.na - 1)) ? (uint32_t)__builtin_ctz(P.na) : 0u;
+    auto to_dev = [&](uint32_t i) { return sh ? (i & (P.na - 1)) * P.ncell + (i >> sh) : P.to_dev(i); };
+    table.resize(nsl);
+    std::unordered_map<uint64_t, std::vector<uint32_t>> seen;  // hash of a slice's words -> slices
+    std::vector<Rec> recs;
+    std::vector<uint32_t> st;
+    uint64_t nrec = 0, nlen = 0;
+    stored = 0;
+    for (uint32_t s = 0; s < nsl; ++s) {
+        const uint32_t d0 = s * kSlice, rows = std::min<uint32_t>(kSlice, n - d0);
+        uint32_t first[kSlice], len[kSlice], most = 0;
+        for (uint32_t l = 0; l < rows; ++l) {
+            const uint32_t r = P.to_ref(d0 + l);
+            first[l] = h.xadj[r];
+            len[l] = h.xadj[r + 1] - h.xadj[r];
+            most = std::max(most, len[l]);
+        }
+        recs.clear();
+        for (uint32_t q = 0; q < most; ++q) {
+            // classes of (offset, couplings) with their lanes; then records: a class and, where
+            // there is one, another with the same couplings or the lanes that have none
+            struct Cls {
+                uint32_t off, entry;
+                uint64_t lanes;
+            } cls[kSlice];
+            uint32_t m = 0;
+            uint64_t none = 0;
+            for (uint32_t l = 0; l < rows; ++l) {
+                if (q >= len[l]) {
+                    none |= 1ull << l;
+                    continue;
+                }
+                const uint32_t p = first[l] + q, off = 8u * (to_dev(h.adj[p]) - (d0 + l));
+                uint32_t k = 0;
+                while (k < m && !(cls[k].off == off && same(cls[k].entry, p))) ++k;
+                if (k == m) cls[m++] = Cls{off, p, 0};
+                cls[k].lanes |= 1ull << l;
+            }
+            bool used[kSlice] = {};
+            const uint64_t all = rows == kSlice ? ~0ull : (1ull << rows) - 1ull;
+            for (uint32_t k = 0; k < m; ++k) {
+                if (used[k]) continue;
+                used[k] = true;
+                uint32_t o = k + 1;
+                while (o < m && (used[o] || !same(cls[k].entry, cls[o].entry))) ++o;
+                // the lanes outside both classes of a record must read nothing
+                if (o < m && (cls[k].lanes | cls[o].lanes) == all) {
+                    used[o] = true;
+                    recs.push_back(Rec{cls[k].off, cls[o].off, cls[o].lanes, cls[k].entry});
+                } else {
+                    recs.push_back(Rec{cls[k].off, kUniNone, all & ~cls[k].lanes, cls[k].entry});
+                }
+            }
+        }
+        nrec += recs.size();
+        nlen += most;
+        if (nrec > 2 * nlen + 256) return false;
+        const uint32_t blocks = ((uint32_t)recs.size() + kUniBlock - 1) / kUniBlock;
+        st.assign((size_t)blocks * BW, 0u);
+        for (uint32_t r = 0; r < blocks * kUniBlock; ++r) {
+            uint32_t* const w = st.data() + (size_t)(r / kUniBlock) * BW;
+            const uint32_t u = r % kUniBlock;
+            const bool pad = r >= recs.size();
+            w[u] = pad ? kUniNone : recs[r].d0;
+            w[4 + u] = pad ? kUniNone : recs[r].d1;
+            if (pad) continue;
+            std::memcpy(w + 8 + 2 * u, &recs[r].mask, 8);
+            for (uint32_t k = 0; k < nc; ++k)
+                std::memcpy(w + 16 + 2 * (u * nc + k), &h.vals[(size_t)k * h.nnz + recs[r].entry], 8);
+        }
+        uint64_t hsh = 1469598103934665603ull;
+        for (uint32_t v : st) hsh = (hsh ^ v) * 1099511628211ull;
+        bool found = false;
+        for (uint32_t o : seen[hsh])
+            if (table[o].y == blocks && !std::memcmp(words.data() + table[o].x, st.data(), st.size() * 4)) {
+                table[s] = table[o];
+                found = true;
+                break;
+            }
+        if (found) continue;
+        if (words.size() + st.size() >= (1ull << 32)) return false;
+        table[s] = make_uint2((uint32_t)words.size(), blocks);
+        words.insert(words.end(), st.begin(), st.end());
+        seen[hsh].push_back(s);
+        ++stored;
+    }
+    return true;
+}
+
+// Sublattice-major device order when the caller declares the basis size (spins ordered
+// cell * n_atoms + t, as the reference orders them).
+Perm csr_order(const llg_ctx* c, uint32_t na) {
+    Perm P;
+    const bool sub = na > 1 && na <= 16 && c->n % na == 0 && !(c->flags & LLG_FLAG_NO_SUBLATTICE_ORDER);
+    P.na = sub ? na : 1;
+    P.ncell = sub ? c->n / na : c->n;
+    return P;
+}
+
+}  // namespace
+
 int build_exchange_fp64(llg_ctx* c, const llg_exchange& e) {
     ExchStore& X = *c->xs;
     SLLG_TRY(validate_and_copy(c, e));
@@ -136,7 +264,22 @@ int build_exchange_fp64(llg_ctx* c, const llg_exchange& e) {
     Exch<double>& x = X.ex64;
     fill_common(x, h, c->n);
     X.encoding = "none";
-    if (h.fmt == LLG_EXCH_CSR) {
+    std::vector<uint2> utable;
+    std::vector<uint32_t> uwords;
+    uint32_t ustored = 0;
+    if (h.fmt == LLG_EXCH_CSR && build_uniform(c, h, csr_order(c, e.n_atoms), utable, uwords, ustored)) {
+        X.perm = csr_order(c, e.n_atoms);
+        uwords.resize(std::max<size_t>(uwords.size(), 4));
+        SLLG_TRY(upload(X.a, utable.data(), utable.size(), c->stream));
+        SLLG_TRY(upload(X.b, uwords.data(), uwords.size(), c->stream));
+        x.fmt = FMT_UNI;
+        x.slice = X.a.as<uint2>();
+        x.ent = X.b.as<uint32_t>();
+        x.nent = uwords.size();
+        char buf[96];
+        std::snprintf(buf, sizeof buf, "csr-uniform-t%u-f64-slices%uof%zu", X.perm.na, ustored, utable.size());
+        X.encoding = buf;
+    } else if (h.fmt == LLG_EXCH_CSR) {
         // The CSR stored by slices of 64 rows: entry q of every row of a slice at [q][lane]
         // (column-major within the slice, the slice as long as its longest row), so one load
         // of entry q by a wave is 64 consecutive words.  Each row keeps its entries in CSR
@@ -786,16 +929,7 @@ int build_exchange_fp32(llg_ctx* c, const llg_exchange& e) {
     fill_common(X.ex64, h, c->n);
     X.encoding = "none";
     if (h.fmt == LLG_EXCH_CSR) {
-        // Sublattice-major device order when the caller declares the basis size (spins
-        // ordered cell * n_atoms + t, as the reference orders them).
-        const uint32_t na = e.n_atoms;
-        if (na > 1 && na <= 16 && c->n % na == 0 && !(c->flags & LLG_FLAG_NO_SUBLATTICE_ORDER)) {
-            X.perm.na = na;
-            X.perm.ncell = c->n / na;
-        } else {
-            X.perm.na = 1;
-            X.perm.ncell = c->n;
-        }
+        X.perm = csr_order(c, e.n_atoms);
         SLLG_TRY(build_sell(c));
     } else if (h.fmt == LLG_EXCH_DIA || h.fmt == LLG_EXCH_STENCIL) {
         std::vector<float> v32(h.vals.size());

@@ -114,6 +114,46 @@ __device__ __forceinline__ void fourspin_row(const Exch<V>& e, uint32_t i, const
     }
 }
 
+// Exchange sum of row i from the lane-uniform records (FMT_UNI, FP64): entry by entry in CSR
+// order.  A record's offsets, mask and couplings are scalar; a lane takes one of the two
+// offsets and loads its neighbour's components (12 loads in flight per block).  An entry that
+// lies outside the spins ("none") loads zeros and adds couplings times zero, which changes no
+// bit of the sum.  Rows come in whole waves (row = 64 k + lane in every caller).
+// Bound by the L1, from which a wave gathers 1.5 KB a record: fcc 64^3 with 42 nnz, predictor
+// and corrector 84 us each (the sliced CSR, 12 bytes an entry and row from HBM and gathers of
+// stride 4, took 274 us for its sums alone).
+template <int NC>
+__device__ __forceinline__ void exch_row_uni(const Exch<double>& e, uint32_t i, const double* __restrict__ S,
+                                             double dot[3]) {
+    dot[0] = dot[1] = dot[2] = 0.0;
+    const u32x2 sd = cview(reinterpret_cast<const u32x2*>(e.slice))[__builtin_amdgcn_readfirstlane(i >> 6)];
+    const auto* p = cview(reinterpret_cast<const u32x4*>(e.ent + sd.x));
+    const uint32_t n8 = 8u * e.n, own = 8u * i;
+    const __amdgpu_buffer_rsrc_t rs =
+        __builtin_amdgcn_make_buffer_rsrc(const_cast<double*>(S), 0, (int)(3u * n8), 0x00020000);
+    for (uint32_t b = 0; b < sd.y; ++b, p += uni_words(NC) / 4) {
+        const u32x4 d0 = p[0], d1 = p[1], ma = p[2], mb = p[3];
+        const uint64_t mask[4] = {((uint64_t)ma.y << 32) | ma.x, ((uint64_t)ma.w << 32) | ma.z,
+                                  ((uint64_t)mb.y << 32) | mb.x, ((uint64_t)mb.w << 32) | mb.z};
+        double s[4][3], v[4][NC];
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+            const uint32_t o = __builtin_amdgcn_inverse_ballot_w64(mask[u]) ? own + d1[u] : own + d0[u];
+#pragma unroll
+            for (int a = 0; a < 3; ++a)
+                s[u][a] = __builtin_bit_cast(double, __builtin_amdgcn_raw_buffer_load_b64(rs, o, a * n8, 0));
+        }
+#pragma unroll
+        for (int w = 0; w < 2 * NC; ++w) {
+            const u32x4 q = p[4 + w];
+            v[(2 * w) / NC][(2 * w) % NC] = __builtin_bit_cast(double, ((uint64_t)q.y << 32) | q.x);
+            v[(2 * w + 1) / NC][(2 * w + 1) % NC] = __builtin_bit_cast(double, ((uint64_t)q.w << 32) | q.z);
+        }
+#pragma unroll
+        for (int u = 0; u < 4; ++u) accum<NC, double>(v[u], s[u], dot);
+    }
+}
+
 template <int NC, class R, class V, class SpinT>
 __device__ __forceinline__ void exch_row_ref(const Exch<V>& e, uint32_t i, const SpinT* __restrict__ S,
                                              R dot[3]) {

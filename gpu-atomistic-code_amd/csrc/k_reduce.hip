@@ -131,7 +131,9 @@ template <int FMT, int NC, class SpinT>
 __device__ __forceinline__ void exch_dispatch(const Exch<double>& e, uint32_t i, const SpinT* S, double dot[3]) {
     if constexpr (FMT == FMT_SELL_PACK || FMT == FMT_SELL_RAW)
         exch_row_sell64<NC, SpinT>(e, i, S, dot);
-    else if constexpr (FMT == FMT_NONE)
+    else if constexpr (FMT == FMT_UNI) {
+        if constexpr (sizeof(SpinT) == sizeof(double)) exch_row_uni<NC>(e, i, S, dot);  // FP64 handles only
+    } else if constexpr (FMT == FMT_NONE)
         dot[0] = dot[1] = dot[2] = 0.0;
     else
         exch_row_ref<NC, double, double, SpinT>(e, i, S, dot);
@@ -179,11 +181,12 @@ __global__ __launch_bounds__(kTPB) void k_energy_partial(EnergyArgs a, const Spi
     if (threadIdx.x == 0) part[blockIdx.x] = r;
 }
 
-__global__ __launch_bounds__(kTPB) void k_noise_f64(uint32_t n, uint64_t seed, uint64_t stream, uint64_t t, double* out) {
+__global__ __launch_bounds__(kTPB) void k_noise_f64(uint32_t n, Perm perm, uint64_t seed, uint64_t stream, uint64_t t,
+                                                    double* out) {
     const uint32_t i = blockIdx.x * kTPB + threadIdx.x;
     if (i >= n) return;
     double z[3];
-    normals3_f64(seed, stream, i, t, z);
+    normals3_f64(seed, stream, perm.to_ref(i), t, z);
     for (int c = 0; c < 3; ++c) out[(size_t)c * n + i] = z[c];
 }
 
@@ -493,6 +496,7 @@ int reduce_energy(llg_ctx* c, const void* dem_now, double* dev_out) {
     switch (fmt) {
         case FMT_NONE: SLLG_E(FMT_NONE, 1); break;
         case FMT_CSR: SLLG_E_NC(FMT_CSR); break;
+        case FMT_UNI: SLLG_E_NC(FMT_UNI); break;
         case FMT_DIA: SLLG_E_NC(FMT_DIA); break;
         case FMT_STENCIL: SLLG_E_NC(FMT_STENCIL); break;
         case FMT_SELL_PACK: SLLG_E_NC(FMT_SELL_PACK); break;
@@ -508,7 +512,7 @@ int reduce_energy(llg_ctx* c, const void* dem_now, double* dev_out) {
 
 int noise_sample(llg_ctx* c, uint64_t t, double* dev_out) {
     if (c->prec == LLG_FP64_PLAIN)
-        k_noise_f64<<<blocks_for(c->n, kTPB), kTPB, 0, c->stream>>>(c->n, c->seed, c->stream_id, t, dev_out);
+        k_noise_f64<<<blocks_for(c->n, kTPB), kTPB, 0, c->stream>>>(c->n, c->perm, c->seed, c->stream_id, t, dev_out);
     else
         k_noise_f32<<<blocks_for(c->n, kTPB), kTPB, 0, c->stream>>>(c->n, c->perm, c->seed, c->stream_id, t, dev_out);
     SLLG_HIP(hipGetLastError());
