@@ -58,6 +58,7 @@ struct llg_batch {
     int xcd = 1;         // XCD-aware block order
     int line = 1;        // line reader for members with a line encoding (else their packed entries)
     int g3 = 0;          // gather from AoS3 copies of S and Y (packed and line readers)
+    int small = 1;       // one-workgroup steps when every member is covered (off after llg_batch_set_launch)
     int persist = 0;     // chunks as persistent launches (grid barriers between half steps)
     int persist_graph = 1;  // with LLG_BATCH_GRAPH: capture them (0 once a capture was refused)
     bool gpersist = false;  // the captured graph holds persistent launches
@@ -152,7 +153,31 @@ int upload_tables(llg_batch* b) {
     return 0;
 }
 
+// Whether every member's chunk runs in one workgroup of its own (k_heun_small_batch): one launch
+// per group and chunk instead of two a step.
+bool small_chunk(const llg_batch* b) {
+    if (!b->small || b->persist || b->groups.empty()) return false;
+    for (const auto& g : b->groups)
+        for (int k : g->idx)
+            if (!small_applies(b->m[k].c, g->fmt)) return false;
+    return true;
+}
+
+int launch_chunk_small(llg_batch* b, uint32_t nsteps) {
+    for (auto& g : b->groups) {
+        std::vector<llg_ctx*> cs;
+        for (int k : g->idx) cs.push_back(b->m[k].c);
+        SLLG_TRY(batch_small_launch(b->stream, cs, g->dmem.p, nsteps));
+        for (llg_ctx* c : cs) {
+            c->g3_valid = false;
+            c->y_soa_valid = true;
+        }
+    }
+    return 0;
+}
+
 int launch_chunk(llg_batch* b, uint32_t nsteps, bool dipolar) {
+    if (small_chunk(b)) return launch_chunk_small(b, nsteps);
     for (auto& m : b->m)
         if (m.c) {  // what the batch kernels leave current: S3 and Y3 with the gather copy, SoA Y without
             m.c->g3_valid = b->g3 != 0;
@@ -518,12 +543,13 @@ int llg_batch_set_launch(llg_batch* b, uint32_t tpb, int xcd, int line_mode, int
     if (!b) SLLG_FAIL(LLG_E_INVALID, "NULL batch");
     if (tpb != 128 && tpb != 256 && tpb != 512) SLLG_FAIL(LLG_E_INVALID, "tile of %u threads (128, 256, 512)", tpb);
     // the captured launches have the old shape
-    if (tpb != b->tpb || (xcd ? 1 : 0) != b->xcd || (gather_copy ? 1 : 0) != b->g3) drop_graph(b);
+    if (tpb != b->tpb || (xcd ? 1 : 0) != b->xcd || (gather_copy ? 1 : 0) != b->g3 || b->small) drop_graph(b);
     b->g3 = gather_copy ? 1 : 0;
     if ((line_mode ? 1 : 0) != b->line) b->dirty = true;        // members regroup by the reader they run
     b->tpb = tpb;
     b->xcd = xcd ? 1 : 0;
     b->line = line_mode ? 1 : 0;
+    b->small = 0;  // the caller wants this shape
     return 0;
 }
 
@@ -562,7 +588,7 @@ int llg_batch_autotune(llg_batch* b, uint32_t nsteps, llg_batch_tune* out) {
             if (b->m[k].active()) b->m[k].t = t_save[k];
     };
     const uint32_t tpb0 = b->tpb;
-    const int xcd0 = b->xcd, line0 = b->line, g30 = b->g3;
+    const int xcd0 = b->xcd, line0 = b->line, g30 = b->g3, small0 = b->small;
     bool any_line = false;
     for (auto& mm : b->m) any_line = any_line || (mm.active() && is_line_fmt(mm.c->ex32.fmt));
     const int nline = any_line ? 2 : 1;
@@ -659,9 +685,12 @@ int llg_batch_autotune(llg_batch* b, uint32_t nsteps, llg_batch_tune* out) {
     if (hipStreamSynchronize(b->stream) != hipSuccess && !rc) rc = LLG_E_DEVICE;
     if (rc) {
         (void)llg_batch_set_launch(b, tpb0, xcd0, line0, g30);
+        b->small = small0;
         return rc;
     }
     SLLG_TRY(llg_batch_set_launch(b, btpb, bxcd, bline, bg3));
+    b->small = 1;  // members of one workgroup's size step there whatever the shape
+    drop_graph(b);
     out->tpb = (int)btpb;
     out->xcd = bxcd;
     out->line_mode = bline;

@@ -262,6 +262,12 @@ int do_steps(llg_ctx* c, uint64_t t0, uint32_t nsteps) {
         c->g3_valid = false;  // RK stages write S without its gather copy
         c->y_soa_valid = true;
     }
+    if (c->tune_small && small_applies(c, exec_fmt(c))) {
+        for (uint32_t k = 0; k < nsteps; k += kSmallSteps)
+            SLLG_TIMED("heun_steps", fused_heun_small(c, t0 + k, std::min(kSmallSteps, nsteps - k)));
+        if (nsteps) c->det_valid = true;
+        return 0;
+    }
     for (uint32_t k = 0; k < nsteps; ++k) {
         if (c->prec == LLG_FP64_PLAIN)
             SLLG_TRY(step_plain(c, t0 + k));
@@ -924,6 +930,7 @@ extern "C" int llg_set_launch(llg_ctx* c, int tpb, int xcd, int unroll, int ther
     c->tune_thc = thermal_cache ? 1 : 0;
     c->tune_g3 = gather_copy ? 1 : 0;
     c->tune_line = line_mode == 2 ? 2 : (line_mode ? 1 : 0);
+    c->tune_small = 0;  // the caller wants this shape
     return 0;
 }
 
@@ -954,6 +961,7 @@ extern "C" int llg_autotune(llg_ctx* c, uint32_t nsteps, llg_tune_result* out) {
             c->tune_thc = out->thermal_cache = it->second.thc;
             c->tune_g3 = out->gather_copy = it->second.g3;
             c->tune_line = out->line_mode = it->second.line;
+            c->tune_small = 1;
             out->from_cache = 1;
             return 0;
         }
@@ -993,8 +1001,9 @@ extern "C" int llg_autotune(llg_ctx* c, uint32_t nsteps, llg_tune_result* out) {
     hipEvent_t e0, e1;
     SLLG_HIP(hipEventCreate(&e0));
     SLLG_HIP(hipEventCreate(&e1));
-    const int noise = c->noise_mode;
+    const int noise = c->noise_mode, caller_small = c->tune_small;
     c->noise_mode = LLG_NOISE_COUNTER;  // no host queue traffic while timing
+    c->tune_small = 0;                  // time the shapes
     int rc = 0;
     for (size_t li = 0; li < readers.size() && !rc; ++li) {
     const int rd = readers[li];
@@ -1084,8 +1093,10 @@ extern "C" int llg_autotune(llg_ctx* c, uint32_t nsteps, llg_tune_result* out) {
         c->tune_thc = caller.thc;
         c->tune_g3 = caller.g3;
         c->tune_line = caller.line;
+        c->tune_small = caller_small;
         return rc;
     }
+    c->tune_small = 1;  // systems of one workgroup's size step there whatever the shape
     c->tune_tpb = out->tpb = b.tpb;
     c->tune_xcd = out->xcd = b.xcd;
     c->tune_unr = out->unroll = b.unr;

@@ -25,6 +25,12 @@ constexpr int kTPB = 256;       // threads per block of the per-spin kernels
 constexpr int kSlice = 64;      // sliced-ELL slice height = one wavefront
 constexpr int kMaxSub = 16;     // sublattices reduced on the device
 constexpr int kDictLds = 2048;  // floats of coupling dictionary staged in LDS (8 KB)
+// Largest system of the one-workgroup Heun steps (two rows a thread), and the most entries of
+// one whose rows are too long for registers (small_applies).
+constexpr uint32_t kSmallSpins = 2048;
+constexpr uint64_t kSmallEntries = 1024 * 42;
+// Steps of one such launch (some 20 ms at most).
+constexpr uint32_t kSmallSteps = 4096;
 
 // Line-mode group records: line_group(nc) neighbour windows per record, line_words(nc) words
 // (the group's shift mask, its window starts, 3 shifts x nc couplings per window, the next
@@ -200,6 +206,7 @@ struct ExchStore {
     Exch<double> ex64;
     Perm perm;
     std::string encoding;
+    uint32_t len_max = 0;  // longest row of the packed entries
     HostExch h;  // scalars kept; the large host vectors are released after upload
     uint64_t bytes() const {
         return a.bytes + b.bytes + c.bytes + d.bytes + e.bytes + f.bytes + g.bytes + dict64.bytes + fs_x.bytes +
@@ -238,6 +245,7 @@ struct llg_ctx {
     int tune_thc = 1;    // predictor hands its thermal field to the corrector (llg_autotune)
     int tune_g3 = 1;     // gather neighbours from the AoS3 copy of the spins (llg_autotune)
     int tune_line = 1;   // line encodings: 0 packed entries, 1 line reader, 2 tile reader (llg_autotune)
+    int tune_small = 1;  // one-workgroup steps for systems they cover (off after llg_set_launch)
     bool g3_valid = false;   // S3 holds the current S
     bool s_soa_valid = true;  // S (SoA) holds the current spins (else only S3 does: see sync_spins)
     bool y_soa_valid = true;  // Y (SoA) holds the last predictor output (else only Y3 does)

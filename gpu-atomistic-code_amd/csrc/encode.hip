@@ -777,6 +777,7 @@ int build_sell(llg_ctx* c) {
     uint64_t tot = 0;
     for (uint32_t s = 0; s < nsl; ++s) {
         slice[s].y = pack ? (mx[s] + 1u) / 2u * 2u : mx[s];
+        X.len_max = std::max(X.len_max, slice[s].y);
         slice[s].x = (uint32_t)tot;
         tot += slice[s].y;
     }

@@ -482,9 +482,11 @@ __device__ __forceinline__ void thermal_field(const FusedArgs& a, uint32_t i, ui
 // and the LLG right-hand side.  The thermal field is drawn here, after the exchange: a
 // global store (the predictor's hand-off of its draw) before the exchange would make the
 // compiler read the read-only coupling streams with vector instead of scalar loads.
-template <bool EDEM>
+// TH: 0 the thermal field is drawn or read here, 1 the same and kept in th, 2 taken from th.
+template <bool EDEM, int TH = 0>
 __device__ __forceinline__ void fused_tail(const FusedArgs& a, uint32_t i, uint32_t iref, const float* __restrict__ src,
-                                           const float s[3], float h[3], float hd[3], float f[3], uint64_t t) {
+                                           const float s[3], float h[3], float hd[3], float f[3], uint64_t t,
+                                           float* keep = nullptr) {
     const uint32_t n = a.n;
     if (a.ex.fs_xadj) {
         float h4[3];
@@ -511,7 +513,18 @@ __device__ __forceinline__ void fused_tail(const FusedArgs& a, uint32_t i, uint3
     const Species<float> sp = species_of(a, i);
     if (a.noise) {
         float th[3];
-        thermal_field(a, i, iref, sp, t, th);
+        if constexpr (TH == 2) {
+            th[0] = keep[0];
+            th[1] = keep[1];
+            th[2] = keep[2];
+        } else {
+            thermal_field(a, i, iref, sp, t, th);
+        }
+        if constexpr (TH == 1) {
+            keep[0] = th[0];
+            keep[1] = th[1];
+            keep[2] = th[2];
+        }
         h[0] += th[0];
         h[1] += th[1];
         h[2] += th[2];
@@ -1019,6 +1032,184 @@ __global__ __launch_bounds__(TPB) void k_heun_batch_persist(const BatchMember* _
     }
 }
 
+// ---------------------------------------------------------------- small systems
+// Up to kSmallSpins spins on the packed entries (or without exchange): one workgroup advances
+// the system nsteps steps in one launch, with the spins in LDS (S and Y, [component][spin]),
+// A and the step's thermal field in registers, and a workgroup barrier between the half steps.
+// Two launches a step cost such a system about 8 us whatever its size; here a step costs what
+// one CU computes, and the noise is drawn once instead of twice.  Every row does what
+// k_heun_pred and k_heun_corr do, in the same order, so the bits are theirs.
+// 10^3 simple cubic at 300 K: 9.2 -> 2.2 us a step.
+// REG: rows of at most kSmallLen entries, whose LDS addresses and (NC = 1) couplings stay in
+// registers over the steps; longer rows are read from the packed stream every half step.
+constexpr uint32_t kSmallLen = 8;
+
+template <int NC, bool REG>
+struct SmallRow {
+    uint32_t w[REG ? kSmallLen : 1];               // LDS index, dictionary index << 16 (NC > 1)
+    float v[REG && NC == 1 ? kSmallLen : 1];
+    uint32_t len;
+};
+
+template <int NC, bool REG>
+__device__ __forceinline__ void small_load(const Exch<float>& e, uint32_t i, bool wave_live, const float* sdict,
+                                           SmallRow<NC, REG>& r) {
+    r.len = 0;
+    if (!wave_live || e.fmt == FMT_NONE) return;
+    const uint32_t lane = i & 63u;
+    const u32x2 sd = cview(reinterpret_cast<const u32x2*>(e.slice))[__builtin_amdgcn_readfirstlane(i >> 6)];
+    r.len = sd.y;
+    if constexpr (REG) {
+        const auto* ent = gview(e.ent) + (size_t)sd.x * kSlice;
+#pragma unroll
+        for (uint32_t q = 0; q < kSmallLen; ++q)
+            if (q < sd.y) {
+                const uint32_t w = ent[pack_pos(q, lane, sd.y)], k = pack_dict(w, e.dbits);
+                r.w[q] = pack_nb(w, i, e.dbits);
+                if constexpr (NC == 1)
+                    r.v[q] = sdict[k];
+                else
+                    r.w[q] |= k << 16;
+            }
+    }
+}
+
+template <int NC>
+__device__ __forceinline__ void small_entry(uint32_t j, const float* v, const float* sp, float dot[3]) {
+    const float s[3] = {sp[j], sp[kSmallSpins + j], sp[2 * kSmallSpins + j]};
+    float c[NC];
+#pragma unroll
+    for (int k = 0; k < NC; ++k) c[k] = v[k];
+    accum<NC, float>(c, s, dot);
+}
+
+template <int NC, bool REG>
+__device__ __forceinline__ void small_exch(const Exch<float>& e, uint32_t i, const SmallRow<NC, REG>& r,
+                                           const float* sdict, const float* sp, float dot[3]) {
+    dot[0] = dot[1] = dot[2] = 0.0f;
+    const uint32_t len = __builtin_amdgcn_readfirstlane(r.len);
+    if constexpr (REG) {
+#pragma unroll
+        for (uint32_t q = 0; q < kSmallLen; ++q)
+            if (q < len) {
+                if constexpr (NC == 1)
+                    small_entry<1>(r.w[q], &r.v[q], sp, dot);
+                else
+                    small_entry<NC>(r.w[q] & 0xFFFFu, sdict + (r.w[q] >> 16) * NC, sp, dot);
+            }
+    } else if (len) {
+        const u32x2 sd = cview(reinterpret_cast<const u32x2*>(e.slice))[__builtin_amdgcn_readfirstlane(i >> 6)];
+        const auto* ent = gview(e.ent) + (size_t)sd.x * kSlice;
+        const uint32_t lane = i & 63u;
+        auto one = [&](uint32_t w) {
+            small_entry<NC>(pack_nb(w, i, e.dbits), sdict + pack_dict(w, e.dbits) * NC, sp, dot);
+        };
+        const uint32_t full = len & ~3u;
+#pragma unroll 2
+        for (uint32_t q = 0; q < full; q += 4) {
+            const u32x4 w = *(const __attribute__((address_space(1))) u32x4*)(ent + pack_pos(q, lane, len));
+            one(w.x);
+            one(w.y);
+            one(w.z);
+            one(w.w);
+        }
+        for (uint32_t q = full; q < len; ++q) one(ent[pack_pos(q, lane, len)]);
+    }
+}
+
+template <int NC, int RPT, bool REG>
+__device__ __forceinline__ void small_run(const FusedArgs& a, float* __restrict__ S, float* __restrict__ Y,
+                                          uint64_t t0, uint32_t nsteps) {
+    __shared__ float ls[3 * kSmallSpins], ly[3 * kSmallSpins], sdict[kDictLds];
+    const uint32_t n = a.n;
+    for (uint32_t k = threadIdx.x; k < a.ex.ndict * NC; k += blockDim.x) sdict[k] = gview(a.ex.dict)[k];
+    __syncthreads();
+    uint32_t row[RPT], iref[RPT];
+    bool live[RPT];
+    float s[RPT][3], A[RPT][3], th[RPT][3];
+    SmallRow<NC, REG> e[RPT];
+#pragma unroll
+    for (int k = 0; k < RPT; ++k) {
+        const uint32_t i = row[k] = threadIdx.x + (uint32_t)k * blockDim.x;
+        live[k] = i < n;
+        iref[k] = a.perm.to_ref(i);
+        small_load<NC, REG>(a.ex, i, __builtin_amdgcn_readfirstlane(i & ~63u) < n, sdict, e[k]);
+#pragma unroll
+        for (int c = 0; c < 3; ++c) {
+            s[k][c] = live[k] ? gview(S)[(size_t)c * n + i] : 0.0f;
+            A[k][c] = th[k][c] = 0.0f;
+            if (i < kSmallSpins) ls[c * kSmallSpins + i] = s[k][c];
+        }
+    }
+    __syncthreads();
+    for (uint32_t q = 0; q < nsteps; ++q) {
+        const uint64_t t = t0 + q;
+#pragma unroll
+        for (int k = 0; k < RPT; ++k) {
+            const uint32_t i = row[k];
+            float h[3], hd[3] = {0.f, 0.f, 0.f}, f[3], y[3];
+            small_exch<NC, REG>(a.ex, i, e[k], sdict, ls, h);
+            if (live[k]) {
+                fused_tail<false, 1>(a, i, iref[k], S, s[k], h, hd, f, t, th[k]);
+#pragma unroll
+                for (int c = 0; c < 3; ++c) y[c] = s[k][c] + a.rdt * f[c];
+                const float r = rsqrtf(y[0] * y[0] + y[1] * y[1] + y[2] * y[2]);
+#pragma unroll
+                for (int c = 0; c < 3; ++c) {
+                    A[k][c] = s[k][c] + a.half_rdt * f[c];
+                    s[k][c] = y[c] * r;  // this row's predicted spin until the corrector
+                    ly[c * kSmallSpins + i] = s[k][c];
+                }
+            }
+        }
+        __syncthreads();
+        if (q + 1 == nsteps) {  // the last predictor output stays readable (llg_get_det_field)
+#pragma unroll
+            for (int k = 0; k < RPT; ++k)
+                if (live[k]) {
+#pragma unroll
+                    for (int c = 0; c < 3; ++c) gview(Y)[(size_t)c * n + row[k]] = s[k][c];
+                }
+        }
+#pragma unroll
+        for (int k = 0; k < RPT; ++k) {
+            const uint32_t i = row[k];
+            float h[3], hd[3] = {0.f, 0.f, 0.f}, f[3], p[3];
+            small_exch<NC, REG>(a.ex, i, e[k], sdict, ly, h);
+            if (live[k]) {
+                fused_tail<false, 2>(a, i, iref[k], Y, s[k], h, hd, f, t, th[k]);
+#pragma unroll
+                for (int c = 0; c < 3; ++c) p[c] = A[k][c] + a.half_rdt * f[c];
+                const float r = rsqrtf(p[0] * p[0] + p[1] * p[1] + p[2] * p[2]);
+#pragma unroll
+                for (int c = 0; c < 3; ++c) {
+                    s[k][c] = p[c] * r;
+                    ls[c * kSmallSpins + i] = s[k][c];
+                }
+            }
+        }
+        __syncthreads();
+    }
+#pragma unroll
+    for (int k = 0; k < RPT; ++k)
+        if (live[k]) {
+#pragma unroll
+            for (int c = 0; c < 3; ++c) gview(S)[(size_t)c * n + row[k]] = s[k][c];
+        }
+}
+
+template <int NC, int RPT, bool REG>
+__global__ __launch_bounds__(1024) void k_heun_small(FusedArgs a, float* S, float* Y, uint32_t nsteps) {
+    small_run<NC, RPT, REG>(a, S, Y, a.t, nsteps);
+}
+
+// One block per member.
+template <int NC, int RPT, bool REG>
+__global__ __launch_bounds__(1024) void k_heun_small_batch(const BatchMember* __restrict__ mem, uint32_t nsteps) {
+    const BatchMember& bm = mem[blockIdx.x];
+    small_run<NC, RPT, REG>(bm.a, bm.S, bm.Y, bm.t0, nsteps);
+}
+
 // RK4: stage m reads Yin (S for m = 0), k = rdt f(Yin);
 //   m0: ACC = k/6, Yout = S + k/2;  m1: ACC += k/3, Yout = S + k/2;  m2: ACC += k/3, Yout = S + k;
 //   m3: S = N(S + ACC + k/6).
@@ -1437,6 +1628,70 @@ int fused_heun_corr(llg_ctx* c, const StepSched& s) {
     SLLG_HIP(hipGetLastError());
     c->g3_valid = g3;  // S3 is current only if the corrector wrote it
     c->s_soa_valid = ssoa;
+    return 0;
+}
+
+#define SLLG_SMALL(NC_VAL, TWO, REG_VAL, MACRO)                                          \
+    do {                                                                                 \
+        const bool two_ = (TWO), reg_ = (REG_VAL);                                       \
+        if ((NC_VAL) == 1) {                                                             \
+            if (two_) { if (reg_) { MACRO(1, 2, true); } else { MACRO(1, 2, false); } }  \
+            else { if (reg_) { MACRO(1, 1, true); } else { MACRO(1, 1, false); } }       \
+        } else if ((NC_VAL) == 3) {                                                      \
+            if (two_) { if (reg_) { MACRO(3, 2, true); } else { MACRO(3, 2, false); } }  \
+            else { if (reg_) { MACRO(3, 1, true); } else { MACRO(3, 1, false); } }       \
+        } else {                                                                         \
+            if (two_) { if (reg_) { MACRO(9, 2, true); } else { MACRO(9, 2, false); } }  \
+            else { if (reg_) { MACRO(9, 1, true); } else { MACRO(9, 1, false); } }       \
+        }                                                                                \
+    } while (0)
+
+// What the one-workgroup steps cover, for a reader of format fmt: no dipolar refresh (other
+// kernels in the step), no four-spin term, counter noise.
+// One CU computes what the launches spread over the GPU, so the work is bounded: rows whose
+// entries stay in registers up to kSmallSpins (two a thread; simple cubic, 300 K: 10^3 spins
+// 2.2 us a step against 9.2 with two launches, 12^3 4.4 against 9.3), longer ones up to one row
+// a thread and kSmallEntries in all (fcc, 42 entries: 840 spins 9.3 us against 12.4, but 2,048
+// spins 16.8 against 13.2).
+bool small_applies(const llg_ctx* c, int fmt) {
+    if (c->prec != LLG_FP32 || c->scheme != LLG_HEUN || c->dip || c->ex32.fs_xadj ||
+        c->noise_mode != LLG_NOISE_COUNTER || (fmt != FMT_SELL_PACK && fmt != FMT_NONE))
+        return false;
+    const uint32_t len = c->xs->len_max;
+    return len <= kSmallLen ? c->n <= kSmallSpins : c->n <= 1024u && (uint64_t)c->n * len <= kSmallEntries;
+}
+
+static int small_nc(const llg_ctx* c) { return c->ex32.fmt == FMT_NONE ? 1 : c->ex32.ncomp; }
+
+// nsteps Heun steps from step t0; the spins are left in S, the last predictor output in Y.
+int fused_heun_small(llg_ctx* c, uint64_t t0, uint32_t nsteps) {
+    SLLG_TRY(sync_spins(c));
+    const FusedArgs a = fused_args(c, StepSched{t0, nullptr});
+    const bool two = c->n > 1024;
+    const uint32_t tpb = two ? 1024u : (c->n + 63u) / 64u * 64u;
+#define SLLG_L(N, P, G) \
+    k_heun_small<N, P, G><<<1, tpb, 0, c->stream>>>(a, c->S.as<float>(), c->Y.as<float>(), nsteps)
+    SLLG_SMALL(small_nc(c), two, c->xs->len_max <= kSmallLen, SLLG_L);
+#undef SLLG_L
+    SLLG_HIP(hipGetLastError());
+    c->g3_valid = false;
+    c->s_soa_valid = c->y_soa_valid = true;
+    return 0;
+}
+
+// The same for the members of a batch group (its table built without gather copies).
+int batch_small_launch(hipStream_t s, const std::vector<llg_ctx*>& members, const void* dmem, uint32_t nsteps) {
+    if (members.empty()) return 0;
+    bool two = false, reg = true;
+    for (const llg_ctx* c : members) {
+        two = two || c->n > 1024;
+        reg = reg && c->xs->len_max <= kSmallLen;
+    }
+    const BatchMember* m = static_cast<const BatchMember*>(dmem);
+#define SLLG_L(N, P, G) k_heun_small_batch<N, P, G><<<(unsigned)members.size(), 1024, 0, s>>>(m, nsteps)
+    SLLG_SMALL(small_nc(members[0]), two, reg, SLLG_L);
+#undef SLLG_L
+    SLLG_HIP(hipGetLastError());
     return 0;
 }
 

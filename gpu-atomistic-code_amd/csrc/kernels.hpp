@@ -20,6 +20,9 @@ struct StepSched {
 };
 int fused_heun_pred(llg_ctx* c, const StepSched& s);
 int fused_heun_corr(llg_ctx* c, const StepSched& s);
+bool small_applies(const llg_ctx* c, int fmt);  // one-workgroup steps cover the handle (reader of format fmt)
+int fused_heun_small(llg_ctx* c, uint64_t t0, uint32_t nsteps);
+int batch_small_launch(hipStream_t s, const std::vector<llg_ctx*>& members, const void* dmem, uint32_t nsteps);
 int fused_y_soa(llg_ctx* c);  // rebuild the SoA predictor output from its AoS3 copy
 int sync_spins(llg_ctx* c);
 int reduce_mag_noalloc(llg_ctx* c, double* m);  // <M> per sublattice through the device scratch array   // rebuild the SoA spins from their AoS3 copy when only that is current
