@@ -65,7 +65,7 @@ struct llg_batch {
     uint32_t spin_limit = LLG_BATCH_SPIN_DEFAULT;  // polls per grid-barrier wait
     DevBuf bar;          // GridBar of the persistent launches
     uint32_t persist_grid = 0;  // blocks of the last persistent launch
-    DevBuf red;
+    DevBuf red, red_work;  // sampled <M> of a call; its member table and partial sums
     std::vector<std::shared_ptr<ExchStore>> pinned;  // coupling stores kept for future members
     std::map<const ExchStore*, uint64_t> store_est;  // admission estimate of each coupling store
 };
@@ -253,6 +253,30 @@ int launch_chunk_persistent(llg_batch* b, uint32_t nsteps, bool dipolar) {
     return 0;
 }
 
+// <M> (3 doubles a member: requests have one sublattice) of the members listed, then the structure
+// factor of those with sq set, whose first double in `out` goes to sq_at: every launch is
+// enqueued, then one copy and one wait fetch all of it.
+int sample_members(llg_batch* b, const std::vector<int>& members, const std::vector<char>& sq,
+                   std::vector<size_t>& sq_at, std::vector<double>& out) {
+    std::vector<llg_ctx*> cs;
+    size_t cnt = 3 * members.size();
+    sq_at.assign(members.size(), 0);
+    for (size_t k = 0; k < members.size(); ++k) {
+        llg_ctx* c = b->m[members[k]].c;
+        cs.push_back(c);
+        sq_at[k] = cnt;
+        if (sq[k]) cnt += (size_t)c->sq_ngroups * c->sq_nk * 2;
+    }
+    out.resize(cnt);
+    if (b->red.bytes < cnt * sizeof(double)) SLLG_TRY(b->red.alloc(2 * cnt * sizeof(double)));
+    SLLG_TRY(batch_reduce_mag(b->stream, cs, b->red.as<double>(), 3, b->red_work));
+    for (size_t k = 0; k < members.size(); ++k)
+        if (sq[k]) SLLG_TRY(sample_sq(cs[k], b->red.as<double>() + sq_at[k]));
+    SLLG_HIP(hipMemcpyAsync(out.data(), b->red.p, cnt * sizeof(double), hipMemcpyDeviceToHost, b->stream));
+    SLLG_HIP(hipStreamSynchronize(b->stream));
+    return 0;
+}
+
 int check_member(llg_batch* b, int k) {
     if (!b || k < 0 || (size_t)k >= b->m.size() || !b->m[k].live) SLLG_FAIL(LLG_E_INVALID, "no such member %d", k);
     return 0;
@@ -328,6 +352,7 @@ void llg_batch_destroy(llg_batch* b) {
         if (mm.c) llg_destroy(mm.c);
     b->groups.clear();
     b->red.release();
+    b->red_work.release();
     (void)hipStreamDestroy(b->stream);
     delete b;
 }
@@ -705,12 +730,14 @@ int llg_batch_reduce(llg_batch* b, const int* members, uint32_t count, uint32_t 
     SLLG_HIP(hipSetDevice(b->device));
     const size_t need = (size_t)count * stride * sizeof(double);
     if (b->red.bytes < need) SLLG_TRY(b->red.alloc(need * 2));
+    std::vector<llg_ctx*> cs;
     for (uint32_t k = 0; k < count; ++k) {
         SLLG_TRY(check_member(b, members[k]));
         llg_ctx* c = b->m[members[k]].c;
         if (c->nsub * 3 > stride) SLLG_FAIL(LLG_E_INVALID, "stride %u < 3 x sublattices of member %d", stride, members[k]);
-        SLLG_TRY(reduce_mag(c, b->red.as<double>() + (size_t)k * stride));
+        cs.push_back(c);
     }
+    SLLG_TRY(batch_reduce_mag(b->stream, cs, b->red.as<double>(), stride, b->red_work));
     SLLG_HIP(hipMemcpyAsync(m, b->red.p, need, hipMemcpyDeviceToHost, b->stream));
     SLLG_HIP(hipStreamSynchronize(b->stream));
     return 0;
@@ -1033,16 +1060,24 @@ extern "C" int llg_serve_run(const llg_serve_config* cfg, const llg_request* req
             }
             // samples due before this chunk (every `update` steps, before the step)
             std::vector<int> due;
+            std::vector<char> due_sq;
             for (auto& lv : live)
-                if (lv.done % reqs[lv.req].update == 0) due.push_back(lv.member);
+                if (lv.done % reqs[lv.req].update == 0) {
+                    due.push_back(lv.member);
+                    due_sq.push_back(reqs[lv.req].type == LLG_REQ_SW);
+                }
             if (!due.empty()) {
-                std::vector<double> m(due.size() * 3);
-                SLLG_TRY(llg_batch_reduce(b, due.data(), (uint32_t)due.size(), 3, m.data()));
+                std::vector<double> m;
+                std::vector<size_t> sq_at;
+                SLLG_TRY(sample_members(b, due, due_sq, sq_at, m));
                 size_t k = 0;
                 for (auto& lv : live)
                     if (lv.done % reqs[lv.req].update == 0) {
-                        // the batch's launches are complete (the reduction synchronised its stream)
-                        SLLG_TRY(sw_sample(reqs[lv.req], (uint32_t)lv.req, lv.samples, b->m[lv.member].c));
+                        if (due_sq[k] && sq_series) {
+                            const uint64_t nk = reqs[lv.req].L / 2 + 1;
+                            std::memcpy(sq_series + sq_offset[lv.req] + (uint64_t)lv.samples * 2 * nk, &m[sq_at[k]],
+                                        2 * nk * sizeof(double));
+                        }
                         record_sample(reqs[lv.req], lv, &m[3 * k], results[lv.req], m_series, series_offset);
                         ++k;
                         if (reqs[lv.req].type == LLG_REQ_RAMP) {

@@ -94,6 +94,9 @@ __global__ __launch_bounds__(kTPB) void k_to_ref(uint32_t n, Perm perm, const T*
 // loop, an FP64 field fetched in 2.0 instead of 8.8); below it three kernels and copies take
 // longer than the loop (10^3 spins: 58 us against 28).
 constexpr uint32_t kIoDevice = 65536;
+// Largest <M> series of llg_run_sampled whose device buffer the handle keeps (1365 samples of one
+// sublattice): an allocation and its release cost a short run some 30 us.
+constexpr size_t kSeriesKeep = 32768;
 // n doubles of device memory that are free between steps: the FP32 path's A, the FP64 path's H
 // (both only carry values within a step).
 double* io_scratch(const llg_ctx* c) { return c->prec == LLG_FP64_PLAIN ? c->H.as<double>() : c->A.as<double>(); }
@@ -659,23 +662,23 @@ int llg_get_field(llg_ctx* c, double* hx, double* hy, double* hz) {
 int llg_reduce(llg_ctx* c, double* m, double* energy) {
     if (!c || !m) SLLG_FAIL(LLG_E_INVALID, "NULL argument");
     SLLG_HIP(hipSetDevice(c->device));
-    DevBuf out;
-    SLLG_TRY(out.alloc((c->nsub * 3 + 1) * sizeof(double)));
-    SLLG_TRY(reduce_mag(c, out.as<double>()));
+    double *dm = nullptr, *de = nullptr;
+    SLLG_TRY(reduce_result(c, &dm, &de));
+    SLLG_TRY(reduce_mag(c, dm));
+    DevBuf dem;
     if (energy) {
-        DevBuf dem;
         if (c->dip) {
             SLLG_TRY(dem.alloc(3 * (size_t)c->n * prec_bytes(c)));
             SLLG_TRY(dipolar_refresh(c, c->S.p, dem.p));
         }
-        SLLG_TRY(reduce_energy(c, c->dip ? dem.p : nullptr, out.as<double>() + c->nsub * 3));
-        SLLG_HIP(hipStreamSynchronize(c->stream));
+        SLLG_TRY(reduce_energy(c, c->dip ? dem.p : nullptr, de));
     }
-    std::vector<double> h(c->nsub * 3 + 1);
-    SLLG_HIP(hipMemcpyAsync(h.data(), out.p, h.size() * 8, hipMemcpyDeviceToHost, c->stream));
+    double h[3 * kMaxSub + 1];
+    const size_t cnt = energy ? (size_t)(de - dm) + 1 : (size_t)c->nsub * 3;
+    SLLG_HIP(hipMemcpyAsync(h, dm, cnt * sizeof(double), hipMemcpyDeviceToHost, c->stream));
     SLLG_HIP(hipStreamSynchronize(c->stream));
-    std::memcpy(m, h.data(), c->nsub * 3 * 8);
-    if (energy) *energy = h[c->nsub * 3];
+    std::memcpy(m, h, c->nsub * 3 * 8);
+    if (energy) *energy = h[de - dm];
     return 0;
 }
 
@@ -723,10 +726,8 @@ int llg_sample_sq(llg_ctx* c, double* out) {
     if (c->sq_nk == 0) SLLG_FAIL(LLG_E_STATE, "no k-points set (llg_set_sq)");
     SLLG_HIP(hipSetDevice(c->device));
     const size_t cnt = (size_t)c->sq_ngroups * c->sq_nk * 2;
-    DevBuf d;
-    SLLG_TRY(d.alloc(cnt * sizeof(double)));
-    SLLG_TRY(sample_sq(c, d.as<double>()));
-    SLLG_HIP(hipMemcpyAsync(out, d.p, cnt * sizeof(double), hipMemcpyDeviceToHost, c->stream));
+    SLLG_TRY(sample_sq(c, c->sq_out.as<double>()));
+    SLLG_HIP(hipMemcpyAsync(out, c->sq_out.p, cnt * sizeof(double), hipMemcpyDeviceToHost, c->stream));
     SLLG_HIP(hipStreamSynchronize(c->stream));
     return 0;
 }
@@ -736,8 +737,11 @@ int llg_run_sampled(llg_ctx* c, uint64_t t0, uint32_t nsteps, uint32_t every, do
     SLLG_HIP(hipSetDevice(c->device));
     const uint32_t nrec = (nsteps + every - 1) / every;
     const size_t rec = (size_t)c->nsub * 3;
-    DevBuf ser;
-    SLLG_TRY(ser.alloc(std::max<size_t>(1, nrec) * rec * sizeof(double)));
+    // short series use a workspace the handle keeps, long ones one of their own
+    const size_t bytes = std::max<size_t>(1, nrec) * rec * sizeof(double);
+    DevBuf own;
+    DevBuf& ser = bytes <= kSeriesKeep ? c->m_series : own;
+    if (ser.bytes < bytes) SLLG_TRY(ser.alloc(bytes <= kSeriesKeep ? kSeriesKeep : bytes));
     uint32_t r = 0;
     for (uint32_t s = 0; s < nsteps; s += every) {
         SLLG_TRY(reduce_mag(c, ser.as<double>() + (size_t)r * rec));
@@ -800,7 +804,7 @@ int llg_get_info(llg_ctx* c, llg_info* info) {
     DevBuf* all[] = {&c->S, &c->Y, &c->A, &c->H, &c->FN, &c->DET, &c->XI, &c->STG, &c->STG0, &c->DEM,
                      &c->K[0], &c->K[1], &c->K[2], &c->K[3], &c->K[4], &c->K[5], &c->spec, &c->sub,
                      &c->sp32, &c->sp64d, &c->p_sigma, &c->p_llgpf, &c->p_lambda, &c->p_k1u, &c->p_k1udir,
-                     &c->p_kc, &c->red_part, &c->red_out};
+                     &c->p_kc, &c->red_part, &c->red_out, &c->m_series, &c->sq_out};
     for (DevBuf* b : all) dev += b->bytes;
     info->device_bytes = dev + dipolar_bytes(c) + (c->xs ? c->xs->bytes() : 0);
     std::snprintf(info->exch_encoding, sizeof info->exch_encoding, "%s", c->xs ? c->xs->encoding.c_str() : "none");

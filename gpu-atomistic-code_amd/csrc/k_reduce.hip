@@ -38,10 +38,9 @@ __device__ __forceinline__ double block_sum(double v, double* lds) {
 }
 
 template <class SpinT>
-__global__ __launch_bounds__(kTPB) void k_mag_partial(uint32_t n, uint32_t nsub, const SpinT* __restrict__ S,
-                                                      const uint8_t* __restrict__ sub, double* __restrict__ part) {
-    __shared__ double lds[kTPB / 64];
-    const uint32_t stride = gridDim.x * kTPB;
+__device__ __forceinline__ void mag_partial(uint32_t n, uint32_t nsub, uint32_t nblocks, const SpinT* __restrict__ S,
+                                            const uint8_t* __restrict__ sub, double* __restrict__ part, double* lds) {
+    const uint32_t stride = nblocks * kTPB;
     for (uint32_t s = 0; s < nsub; ++s) {
         double a[3] = {0.0, 0.0, 0.0};
         for (uint32_t i = blockIdx.x * kTPB + threadIdx.x; i < n; i += stride) {
@@ -57,16 +56,59 @@ __global__ __launch_bounds__(kTPB) void k_mag_partial(uint32_t n, uint32_t nsub,
     }
 }
 
-// out[v] = scale[v / 3] * sum_b part[b][v]
-__global__ __launch_bounds__(kTPB) void k_sum_partials(uint32_t nblocks, uint32_t nval, const double* __restrict__ part,
-                                                       const double* __restrict__ scale, double* __restrict__ out) {
+template <class SpinT>
+__global__ __launch_bounds__(kTPB) void k_mag_partial(uint32_t n, uint32_t nsub, const SpinT* __restrict__ S,
+                                                      const uint8_t* __restrict__ sub, double* __restrict__ part) {
     __shared__ double lds[kTPB / 64];
+    mag_partial<SpinT>(n, nsub, gridDim.x, S, sub, part, lds);
+}
+
+// Factors of a sum's values by sublattice (1 / its spins for <M>), passed with the launch.
+struct SubScale {
+    double v[kMaxSub];
+};
+
+// out[v] = scale[v / 3] * sum_b part[b][v]
+__device__ __forceinline__ void sum_partials(uint32_t nblocks, uint32_t nval, const double* __restrict__ part,
+                                             const double* scale, double* __restrict__ out, double* lds) {
     for (uint32_t v = 0; v < nval; ++v) {
         double a = 0.0;
         for (uint32_t b = threadIdx.x; b < nblocks; b += kTPB) a += part[(size_t)b * nval + v];
         const double r = block_sum(a, lds);
-        if (threadIdx.x == 0) out[v] = r * (scale ? scale[v / 3] : 1.0);
+        if (threadIdx.x == 0) out[v] = r * scale[v / 3];
     }
+}
+
+__global__ __launch_bounds__(kTPB) void k_sum_partials(uint32_t nblocks, uint32_t nval, const double* __restrict__ part,
+                                                       SubScale scale, double* __restrict__ out) {
+    __shared__ double lds[kTPB / 64];
+    sum_partials(nblocks, nval, part, scale.v, out, lds);
+}
+
+// <M> of many FP32 systems in one pair of launches.  A system alone keeps the chip busy for
+// some 3 us but costs two launches of 3.6 us each: the members' blocks share a grid, block
+// row blockIdx.y being member blockIdx.y, with the blocks, strides and order of sums of the
+// single-system kernels (the same bits).
+struct MagMember {
+    const float* S;
+    const uint8_t* sub;  // sublattice per spin, null for one
+    double* part;
+    double* out;
+    uint32_t n, nsub, nblocks, pad_;
+    SubScale scale;
+};
+
+__global__ __launch_bounds__(kTPB) void k_mag_batch_partial(const MagMember* __restrict__ mem) {
+    const MagMember& m = mem[blockIdx.y];
+    if (blockIdx.x >= m.nblocks) return;
+    __shared__ double lds[kTPB / 64];
+    mag_partial<float>(m.n, m.nsub, m.nblocks, m.S, m.sub, m.part, lds);
+}
+
+__global__ __launch_bounds__(kTPB) void k_mag_batch_sum(const MagMember* __restrict__ mem) {
+    __shared__ double lds[kTPB / 64];
+    const MagMember& m = mem[blockIdx.x];
+    sum_partials(m.nblocks, m.nsub * 3, m.part, m.scale.v, m.out, lds);
 }
 
 // Per-spin energy (J) in FP64:
@@ -367,12 +409,27 @@ __global__ __launch_bounds__(kTPB) void k_sq_finish(SqArgs a, uint32_t ngroups, 
 
 // ---------------------------------------------------------------- host launchers
 
+// A handle's red_out, in doubles: <M> per sublattice [0, 48), the energy, the flag of
+// check_finite [63], the species' moments from kRedMu.
+constexpr size_t kRedEnergy = kMaxSub * 3, kRedMu = 64;
+static_assert(kRedEnergy < 63, "red_out layout");
+constexpr size_t kGridRows = 65535;
+
 static int ensure_red(llg_ctx* c) {
     const size_t need = (size_t)kRedBlocks * (size_t)std::max<uint32_t>(c->nsub * 3, 1) * sizeof(double);
     if (c->red_part.bytes < need) SLLG_TRY(c->red_part.alloc(need));
-    if (c->red_out.bytes < 64 * sizeof(double) + kMaxSub * sizeof(double) + 64 * sizeof(double))
-        SLLG_TRY(c->red_out.alloc(64 * sizeof(double) + kMaxSub * sizeof(double) + 64 * sizeof(double)));
+    if (!c->red_out.p) {
+        SLLG_TRY(c->red_out.alloc((kRedMu + std::max<size_t>(64, c->mu_sp.size())) * sizeof(double)));
+        SLLG_HIP(hipMemcpyAsync(c->red_out.as<double>() + kRedMu, c->mu_sp.data(), c->mu_sp.size() * sizeof(double),
+                                hipMemcpyHostToDevice, c->stream));
+    }
     return 0;
+}
+
+static SubScale inverse_counts(const llg_ctx* c) {
+    SubScale s{};
+    for (uint32_t k = 0; k < c->nsub; ++k) s.v[k] = c->sub_count[k] ? 1. / (double)c->sub_count[k] : 0.0;
+    return s;
 }
 
 static unsigned red_blocks(uint32_t n) { return std::min<unsigned>(kRedBlocks, std::max<unsigned>(1, blocks_for(n, kTPB))); }
@@ -382,18 +439,63 @@ int reduce_mag(llg_ctx* c, double* dev_out) {
     SLLG_TRY(ensure_red(c));
     const unsigned nb = red_blocks(c->n);
     const uint8_t* sub = (c->nsub > 1) ? c->sub.as<uint8_t>() : nullptr;
-    // inverse sublattice counts live after the first 64 doubles of red_out
-    double* inv = c->red_out.as<double>() + 64;
-    std::vector<double> hinv(c->nsub);
-    for (uint32_t s = 0; s < c->nsub; ++s) hinv[s] = c->sub_count[s] ? 1. / (double)c->sub_count[s] : 0.0;
-    SLLG_HIP(hipMemcpyAsync(inv, hinv.data(), c->nsub * sizeof(double), hipMemcpyHostToDevice, c->stream));
     if (c->prec == LLG_FP64_PLAIN)
         k_mag_partial<double><<<nb, kTPB, 0, c->stream>>>(c->n, c->nsub, c->S.as<double>(), sub, c->red_part.as<double>());
     else
         k_mag_partial<float><<<nb, kTPB, 0, c->stream>>>(c->n, c->nsub, c->S.as<float>(), sub, c->red_part.as<double>());
     SLLG_HIP(hipGetLastError());
-    k_sum_partials<<<1, kTPB, 0, c->stream>>>(nb, c->nsub * 3, c->red_part.as<double>(), inv, dev_out);
+    k_sum_partials<<<1, kTPB, 0, c->stream>>>(nb, c->nsub * 3, c->red_part.as<double>(), inverse_counts(c),
+                                              dev_out);
     SLLG_HIP(hipGetLastError());
+    return 0;
+}
+
+int reduce_result(llg_ctx* c, double** m, double** energy) {
+    SLLG_TRY(ensure_red(c));
+    *m = c->red_out.as<double>();
+    *energy = *m + kRedEnergy;
+    return 0;
+}
+
+// One table upload and two launches for all the members (each on stream s).  48 requests of
+// 10^3..48^3 spins with 650 member samples: 174 ms, and 188 ms with two launches and an upload
+// of the counts a member.
+int batch_reduce_mag(hipStream_t s, const std::vector<llg_ctx*>& members, double* dev_out, uint32_t stride,
+                     DevBuf& work) {
+    if (members.empty()) return 0;
+    std::vector<MagMember> tab(members.size());
+    size_t parts = 0;
+    uint32_t most = 1;
+    for (size_t k = 0; k < members.size(); ++k) {
+        llg_ctx* c = members[k];
+        SLLG_TRY(sync_spins(c));
+        MagMember& m = tab[k];
+        m = MagMember{};
+        m.n = c->n;
+        m.nsub = c->nsub;
+        m.nblocks = red_blocks(c->n);
+        m.S = c->S.as<float>();
+        m.sub = c->nsub > 1 ? c->sub.as<uint8_t>() : nullptr;
+        m.out = dev_out + k * (size_t)stride;
+        m.scale = inverse_counts(c);
+        parts += (size_t)m.nblocks * m.nsub * 3;
+        most = std::max(most, m.nblocks);
+    }
+    const size_t tb = tab.size() * sizeof(MagMember), need = tb + parts * sizeof(double);
+    if (work.bytes < need) SLLG_TRY(work.alloc(need + need / 2));
+    double* part = reinterpret_cast<double*>(work.as<char>() + tb);
+    for (auto& m : tab) {
+        m.part = part;
+        part += (size_t)m.nblocks * m.nsub * 3;
+    }
+    SLLG_HIP(hipMemcpyAsync(work.p, tab.data(), tb, hipMemcpyHostToDevice, s));
+    for (size_t k0 = 0; k0 < tab.size(); k0 += kGridRows) {  // grid.y holds at most 65535 members
+        const unsigned cnt = (unsigned)std::min<size_t>(kGridRows, tab.size() - k0);
+        k_mag_batch_partial<<<dim3(most, cnt), kTPB, 0, s>>>(work.as<MagMember>() + k0);
+        SLLG_HIP(hipGetLastError());
+        k_mag_batch_sum<<<cnt, kTPB, 0, s>>>(work.as<MagMember>() + k0);
+        SLLG_HIP(hipGetLastError());
+    }
     return 0;
 }
 
@@ -402,12 +504,11 @@ int reduce_mag(llg_ctx* c, double* dev_out) {
 // Device scratch of llg_reduce_mag_noalloc: one file-scope array per GPU (each GPU that runs
 // the library holds its own copy until the process ends).  Layout of one call:
 //   [0, nb nsub 3)          per-block partial sums (every slot written by its block)
-//   [kPartDoubles, + 16)    1 / (spins per sublattice)
-//   [kPartDoubles + 16, +48) the results, nsub x 3
+//   [kPartDoubles, +48)     the results, nsub x 3
 // Every call on one GPU uses the same array: calls that overlap on one GPU (two host
 // threads, or two streams without ordering between them) race.
 constexpr size_t kPartDoubles = (size_t)kRedBlocks * kMaxSub * 3;
-constexpr size_t kScratchDoubles = kPartDoubles + kMaxSub + kMaxSub * 3;  // 197,120 bytes
+constexpr size_t kScratchDoubles = kPartDoubles + kMaxSub * 3;  // 196,992 bytes
 static __device__ __align__(256) double scratch[kScratchDoubles];
 
 namespace {
@@ -440,19 +541,15 @@ int reduce_mag_noalloc(llg_ctx* c, double* m) {
     double* base = nullptr;
     SLLG_TRY(scratch_of(c->device, &base));
     double* part = base;
-    double* inv = base + kPartDoubles;
-    double* out = inv + kMaxSub;
+    double* out = base + kPartDoubles;
     SLLG_TRY(sync_spins(c));  // rebuilds S in place when only its AoS3 copy is current
-    double hinv[kMaxSub];
-    for (uint32_t s = 0; s < nsub; ++s) hinv[s] = c->sub_count[s] ? 1. / (double)c->sub_count[s] : 0.0;
-    SLLG_HIP(hipMemcpyAsync(inv, hinv, nsub * sizeof(double), hipMemcpyHostToDevice, c->stream));
     const uint8_t* sub = (nsub > 1) ? c->sub.as<uint8_t>() : nullptr;
     if (c->prec == LLG_FP64_PLAIN)
         k_mag_partial<double><<<nb, kTPB, 0, c->stream>>>(c->n, nsub, c->S.as<double>(), sub, part);
     else
         k_mag_partial<float><<<nb, kTPB, 0, c->stream>>>(c->n, nsub, c->S.as<float>(), sub, part);
     SLLG_HIP(hipGetLastError());
-    k_sum_partials<<<1, kTPB, 0, c->stream>>>(nb, nsub * 3, part, inv, out);
+    k_sum_partials<<<1, kTPB, 0, c->stream>>>(nb, nsub * 3, part, inverse_counts(c), out);
     SLLG_HIP(hipGetLastError());
     SLLG_HIP(hipMemcpyAsync(m, out, nsub * 3 * sizeof(double), hipMemcpyDeviceToHost, c->stream));
     SLLG_HIP(hipStreamSynchronize(c->stream));
@@ -472,9 +569,7 @@ int reduce_energy(llg_ctx* c, const void* dem_now, double* dev_out) {
     a.stg = c->stag_set ? c->STG.p : nullptr;
     a.spec = c->spec.as<uint8_t>();
     a.sp = c->sp64d.as<Species<double>>();
-    a.mu = c->red_out.as<double>() + 64 + kMaxSub;
-    SLLG_HIP(hipMemcpyAsync((void*)a.mu, c->mu_sp.data(), c->mu_sp.size() * sizeof(double), hipMemcpyHostToDevice,
-                            c->stream));
+    a.mu = c->red_out.as<double>() + kRedMu;
     a.an = c->an64;
     a.ex = c->ex64;
     double* part = c->red_part.as<double>();
@@ -505,7 +600,9 @@ int reduce_energy(llg_ctx* c, const void* dem_now, double* dev_out) {
 #undef SLLG_E_NC
 #undef SLLG_E
     SLLG_HIP(hipGetLastError());
-    k_sum_partials<<<1, kTPB, 0, c->stream>>>(nb, 1, part, nullptr, dev_out);
+    SubScale one{};
+    one.v[0] = 1.0;
+    k_sum_partials<<<1, kTPB, 0, c->stream>>>(nb, 1, part, one, dev_out);
     SLLG_HIP(hipGetLastError());
     return 0;
 }
@@ -667,6 +764,7 @@ int set_sq(llg_ctx* c, const uint32_t grid[3], const uint32_t* mesh, uint32_t nk
     SLLG_TRY(up(c->sq_proj, proj.data(), proj.size() * sizeof(uint2)));
     SLLG_TRY(up(c->sq_k, kp.data(), kp.size() * sizeof(uint2)));
     SLLG_TRY(c->sq_part.alloc(std::max<size_t>(1, (size_t)nch * proj.size()) * 2 * sizeof(double)));
+    SLLG_TRY(c->sq_out.alloc(std::max<size_t>(1, (size_t)ngroups * nk) * 2 * sizeof(double)));
     SLLG_HIP(hipStreamSynchronize(c->stream));
     c->sq_nk = nk;
     c->sq_np = (uint32_t)proj.size();

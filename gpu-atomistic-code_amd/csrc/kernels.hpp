@@ -68,6 +68,12 @@ int create_with_store(const llg_desc* d, const std::shared_ptr<ExchStore>& store
 
 // Reductions (k_reduce.hip): FP64 sublattice magnetisation and energy.
 int reduce_mag(llg_ctx* c, double* dev_out /* nsub*3 */);
+// <M> of FP32 members on one stream, member k's values at dev_out + k stride; work holds the
+// member table and partial sums and grows as needed.
+int batch_reduce_mag(hipStream_t s, const std::vector<llg_ctx*>& members, double* dev_out, uint32_t stride,
+                     DevBuf& work);
+// The handle's own result slots: <M> (nsub*3) and the energy, 48 doubles after it.
+int reduce_result(llg_ctx* c, double** m, double** energy);
 int reduce_energy(llg_ctx* c, const void* dem_now /* dipolar field at the current spins or null */,
                   double* dev_out /* 1 */);
 int noise_sample(llg_ctx* c, uint64_t t, double* dev_out);
