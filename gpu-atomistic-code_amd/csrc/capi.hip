@@ -89,6 +89,18 @@ __global__ __launch_bounds__(kTPB) void k_to_ref(uint32_t n, Perm perm, const T*
     if (i < n) ref[i] = (double)dev[perm.to_dev(i)];
 }
 
+// A new handle's state: spins along +z (predicted spins too), no staggered field.
+template <class T>
+__global__ __launch_bounds__(kTPB) void k_init_state(uint32_t n, T* __restrict__ S, T* __restrict__ Y,
+                                                     T* __restrict__ STG) {
+    const uint32_t i = blockIdx.x * kTPB + threadIdx.x;
+    if (i >= n) return;
+    for (size_t a = 0; a < 3; ++a) {
+        S[a * n + i] = Y[a * n + i] = a == 2 ? T(1) : T(0);
+        STG[a * n + i] = T(0);
+    }
+}
+
 // From this size on order and precision are converted on the device, one component at a time
 // (fcc 64^3: FP32 spins set in 1.9 ms and fetched in 1.9 instead of 3.3 and 2.5 with the host
 // loop, an FP64 field fetched in 2.0 instead of 8.8); below it three kernels and copies take
@@ -311,7 +323,7 @@ void llg_desc_init(llg_desc* d) {
     d->exch.ncomp = 1;
 }
 
-static int create_impl(const llg_desc* d, const std::shared_ptr<ExchStore>& share, llg_ctx** out) {
+static int create_impl(const llg_desc* d, const std::shared_ptr<ExchStore>& share, hipStream_t stream, llg_ctx** out) {
     if (!d || !out) SLLG_FAIL(LLG_E_INVALID, "descriptor or output pointer is NULL");
     *out = nullptr;
     if (share && (share->n != d->n || share->prec != d->precision || share->device != d->device))
@@ -348,7 +360,12 @@ static int create_impl(const llg_desc* d, const std::shared_ptr<ExchStore>& shar
         ~Guard() { if (c) llg_destroy(c); }
     } guard{c};
     c->device = d->device;
-    SLLG_HIP(hipStreamCreateWithFlags(&c->stream, hipStreamNonBlocking));
+    if (stream) {
+        c->stream = stream;
+        c->own_stream = false;
+    } else {
+        SLLG_HIP(hipStreamCreateWithFlags(&c->stream, hipStreamNonBlocking));
+    }
     c->n = d->n;
     c->ns = d->n_species;
     c->nsub = nsub;
@@ -498,24 +515,23 @@ static int create_impl(const llg_desc* d, const std::shared_ptr<ExchStore>& shar
         SLLG_HIP(hipMemset(c->DEM.p, 0, v3));
         SLLG_TRY(dipolar_create(c, d->dip, d->spin_species, fftx ? &d->fftx : nullptr, d->dip.enabled != 0));
     }
-    SLLG_HIP(hipMemset(c->STG.p, 0, v3));
-    // initial state: all spins along +z
-    {
-        std::vector<double> zx(n, 0.0), zz(n, 1.0);
-        SLLG_TRY(upload_state(c, c->S, zx.data(), zx.data(), zz.data()));
-        SLLG_TRY(upload_state(c, c->Y, zx.data(), zx.data(), zz.data()));
-    }
+    // initial state: all spins along +z, no staggered field
+    if (c->prec == LLG_FP64_PLAIN)
+        k_init_state<double><<<blocks_for(n, kTPB), kTPB, 0, c->stream>>>(n, c->S.as<double>(), c->Y.as<double>(), c->STG.as<double>());
+    else
+        k_init_state<float><<<blocks_for(n, kTPB), kTPB, 0, c->stream>>>(n, c->S.as<float>(), c->Y.as<float>(), c->STG.as<float>());
+    SLLG_HIP(hipGetLastError());
     SLLG_HIP(hipDeviceSynchronize());
     *out = c;
     c = nullptr;  // disarm guard
     return 0;
 }
 
-int llg_create(const llg_desc* d, llg_ctx** out) { return create_impl(d, nullptr, out); }
+int llg_create(const llg_desc* d, llg_ctx** out) { return create_impl(d, nullptr, nullptr, out); }
 
 int llg_create_like(const llg_desc* d, llg_ctx* proto, llg_ctx** out) {
     if (!proto || !proto->xs) SLLG_FAIL(LLG_E_INVALID, "NULL prototype");
-    return create_impl(d, proto->xs, out);
+    return create_impl(d, proto->xs, nullptr, out);
 }
 
 void llg_destroy(llg_ctx* c) {
@@ -873,8 +889,8 @@ int llg_get_info(llg_ctx* c, llg_info* info) {
 
 namespace sllg {
 // Internal: create a handle over an existing coupling store (batch.hip, serving).
-int create_with_store(const llg_desc* d, const std::shared_ptr<ExchStore>& store, llg_ctx** out) {
-    return create_impl(d, store, out);
+int create_with_store(const llg_desc* d, const std::shared_ptr<ExchStore>& store, hipStream_t stream, llg_ctx** out) {
+    return create_impl(d, store, stream, out);
 }
 }  // namespace sllg
 

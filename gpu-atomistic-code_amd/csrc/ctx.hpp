@@ -208,6 +208,10 @@ struct ExchStore {
     std::string encoding;
     uint32_t len_max = 0;  // longest row of the packed entries
     HostExch h;  // scalars kept; the large host vectors are released after upload
+    // host_only: encoded away from the device; the buffers' contents wait in `pending` until
+    // upload_store
+    bool host_only = false;
+    std::vector<std::pair<DevBuf*, std::vector<char>>> pending;
     uint64_t bytes() const {
         return a.bytes + b.bytes + c.bytes + d.bytes + e.bytes + f.bytes + g.bytes + dict64.bytes + fs_x.bytes +
                fs_q.bytes;

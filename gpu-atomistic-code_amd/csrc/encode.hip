@@ -35,6 +35,15 @@ int upload(DevBuf& b, const T* h, size_t count, hipStream_t s) {
     return 0;
 }
 
+// The same for a buffer of X, kept on the host while X is encoded away from the device.
+template <class T>
+int put(ExchStore& X, DevBuf& b, const T* h, size_t count, hipStream_t s) {
+    if (!X.host_only) return upload(b, h, count, s);
+    const char* p = reinterpret_cast<const char*>(h);
+    X.pending.emplace_back(&b, std::vector<char>(p, p + count * sizeof(T)));
+    return 0;
+}
+
 int validate_and_copy(llg_ctx* c, const llg_exchange& e) {
     ExchStore& X = *c->xs;
     HostExch& h = X.h;
@@ -508,10 +517,8 @@ void build_tiles(llg_ctx* c, const std::vector<uint2>& table,
         }
         if (!ok) continue;
         tw.insert(tw.end(), (size_t)TW, 0u);
-        if (upload(X.f, tw.data(), tw.size(), c->stream)) return;
-        if (upload(X.g, offs.data(), offs.size(), c->stream)) return;
-        x.tent = X.f.as<uint32_t>();
-        x.tgrp = X.g.as<uint32_t>();
+        if (put(X, X.f, tw.data(), tw.size(), c->stream)) return;
+        if (put(X, X.g, offs.data(), offs.size(), c->stream)) return;
         x.tnw = nw;
         x.tumax = umax;
         x.tlps = lps;
@@ -689,14 +696,12 @@ bool build_lines(llg_ctx* c, const std::vector<uint32_t>& ref_of, const std::vec
     }
     // worth it only when most slices are lines
     if (lined == 0 || 4u * nfall > nsl) return false;
-    if (upload(X.d, words.data(), words.size(), c->stream)) return false;
-    if (upload(X.e, table.data(), table.size(), c->stream)) return false;
+    if (put(X, X.d, words.data(), words.size(), c->stream)) return false;
+    if (put(X, X.e, table.data(), table.size(), c->stream)) return false;
     Exch<float>& x = X.ex32;
     x.tnw = x.tumax = x.tlps = 0;
     if (len == 64 && nfall == 0) build_tiles(c, table, kept);
     x.fmt = len == 64 ? (open ? FMT_SELL_LINE_OPEN : FMT_SELL_LINE) : (open ? FMT_SELL_LINE16_OPEN : FMT_SELL_LINE16);
-    x.lslice = X.e.as<uint2>();
-    x.lent = X.d.as<uint32_t>();
     x.lfall = nfall;
     lines_row = (uint32_t)(lines_total / lined);
     return true;
@@ -840,9 +845,9 @@ int build_sell(llg_ctx* c) {
                 d64[t * nc + a] = tuples[t].v[a];
                 d32[t * nc + a] = (float)tuples[t].v[a];
             }
-        SLLG_TRY(upload(X.b, ent.data(), ent.size(), c->stream));
-        SLLG_TRY(upload(X.c, d32.data(), d32.size(), c->stream));
-        SLLG_TRY(upload(X.dict64, d64.data(), d64.size(), c->stream));
+        SLLG_TRY(put(X, X.b, ent.data(), ent.size(), c->stream));
+        SLLG_TRY(put(X, X.c, d32.data(), d32.size(), c->stream));
+        SLLG_TRY(put(X, X.dict64, d64.data(), d64.size(), c->stream));
         x.fmt = FMT_SELL_PACK;
         x.ndict = (uint32_t)tuples.size();
         char buf[96];
@@ -872,26 +877,20 @@ int build_sell(llg_ctx* c) {
                 }
             }
         }
-        SLLG_TRY(upload(X.b, ent.data(), ent.size(), c->stream));
-        SLLG_TRY(upload(X.c, v32.data(), v32.size(), c->stream));
-        SLLG_TRY(upload(X.dict64, v64.data(), v64.size(), c->stream));
+        SLLG_TRY(put(X, X.b, ent.data(), ent.size(), c->stream));
+        SLLG_TRY(put(X, X.c, v32.data(), v32.size(), c->stream));
+        SLLG_TRY(put(X, X.dict64, v64.data(), v64.size(), c->stream));
         x.fmt = FMT_SELL_RAW;
         x.ndict = 0;
         X.encoding = P.na > 1 ? "sell64-u32-f32-sublattice-major" : "sell64-u32-f32";
     }
-    SLLG_TRY(upload(X.a, slice.data(), slice.size(), c->stream));
-    x.slice = X.a.as<uint2>();
-    x.ent = X.b.as<uint32_t>();
-    x.dict = X.c.as<float>();
+    SLLG_TRY(put(X, X.a, slice.data(), slice.size(), c->stream));
     x.nent = nent;
     x.ncell = ncell;
     x.dbits = pack ? dbits : 0;
     x64 = Exch<double>();
     fill_common(x64, h, n);
     x64.fmt = x.fmt;
-    x64.slice = x.slice;
-    x64.ent = x.ent;
-    x64.dict = X.dict64.as<double>();
     x64.ndict = x.ndict;
     x64.nent = nent;
     x64.ncell = ncell;
@@ -921,6 +920,63 @@ int build_sell(llg_ctx* c) {
 
 }  // namespace
 
+// Point both views of a sliced-ELL store at its device buffers.
+static void bind_sell(ExchStore& X) {
+    Exch<float>& x = X.ex32;
+    Exch<double>& x64 = X.ex64;
+    x.slice = x64.slice = X.a.as<uint2>();
+    x.ent = x64.ent = X.b.as<uint32_t>();
+    x.dict = X.c.as<float>();
+    x64.dict = X.dict64.as<double>();
+    x.lslice = X.e.as<uint2>();
+    x.lent = X.d.as<uint32_t>();
+    x.tent = X.f.as<uint32_t>();
+    x.tgrp = X.g.as<uint32_t>();
+}
+
+int encode_store(const llg_desc& d, std::shared_ptr<ExchStore>& out) {
+    if (d.precision != LLG_FP32 || d.exch.format != LLG_EXCH_CSR)
+        SLLG_FAIL(LLG_E_UNSUPPORTED, "couplings are encoded on the host for FP32 CSR only");
+    auto X = std::make_shared<ExchStore>();
+    X->device = d.device;
+    X->prec = d.precision;
+    X->n = d.n;
+    X->host_only = true;
+    llg_ctx c;  // what the encoder reads of a handle; no device state
+    c.n = d.n;
+    c.prec = d.precision;
+    c.flags = d.flags;
+    c.perm.na = 1;
+    c.perm.ncell = d.n;
+    X->perm = c.perm;
+    c.xs = X;
+    SLLG_TRY(build_exchange_fp32(&c, d.exch));
+    out = X;
+    return 0;
+}
+
+int upload_store(ExchStore& X, hipStream_t s) {
+    for (auto& p : X.pending) {
+        SLLG_TRY(p.first->alloc(p.second.size()));
+        if (!p.second.empty())
+            SLLG_HIP(hipMemcpyAsync(p.first->p, p.second.data(), p.second.size(), hipMemcpyHostToDevice, s));
+    }
+    SLLG_HIP(hipStreamSynchronize(s));
+    bind_sell(X);
+    return 0;
+}
+
+void keep_store(ExchStore& X) {
+    X.pending.clear();
+    X.pending.shrink_to_fit();
+    X.host_only = false;
+}
+
+void drop_store(ExchStore& X) {
+    for (auto& p : X.pending) p.first->release();
+    bind_sell(X);
+}
+
 int build_exchange_fp32(llg_ctx* c, const llg_exchange& e) {
     ExchStore& X = *c->xs;
     SLLG_TRY(validate_and_copy(c, e));
@@ -932,6 +988,7 @@ int build_exchange_fp32(llg_ctx* c, const llg_exchange& e) {
     if (h.fmt == LLG_EXCH_CSR) {
         X.perm = csr_order(c, e.n_atoms);
         SLLG_TRY(build_sell(c));
+        bind_sell(X);
     } else if (h.fmt == LLG_EXCH_DIA || h.fmt == LLG_EXCH_STENCIL) {
         std::vector<float> v32(h.vals.size());
         for (size_t q = 0; q < v32.size(); ++q) v32[q] = (float)h.vals[q];

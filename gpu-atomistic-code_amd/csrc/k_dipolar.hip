@@ -1052,13 +1052,6 @@ int dipolar_create(llg_ctx* c, const llg_dipolar& d, const uint32_t* spin_specie
     return 0;
 }
 
-int dipolar_set_stream(llg_ctx* c) {
-    if (!c->dplan) return 0;
-    if (c->dplan->have_fwd) SLLG_FFT(hipfftSetStream(c->dplan->fwd, c->stream));
-    if (c->dplan->have_inv) SLLG_FFT(hipfftSetStream(c->dplan->inv, c->stream));
-    return 0;
-}
-
 bool dipolar_is_exchange(const llg_ctx* c) { return c->dplan && c->dplan->general; }
 
 // The FP32 register-transform and half-grid plane paths run only this library's kernels (no

@@ -62,9 +62,16 @@ struct GridBar {
 int batch_heun_persistent(hipStream_t s, int fmt, int nc, const void* dmem, const void* dmap, uint32_t ntiles,
                           uint32_t step_off, uint32_t nsteps, uint32_t tpb, int xcd, bool g3, GridBar* bar,
                           uint32_t spin_limit, uint32_t* grid);
-int dipolar_set_stream(llg_ctx* c);
 // Handle over an existing coupling store (capi.hip).
-int create_with_store(const llg_desc* d, const std::shared_ptr<ExchStore>& store, llg_ctx** out);
+// (stream: the owner's stream to run on, or null for one of its own).
+int create_with_store(const llg_desc* d, const std::shared_ptr<ExchStore>& store, hipStream_t stream, llg_ctx** out);
+// Couplings of an FP32 CSR descriptor in two halves (encode.hip): validated and encoded on the
+// host by any thread, without device calls; then copied to the current device.  The host
+// contents stay until keep_store; drop_store takes the device buffers back.
+int encode_store(const llg_desc& d, std::shared_ptr<ExchStore>& out);
+int upload_store(ExchStore& x, hipStream_t s);
+void keep_store(ExchStore& x);
+void drop_store(ExchStore& x);
 
 // Reductions (k_reduce.hip): FP64 sublattice magnetisation and energy.
 int reduce_mag(llg_ctx* c, double* dev_out /* nsub*3 */);
