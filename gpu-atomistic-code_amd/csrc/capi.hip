@@ -482,6 +482,7 @@ static int create_impl(const llg_desc* d, const std::shared_ptr<ExchStore>& shar
     c->ex32 = c->xs->ex32;
     c->ex64 = c->xs->ex64;
     c->perm = c->xs->perm;
+    if (c->xs->blk_wgs) c->tune_line = 2;
     // per-spin species / sublattice bytes in the device order chosen by the encoder
     {
         std::vector<uint8_t> s8(n), u8(n);
@@ -1006,6 +1007,9 @@ extern "C" int llg_autotune(llg_ctx* c, uint32_t nsteps, llg_tune_result* out) {
         if (c->ex32.tnw) readers.push_back(2);
         readers.push_back(1);
         readers.push_back(0);
+    } else if (c->xs->blk_wgs && !(c->flags & LLG_FLAG_TUNE_FIXED_READER)) {  // line blocks, packed entries
+        readers.push_back(2);
+        readers.push_back(1);
     } else {
         readers.push_back(c->tune_line);
     }
@@ -1014,7 +1018,7 @@ extern "C" int llg_autotune(llg_ctx* c, uint32_t nsteps, llg_tune_result* out) {
     const int nthc = (c->T > 0.0 && c->noise_mode == LLG_NOISE_COUNTER) ? 2 : 1;
     // the AoS3 gather copy applies to the packed and line encodings
     const int ng3 = (c->ex32.fmt == FMT_SELL_PACK || lfmt) ? 2 : 1;
-    const int rd_default = lfmt ? 1 : c->tune_line;
+    const int rd_default = lfmt || readers.size() > 1 ? 1 : c->tune_line;
     double best = 1e300;
     TuneChoice b{256, 1, 2, c->tune_thc, c->tune_g3, c->tune_line};
     std::vector<std::pair<double, TuneChoice>> timed;  // every candidate's first timing
@@ -1027,20 +1031,21 @@ extern "C" int llg_autotune(llg_ctx* c, uint32_t nsteps, llg_tune_result* out) {
     int rc = 0;
     for (size_t li = 0; li < readers.size() && !rc; ++li) {
     const int rd = readers[li];
-    // the tile reader has one block size (its workgroup's slices) and stages from the AoS3
-    // copy; the gather depth applies to the packed reader only
-    const bool packed = lfmt ? rd == 0 : c->ex32.fmt == FMT_SELL_PACK;
-    for (int gi = 0; gi < (rd == 2 ? 1 : ng3) && !rc; ++gi)
+    // the LDS-staged readers have one block size (what their workgroups hold) and stage from the
+    // AoS3 copy; the gather depth applies to the packed reader only
+    const bool staged = rd == 2 && c->ex32.tnw;
+    const bool packed = lfmt ? rd == 0 : c->ex32.fmt == FMT_SELL_PACK && !staged;
+    for (int gi = 0; gi < (staged ? 1 : ng3) && !rc; ++gi)
     for (int hi = 0; hi < nthc && !rc; ++hi)
     for (int ui = 0; ui < (packed ? 2 : 1) && !rc; ++ui)
-        for (int ti = 0; ti < (rd == 2 ? 1 : 3) && !rc; ++ti)
+        for (int ti = 0; ti < (staged ? 1 : 3) && !rc; ++ti)
             for (int xcd = 1; xcd >= 0 && !rc; --xcd) {
-                const int tpb = rd == 2 ? (int)(64 * c->ex32.tnw) : tpbs[ti];
+                const int tpb = !staged ? tpbs[ti] : c->xs->blk_wgs ? 256 : (int)(64 * c->ex32.tnw);
                 c->tune_tpb = tpb;
                 c->tune_xcd = xcd;
                 c->tune_unr = unrs[ui];
                 if (nthc == 2) c->tune_thc = 1 - hi;
-                if (ng3 == 2) c->tune_g3 = rd == 2 ? 1 : 1 - gi;
+                if (ng3 == 2) c->tune_g3 = staged ? 1 : 1 - gi;
                 c->tune_line = rd;
                 rc = do_steps(c, 0, 2);
                 if (rc) break;

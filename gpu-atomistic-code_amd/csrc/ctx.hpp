@@ -49,6 +49,17 @@ constexpr int tile_head(int nw) { return (2 + 3 * nw + 7) / 8 * 8; }  // start o
 // bits of the first) and their couplings, tile_words(nc) words (12 for isotropic couplings).
 constexpr int tile_words(int nc) { return (line_group(nc) + 3 * line_group(nc) * nc + 3) / 4 * 4; }
 
+// Line-block reader (beside packed entries and 16-cell lines, k_block.hip): records of four entries, their LDS byte
+// offsets and couplings; the head of a workgroup's stream; sublattices it can hold.
+constexpr int block_words(int nc) { return 4 + 4 * nc; }
+constexpr uint32_t kBlockHead = 28;
+constexpr uint32_t kBlockSub = 8;
+constexpr uint32_t kBlockWaves = 16;         // waves of a workgroup at most
+// Shortest rows it is used for: with 8 entries (bct 50 x 51 x 52) 11.9 us a step against 13.6 with
+// packed entries, with 6 (simple cubic 60 x 61 x 62) 13.0 against 11.2.
+constexpr uint32_t kBlockMinLen = 8;
+constexpr uint32_t kBlockLdsMax = 64 * 1024;
+
 enum ExchFmt : int {
     FMT_NONE = 0,
     FMT_DIA = 1,
@@ -138,6 +149,9 @@ template <class V> struct Exch {
     uint32_t tnw = 0;                     // slices (waves) per workgroup
     uint32_t tumax = 0;                   // most lines any workgroup stages
     uint32_t tlps = 0;                    // slices per sublattice block
+    // line blocks (build_blocks, encodings without tile streams) use the same fields: tgrp the
+    // uint4 table of the workgroups, tent their streams, tnw waves per sublattice, tumax cells
+    // staged past each end of a line, tlps cells per line
     // four-spin quartets of each row (same row order as the spins of this path)
     const uint32_t* fs_xadj = nullptr;    // [n+1]; null = term off
     const uint4* fs_jkl = nullptr;        // (j, k, l, 0)
@@ -207,6 +221,7 @@ struct ExchStore {
     Perm perm;
     std::string encoding;
     uint32_t len_max = 0;  // longest row of the packed entries
+    uint32_t blk_wgs = 0, blk_waves = 0, blk_lds = 0;  // line blocks: workgroups (0: none), waves and LDS bytes of each
     HostExch h;  // scalars kept; the large host vectors are released after upload
     // host_only: encoded away from the device; the buffers' contents wait in `pending` until
     // upload_store
@@ -248,7 +263,7 @@ struct llg_ctx {
     int tune_unr = 2;    // packed-exchange chunks loaded ahead per wave (llg_autotune)
     int tune_thc = 1;    // predictor hands its thermal field to the corrector (llg_autotune)
     int tune_g3 = 1;     // gather neighbours from the AoS3 copy of the spins (llg_autotune)
-    int tune_line = 1;   // line encodings: 0 packed entries, 1 line reader, 2 tile reader (llg_autotune)
+    int tune_line = 1;   // line encodings: 0 packed entries, 1 line reader, 2 tile or line-block reader (llg_autotune)
     int tune_small = 1;  // one-workgroup steps for systems they cover (off after llg_set_launch)
     bool g3_valid = false;   // S3 holds the current S
     bool s_soa_valid = true;  // S (SoA) holds the current spins (else only S3 does: see sync_spins)

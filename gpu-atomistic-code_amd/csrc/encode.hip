@@ -15,6 +15,7 @@
 // their stored order, so the per-row summation order of the reference CSR
 // (src/cufields.cu:192-200) is kept.
 #include <algorithm>
+#include <cstdlib>
 #include <cstring>
 #include <map>
 #include <tuple>
@@ -699,11 +700,287 @@ bool build_lines(llg_ctx* c, const std::vector<uint32_t>& ref_of, const std::vec
     if (put(X, X.d, words.data(), words.size(), c->stream)) return false;
     if (put(X, X.e, table.data(), table.size(), c->stream)) return false;
     Exch<float>& x = X.ex32;
-    x.tnw = x.tumax = x.tlps = 0;
     if (len == 64 && nfall == 0) build_tiles(c, table, kept);
     x.fmt = len == 64 ? (open ? FMT_SELL_LINE_OPEN : FMT_SELL_LINE) : (open ? FMT_SELL_LINE16_OPEN : FMT_SELL_LINE16);
     x.lfall = nfall;
     lines_row = (uint32_t)(lines_total / lined);
+    return true;
+}
+
+// Line blocks of a packed encoding (read by k_block.hip).  When the rows of a sublattice that
+// share a lattice line (len cells, the fastest index) have the same entries, each to the same
+// neighbour line with the same shift along the (periodic) line and the same couplings, a
+// workgroup of m consecutive lines can stage whole neighbour lines in LDS, and entry q of every
+// one of its rows lies at one LDS distance from the row's own spin: the neighbour lines of
+// entry q, one per line of the workgroup, form a chain, and chains are staged as consecutive
+// lines (overlapping ones share lines: the chains of y - 1, y and y + 1 take m + 2).  Found
+// from the couplings alone: the shortest line length that fits.
+struct BlockEnt {
+    uint32_t t, line, id;  // neighbour's sublattice and line, coupling tuple
+    int32_t dz;
+    bool like(const BlockEnt& o) const { return t == o.t && id == o.id && dz == o.dz; }
+};
+constexpr int32_t kBlockShift = 4;  // largest shift along a line
+
+// Entries of line L of sublattice t; false when its rows differ.
+bool block_line(const HostExch& h, const Perm& P, const std::vector<uint32_t>& idx, uint32_t Z, uint32_t t, uint32_t L,
+                std::vector<BlockEnt>& out) {
+    out.clear();
+    const uint32_t r0 = P.to_ref(t * P.ncell + L * Z), q00 = h.xadj[r0], len = h.xadj[r0 + 1] - q00;
+    for (uint32_t q = 0; q < len; ++q) {
+        const uint32_t j = P.to_dev(h.adj[q00 + q]), tj = j / P.ncell, cj = j - tj * P.ncell, zj = cj % Z;
+        const int32_t dz = 2 * zj > Z ? (int32_t)zj - (int32_t)Z : (int32_t)zj;
+        if (std::abs(dz) > kBlockShift || 2 * std::abs(dz) >= (int32_t)Z) return false;
+        out.push_back(BlockEnt{tj, cj / Z, idx[q00 + q], dz});
+    }
+    for (uint32_t z = 1; z < Z; ++z) {  // reference rows of a line are na apart
+        const uint32_t r = r0 + z * P.na, q0 = h.xadj[r];
+        if (h.xadj[r + 1] - q0 != len) return false;
+        for (uint32_t q = 0; q < len; ++q) {
+            const BlockEnt& e = out[q];
+            int32_t w = (int32_t)z + e.dz;
+            w += w < 0 ? (int32_t)Z : 0;
+            w -= w >= (int32_t)Z ? (int32_t)Z : 0;
+            if (h.adj[q0 + q] != (e.line * Z + (uint32_t)w) * P.na + e.t || idx[q0 + q] != e.id) return false;
+        }
+    }
+    return true;
+}
+
+// Lines a workgroup stages: chains of g lines placed on tracks of consecutive lines.
+struct BlockLayout {
+    struct Track {
+        uint32_t t;
+        std::vector<uint32_t> lines;
+    };
+    std::vector<Track> tracks;
+    std::map<std::vector<uint32_t>, std::pair<uint32_t, uint32_t>> at;  // chain {t, lines} -> track, first line
+
+    uint32_t staged() const {
+        uint32_t k = 0;
+        for (const Track& tr : tracks) k += (uint32_t)tr.lines.size();
+        return k;
+    }
+    void build(const std::vector<std::vector<BlockEnt>>& lists, uint32_t na, uint32_t nl, uint32_t L0, uint32_t g) {
+        tracks.clear();
+        at.clear();
+        std::vector<uint32_t> key(g + 1);
+        for (uint32_t t = 0; t < na; ++t) {
+            key[0] = t;
+            for (uint32_t j = 0; j < g; ++j) key[j + 1] = L0 + j;
+            at.emplace(key, std::make_pair(0u, 0u));
+            const size_t len = lists[(size_t)t * nl + L0].size();
+            for (size_t q = 0; q < len; ++q) {
+                key[0] = lists[(size_t)t * nl + L0][q].t;
+                for (uint32_t j = 0; j < g; ++j) key[j + 1] = lists[(size_t)t * nl + L0 + j][q].line;
+                at.emplace(key, std::make_pair(0u, 0u));
+            }
+        }
+        std::vector<std::pair<uint32_t, int64_t>> pos;  // per chain: track, first line (relative to the track's base)
+        std::vector<int64_t> base;                      // of each track's first line
+        for (auto& c : at) {
+            const uint32_t* lines = c.first.data() + 1;
+            uint32_t best = 0, track = 0;
+            int64_t where = 0;
+            for (uint32_t k = 0; k < tracks.size(); ++k) {
+                if (tracks[k].t != c.first[0]) continue;
+                const std::vector<uint32_t>& tl = tracks[k].lines;
+                const int64_t n = (int64_t)tl.size();
+                for (int64_t o = 1 - (int64_t)g; o < n; ++o) {
+                    uint32_t same = 0;
+                    bool ok = true;
+                    for (int64_t j = std::max<int64_t>(0, -o); j < (int64_t)g && o + j < n && ok; ++j) {
+                        ok = tl[(size_t)(o + j)] == lines[j];
+                        ++same;
+                    }
+                    if (ok && same > best) {
+                        best = same;
+                        track = k;
+                        where = o;
+                    }
+                }
+            }
+            if (!best) {
+                track = (uint32_t)tracks.size();
+                tracks.push_back(Track{c.first[0], {}});
+                base.push_back(0);
+                where = 0;
+            }
+            std::vector<uint32_t>& tl = tracks[track].lines;
+            if (where < 0) {  // lines before the track's first
+                tl.insert(tl.begin(), lines, lines - where);
+                base[track] += where;
+                where = 0;
+            }
+            for (uint32_t j = (uint32_t)((int64_t)tl.size() - where); j < g; ++j) tl.push_back(lines[j]);
+            pos.emplace_back(track, where + base[track]);
+        }
+        std::vector<uint32_t> first(tracks.size(), 0);
+        for (size_t k = 1; k < tracks.size(); ++k) first[k] = first[k - 1] + (uint32_t)tracks[k - 1].lines.size();
+        size_t k = 0;
+        for (auto& c : at) {
+            c.second = std::make_pair(pos[k].first, first[pos[k].first] + (uint32_t)(pos[k].second - base[pos[k].first]));
+            ++k;
+        }
+    }
+};
+
+bool build_blocks(llg_ctx* c, const std::vector<uint32_t>& idx, const std::vector<TupleKey>& tuples) {
+    ExchStore& X = *c->xs;
+    const HostExch& h = X.h;
+    const Perm P = X.perm;
+    const uint32_t na = P.na, ncell = P.ncell, nc = (uint32_t)h.ncomp;
+    if (na > kBlockSub || X.len_max < kBlockMinLen || c->n <= kSmallSpins) return false;
+    const uint32_t zmax = kBlockWaves / na * 64u;  // a workgroup holds one line of every sublattice
+    std::vector<std::vector<BlockEnt>> lists;
+    uint32_t Z = 0, nl = 0;
+    std::vector<BlockEnt> e;
+    for (uint32_t z = 4; z <= zmax && z <= ncell && !Z; ++z) {
+        if (ncell % z) continue;
+        nl = ncell / z;
+        if (!block_line(h, P, idx, z, 0, 0, e) || !block_line(h, P, idx, z, 0, nl / 2, e)) continue;
+        lists.assign((size_t)na * nl, {});
+        bool ok = true;
+        for (uint32_t k = 0; k < na * nl && ok; ++k) ok = block_line(h, P, idx, z, k / nl, k % nl, lists[k]);
+        if (ok) Z = z;
+    }
+    if (!Z) return false;
+    uint32_t H = 0;
+    for (const auto& l : lists)
+        for (const BlockEnt& q : l) H = std::max(H, (uint32_t)std::abs(q.dz));
+    const uint32_t len = Z + 2 * H, line_bytes = len * 12u;
+    // lines g .. of a group starting at L0 that may follow it: entries alike, line by line
+    auto alike = [&](uint32_t L0, uint32_t L) {
+        for (uint32_t t = 0; t < na; ++t) {
+            const auto &a = lists[(size_t)t * nl + L0], &b = lists[(size_t)t * nl + L];
+            if (a.size() != b.size()) return false;
+            for (size_t q = 0; q < a.size(); ++q)
+                if (!a[q].like(b[q])) return false;
+        }
+        return true;
+    };
+    BlockLayout lay;
+    // groups of at most m lines: one more line is taken while it does not stage more than half
+    // as many lines as a line alone needs (a step over a lattice boundary does)
+    auto group_at = [&](uint32_t L0, uint32_t m) -> uint32_t {
+        uint32_t g = 1, prev = 0, one = 0;
+        lay.build(lists, na, nl, L0, 1);
+        prev = one = lay.staged();
+        while (g < m && L0 + g < nl && alike(L0, L0 + g)) {
+            lay.build(lists, na, nl, L0, g + 1);
+            const uint32_t s = lay.staged();
+            if (g == 1 ? s > 2 * one : (s - prev) * 2 > one) break;
+            if (s * line_bytes > kBlockLdsMax) break;
+            prev = s;
+            ++g;
+        }
+        if (g < m) lay.build(lists, na, nl, L0, g);
+        return g;
+    };
+    // Lines of a workgroup: the least estimated time of a cell, from the cycles of a wave (the row
+    // itself, its entries, its share of the staging loads), lanes without a row (they cost half:
+    // they take no bandwidth) and waves waiting at one barrier; at least three workgroups for
+    // two CUs.  us a step of fcc with 42 entries a row, by lines: 37 x 45 x 51 cells 19.8 (1), 22.4
+    // (2), 24.8 (5); 60 x 60 x 33 30.9 (1), 27.9 (3), 28.2 (5); 60 x 60 x 20 27.6 (1), 18.7 (3), 21.8
+    // (5); 80 x 80 x 12 40.1 (1), 18.8 (5); 20^3, too few lines, 10.4 (1), 11.2 (3).
+    uint32_t m = 1;
+    double best = 0.0;
+    for (uint32_t k = 1; k <= std::min(zmax / Z, 16u); ++k) {
+        if (k > 1 && nl / k < 384) break;
+        uint32_t nst = 0xFFFFFFFFu;
+        for (uint32_t s = 0; s < 4; ++s) {  // the fewest of four places: away from the boundaries
+            const uint32_t L0 = (uint32_t)((uint64_t)(nl - k) * s / 3);
+            bool same = true;
+            for (uint32_t j = 1; j < k && same; ++j) same = alike(L0, L0 + j);
+            if (!same) continue;
+            lay.build(lists, na, nl, L0, k);
+            nst = std::min(nst, lay.staged());
+        }
+        if (nst == 0xFFFFFFFFu || nst * line_bytes > kBlockLdsMax) continue;
+        const uint32_t wv = (k * Z + 63) / 64;
+        const double loads = (len <= 32 ? (double)nst / (64 / len) : (double)nst * ((len + 63) / 64)) / (wv * na);
+        const double lanes = wv * 64.0 / (k * Z);
+        const double cost = (300.0 + 8.0 * X.len_max + 20.0 * loads) * (0.5 + 0.5 * lanes) *
+                            (1.0 + 0.025 * std::max(0.0, (double)(wv * na) - 4.0));
+        if (best == 0.0 || cost < best) {
+            best = cost;
+            m = k;
+        }
+    }
+    if (best == 0.0) return false;
+    const uint32_t ws = (m * Z + 63) / 64;
+    std::vector<uint32_t> tw, table, st;
+    std::unordered_map<uint64_t, std::vector<std::pair<uint32_t, uint32_t>>> seen;  // record lists: first word, words
+    uint32_t umax = 0;
+    const uint32_t RW = (uint32_t)block_words((int)nc);
+    std::vector<uint32_t> key, recs;
+    for (uint32_t L0 = 0, g; L0 < nl; L0 += g) {
+        g = group_at(L0, m);
+        const uint32_t nst = lay.staged();
+        if (nst * line_bytes > kBlockLdsMax) return false;
+        umax = std::max(umax, nst);
+        const uint32_t base = (uint32_t)tw.size();
+        if ((uint64_t)base + kBlockHead + nst + 16 + (uint64_t)na * (X.len_max + 4) * RW >= (1ull << 31)) return false;
+        table.insert(table.end(), {base, L0, g, nst});
+        tw.resize(base + kBlockHead, 0u);
+        tw[base] = ((1u << 20) + Z - 1) / Z;
+        tw[base + 1] = ((1u << 20) + len - 1) / len;
+        tw[base + 2] = 64u / len;
+        for (const auto& tr : lay.tracks)
+            for (uint32_t L : tr.lines) tw.push_back(tr.t * ncell + L * Z);
+        while (tw.size() % 4) tw.push_back(0u);
+        key.assign(g + 1, 0u);
+        for (uint32_t t = 0; t < na; ++t) {
+            key[0] = t;
+            for (uint32_t j = 0; j < g; ++j) key[j + 1] = L0 + j;
+            const uint32_t own = lay.at.at(key).second;
+            tw[base + 4 + t] = own * line_bytes + H * 12u;
+            const auto& l0 = lists[(size_t)t * nl + L0];
+            const uint32_t nrec = ((uint32_t)l0.size() + 3) / 4;
+            recs.assign((size_t)nrec * RW, 0u);  // unused entries: the row itself, zero couplings
+            for (size_t q = 0; q < l0.size(); ++q) {
+                key[0] = l0[q].t;
+                for (uint32_t j = 0; j < g; ++j) key[j + 1] = lists[(size_t)t * nl + L0 + j][q].line;
+                uint32_t* rec = &recs[q / 4 * RW];
+                const int32_t off = ((int32_t)lay.at.at(key).second - (int32_t)own) * (int32_t)line_bytes + l0[q].dz * 12;
+                rec[q % 4] = (uint32_t)off;
+                for (uint32_t a = 0; a < nc; ++a) {
+                    const float v = (float)tuples[l0[q].id].v[a];
+                    std::memcpy(&rec[4 + q % 4 * nc + a], &v, 4);
+                }
+            }
+            uint64_t hsh = 1469598103934665603ull;
+            for (uint32_t v : recs) hsh = (hsh ^ v) * 1099511628211ull;
+            uint32_t where = 0;
+            bool found = false;
+            for (const auto& s : seen[hsh])
+                if (s.second == recs.size() && std::memcmp(&tw[s.first], recs.data(), recs.size() * 4) == 0) {
+                    where = s.first;
+                    found = true;
+                    break;
+                }
+            if (!found) {
+                where = (uint32_t)tw.size();
+                tw.insert(tw.end(), recs.begin(), recs.end());
+                seen[hsh].emplace_back(where, (uint32_t)recs.size());
+            }
+            tw[base + 12 + t] = where - base;  // modulo 2^32: lists of earlier workgroups lie before
+            tw[base + 20 + t] = nrec;
+        }
+    }
+    tw.insert(tw.end(), 2 * (size_t)RW, 0u);  // the reader fetches a record or two past a list
+    if (put(X, X.f, tw.data(), tw.size(), c->stream)) return false;
+    if (put(X, X.g, table.data(), table.size(), c->stream)) return false;
+    Exch<float>& x = X.ex32;
+    x.tnw = ws;
+    x.tumax = H;
+    x.tlps = Z;
+    X.blk_wgs = (uint32_t)(table.size() / 4);
+    X.blk_waves = ws * na;
+    X.blk_lds = umax * line_bytes;
+    char buf[64];
+    std::snprintf(buf, sizeof buf, "-blocks%ux%u", Z, m);
+    X.encoding += buf;
     return true;
 }
 
@@ -914,6 +1191,7 @@ int build_sell(llg_ctx* c) {
                     X.encoding = buf;
                     done = true;
                 }
+        if (!x.tnw) (void)build_blocks(c, idx, tuples);
     }
     return 0;
 }

@@ -358,8 +358,9 @@ typedef struct llg_tune_result {
     int unroll;
     int thermal_cache;  /* 1: the predictor hands its thermal field to the corrector */
     int gather_copy;    /* 1: neighbours are gathered from an AoS3 copy of the spins */
-    int line_mode;      /* line encodings: 1 line reader, 2 LDS-staged line reader (when the encoding has
-                           tile streams; else as 1), 0 the packed entries kept beside them */
+    int line_mode;      /* 2 LDS-staged reader, where the encoding has tile streams or line blocks (else as
+                           1); 1 the line reader of a line encoding, else the packed entries; 0 the
+                           packed entries.  A new handle has 2 with line blocks, else 1 */
 } llg_tune_result;
 int llg_autotune(llg_ctx* ctx, uint32_t nsteps, llg_tune_result* out);
 int llg_set_launch(llg_ctx* ctx, int tpb, int xcd, int unroll, int thermal_cache, int gather_copy, int line_mode);
