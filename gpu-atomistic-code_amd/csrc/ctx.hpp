@@ -1,9 +1,9 @@
 // ctx.hpp - device-side description of one spin system and the host handle.
 //
 // HBM layout (all SoA, component-major: component c of spin i at [c*n + i]):
-//   FP64 plain path : S, Y (predicted / stage input), H (exchange + demag), FN (f(S_n)),
-//                     DET, XI (noise), per-spin sigma/llgpf/lambda/k1u/k1udir, CSR with
-//                     FP64 values per nnz - the reference GPU data structures, SoA.
+//   FP64 plain path : S, Y (predicted / stage input), H (RK inputs, host I/O), FN (f(S_n)),
+//                     DET, XI (noise), per-spin sigma/llgpf/lambda/k1u/k1udir, CSR as
+//                     lane-uniform FP64 records or FP64 values per nnz.
 //   FP32 fused path : S, Y, A (= S + rdt/2 f(S)), per-species constants, a compact
 //                     exchange encoding (sliced ELL whose u32 entry packs the neighbour's
 //                     row offset with a coupling-dictionary index, repeated slices stored

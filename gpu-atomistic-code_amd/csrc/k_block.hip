@@ -11,11 +11,13 @@
 // Rows keep their entries' order, so the sums have the packed reader's bits.
 //
 // us a step (two half steps), packed entries and line blocks, 300 K: fcc, 42 entries, 37 x 45 x 51
-// cells 30.7 and 19.8, 59^3 53.4 and 34.4, 20^3 13.1 and 10.4; fcc, 12 entries, 37 x 45 x 51 18.9 and
+// cells 30.7 and 19.8, 59^3 53.4 and 33.0, 20^3 13.1 and 10.4; fcc, 12 entries, 37 x 45 x 51 18.9 and
 // 14.0; simple cubic, 56 entries, 60 x 61 x 62 25.2 and 19.4; bct, 8 entries, 50 x 51 x 52 13.6 and
 // 11.9.  What is left: the staging loads (every line is fetched by some nine workgroups), the LDS
 // reads (two instructions an entry) and the arithmetic follow each other in waves that start
 // together, 8 to 32 a CU.
+#include <type_traits>
+
 #include "fused.hpp"
 
 namespace sllg {
@@ -57,11 +59,15 @@ __device__ __forceinline__ BlockRow block_row(const FusedArgs& a) {
     return r;
 }
 
-// The staged lines, [line][cell -H .. Z + H) of 12 bytes, four loads in flight.  Lines of at most
-// 32 staged cells: as many to a wave load as fit its 64 lanes; longer ones: a load per line and
-// 64 cells with the line's first row in a scalar.  (One run of cells over all lines, full loads but
-// a row looked up by every lane, took 20.5 us a step where this takes 19.8, 37 x 45 x 51 fcc cells;
-// 26.5 instead of 27.9 for 60 x 60 x 33.)
+// The staged lines, [line][cell -H .. Z + H) of 12 bytes.  Lines of at most 32 staged cells: as
+// many to a wave load as fit its 64 lanes, four loads in flight; longer ones: a load per line and
+// 64 cells with the line's first row in a scalar, eight in flight where that adds no load past the
+// list (59^3 fcc cells, 8 lines a wave: 32.9 us a step, 34.7 with four; 40 x 40 x 80, 4 lines:
+// 35.1 with eight, 30.5 with four).  One run of cells over all lines (full loads, a row looked up
+// by every lane) took 20.5 us a step where this takes 19.5, 37 x 45 x 51 cells, and 26.5 where it
+// takes 27.9, 60 x 60 x 33; wrapped cells copied at the LDS store instead of loaded 22.2 for the first.
+// Loads past the list or a line's end repeat the last of it (the same value to the same place), so
+// that the waves stay out of divergent control flow.
 __device__ __forceinline__ void block_stage(const FusedArgs& a, const BlockRow& r, const float* __restrict__ src,
                                             char* lds) {
     const SpinBuf sb = spin_buf(src, a.n);
@@ -80,8 +86,6 @@ __device__ __forceinline__ void block_stage(const FusedArgs& a, const BlockRow& 
         d[2] = __uint_as_float(v[2]);
     };
     using V3 = decltype(__builtin_amdgcn_raw_buffer_load_b96(sb.r, 0, 0, 0));
-    // Loads past the list or a line's end repeat the last of it (the same value to the same place),
-    // so that the waves stay out of divergent control flow.
     const uint32_t last = r.nstaged - 1u;
     if (P <= 32u) {
         const uint32_t per = r.ts[2], sub = min((r.lane * r.ts[1]) >> 20, per - 1u), zz = min(r.lane - sub * P, P - 1u);
@@ -102,16 +106,23 @@ __device__ __forceinline__ void block_stage(const FusedArgs& a, const BlockRow& 
 #pragma unroll 1
     for (uint32_t z0 = 0; z0 < P; z0 += 64u) {
         const uint32_t zz = min(z0 + r.lane, P - 1u), vo = cell_of(zz) * 12u;
+        auto run = [&](auto depth) {
+            constexpr uint32_t D = decltype(depth)::value;
 #pragma unroll 1
-        for (uint32_t l0 = r.k; l0 <= last; l0 += 4u * nw) {
-            V3 v[4];
+            for (uint32_t l0 = r.k; l0 <= last; l0 += D * nw) {
+                V3 v[D];
 #pragma unroll
-            for (uint32_t u = 0; u < 4; ++u)
-                v[u] = __builtin_amdgcn_raw_buffer_load_b96(
-                    sb.r, vo, __builtin_amdgcn_readfirstlane(ls[min(l0 + u * nw, last)]) * 12u, 0);
+                for (uint32_t u = 0; u < D; ++u)
+                    v[u] = __builtin_amdgcn_raw_buffer_load_b96(
+                        sb.r, vo, __builtin_amdgcn_readfirstlane(ls[min(l0 + u * nw, last)]) * 12u, 0);
 #pragma unroll
-            for (uint32_t u = 0; u < 4; ++u) put(min(l0 + u * nw, last), zz, v[u]);
-        }
+                for (uint32_t u = 0; u < D; ++u) put(min(l0 + u * nw, last), zz, v[u]);
+            }
+        };
+        if ((last / nw / 4u) & 1u)  // an even number of fours
+            run(std::integral_constant<uint32_t, 8>());
+        else
+            run(std::integral_constant<uint32_t, 4>());
     }
 }
 
