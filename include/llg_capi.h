@@ -61,8 +61,8 @@ typedef enum llg_status {
 typedef enum llg_scheme { LLG_HEUN = 0, LLG_RK4 = 1, LLG_RK5 = 2 } llg_scheme;
 
 /* Arithmetic of the time step.
- * LLG_FP64_PLAIN: FP64 everywhere, reference structure (separate SpMV and integrator
- *   passes, per-nnz FP64 couplings, per-spin parameter arrays); the correctness path.
+ * LLG_FP64_PLAIN: FP64 everywhere, every sum in the reference's order (FP64 couplings,
+ *   per-spin parameter arrays, a kernel per field evaluation); the correctness path.
  * LLG_FP32: FP32 fused field assembly + integrator, |S|=1 renormalised each step,
  *   FP64 reductions and FP64 dipolar-kernel setup; the performance path. */
 typedef enum llg_precision { LLG_FP64_PLAIN = 0, LLG_FP32 = 1 } llg_precision;
@@ -290,7 +290,7 @@ int llg_get_field(llg_ctx* ctx, double* hx, double* hy, double* hz);
 int llg_reduce(llg_ctx* ctx, double* m, double* energy);
 
 /* llg_reduce(ctx, m, NULL) without any device allocation: the per-block partial sums and the
- * results go through a fixed device array of the library (197,120 bytes per GPU, held until the
+ * results go through a fixed device array of the library (196,992 bytes per GPU, held until the
  * process ends), so callers that cannot allocate (a tight serving loop, a harness that forbids
  * hipMalloc) can sample <M>.  No counterpart in the reference.  Same kernels and block count
  * as llg_reduce, so the same bits.  At most 16 sublattices (LLG_E_UNSUPPORTED beyond the
