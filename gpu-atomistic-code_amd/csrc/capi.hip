@@ -109,6 +109,13 @@ constexpr uint32_t kIoDevice = 65536;
 // Largest <M> series of llg_run_sampled whose device buffer the handle keeps (1365 samples of one
 // sublattice): an allocation and its release cost a short run some 30 us.
 constexpr size_t kSeriesKeep = 32768;
+// From this size on a new handle's Heun corrector draws its noise again instead of reading what
+// the predictor stored: the draw is 90 instructions a row, the hand-off 24 bytes of traffic, and
+// large systems wait for memory (us a step, handed over and drawn twice: simple cubic 30^3 9.1
+// and 10.0, 64^3 11.6 and 12.0, 72^3 13.2 and 13.1, 100^3 24.5 and 22.6; fcc 37 x 45 x 51 x 4 19.7
+// and 19.2, 64^3 x 4 31.5 and 30.6).  The same values either way.
+constexpr uint32_t kDrawTwice = 300000;
+int default_thermal_cache(const llg_ctx* c) { return c->n < kDrawTwice ? 1 : 0; }
 // n doubles of device memory that are free between steps: the FP32 path's A, the FP64 path's H
 // (both only carry values within a step).
 double* io_scratch(const llg_ctx* c) { return c->prec == LLG_FP64_PLAIN ? c->H.as<double>() : c->A.as<double>(); }
@@ -483,6 +490,7 @@ static int create_impl(const llg_desc* d, const std::shared_ptr<ExchStore>& shar
     c->ex64 = c->xs->ex64;
     c->perm = c->xs->perm;
     if (c->xs->blk_wgs) c->tune_line = 2;
+    c->tune_thc = default_thermal_cache(c);
     // per-spin species / sublattice bytes in the device order chosen by the encoder
     {
         std::vector<uint8_t> s8(n), u8(n);
@@ -1056,7 +1064,7 @@ extern "C" int llg_autotune(llg_ctx* c, uint32_t nsteps, llg_tune_result* out) {
                 float ms = 0.f;
                 (void)hipEventElapsedTime(&ms, e0, e1);
                 const double per = ms / nsteps;
-                if (tpb == 256 && xcd == 1 && unrs[ui] == 2 && hi == 0 && gi == 0 && rd == rd_default)
+                if (tpb == 256 && xcd == 1 && unrs[ui] == 2 && (nthc == 1 || c->tune_thc == default_thermal_cache(c)) && gi == 0 && rd == rd_default)
                     out->ms_per_step_default = per;
                 out->candidates++;
                 timed.push_back({per, TuneChoice{tpb, xcd, unrs[ui], c->tune_thc, c->tune_g3, c->tune_line}});
