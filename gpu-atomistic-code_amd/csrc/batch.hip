@@ -69,6 +69,7 @@ struct llg_batch {
     int persist = 0;     // chunks as persistent launches (grid barriers between half steps)
     int persist_graph = 1;  // with LLG_BATCH_GRAPH: capture them (0 once a capture was refused)
     bool gpersist = false;  // the captured graph holds persistent launches
+    bool gsmall = false;    // the captured graph holds one-workgroup steps
     uint32_t spin_limit = LLG_BATCH_SPIN_DEFAULT;  // polls per grid-barrier wait
     DevBuf bar;          // GridBar of the persistent launches
     uint32_t persist_grid = 0;  // blocks of the last persistent launch
@@ -108,7 +109,7 @@ void drop_graph(llg_batch* b) {
     b->graph = nullptr;
     b->gsteps = 0;
     b->gsig.clear();
-    b->gpersist = false;
+    b->gpersist = b->gsmall = false;
 }
 
 // Where the dipolar refreshes of the next chunk fall: they depend only on each dipolar
@@ -146,8 +147,9 @@ int regroup(llg_batch* b) {
     return 0;
 }
 
-// Member tables with the members' current step counters, temperatures and fields.
-int upload_tables(llg_batch* b) {
+// Member tables with the members' current step counters, temperatures and fields; g3: the
+// chunk's kernels gather from the AoS3 copies, which are brought up to date.
+int upload_tables(llg_batch* b, bool g3) {
     for (auto& g : b->groups) {
         std::vector<llg_ctx*> cs;
         std::vector<uint64_t> t0;
@@ -155,7 +157,7 @@ int upload_tables(llg_batch* b) {
             cs.push_back(b->m[k].c);
             t0.push_back(b->m[k].t);
         }
-        SLLG_TRY(batch_build_table(cs, t0, b->tpb, b->g3 != 0, g->dmem, g->dmap, g->ntiles, b->stream));
+        SLLG_TRY(batch_build_table(cs, t0, b->tpb, g3, g->dmem, g->dmap, g->ntiles, b->stream));
     }
     return 0;
 }
@@ -175,21 +177,22 @@ int launch_chunk_small(llg_batch* b, uint32_t nsteps) {
         std::vector<llg_ctx*> cs;
         for (int k : g->idx) cs.push_back(b->m[k].c);
         SLLG_TRY(batch_small_launch(b->stream, cs, g->dmem.p, nsteps));
-        for (llg_ctx* c : cs) {
-            c->g3_valid = false;
-            c->y_soa_valid = true;
-        }
     }
     return 0;
 }
 
-int launch_chunk(llg_batch* b, uint32_t nsteps, bool dipolar) {
-    if (small_chunk(b)) return launch_chunk_small(b, nsteps);
+// What a chunk's kernels leave current: S3 and Y3 with the gather copy, SoA Y without.  Set for
+// every chunk, since a replayed graph runs none of the code that captured it.
+void mark_current(llg_batch* b, bool g3) {
     for (auto& m : b->m)
-        if (m.c) {  // what the batch kernels leave current: S3 and Y3 with the gather copy, SoA Y without
-            m.c->g3_valid = b->g3 != 0;
-            m.c->y_soa_valid = !b->g3 || batch_needs_y_soa(m.c);
+        if (m.active()) {
+            m.c->g3_valid = g3;
+            m.c->y_soa_valid = !g3 || batch_needs_y_soa(m.c);
         }
+}
+
+int launch_chunk(llg_batch* b, uint32_t nsteps, bool dipolar, bool small) {
+    if (small) return launch_chunk_small(b, nsteps);
     for (uint32_t k = 0; k < nsteps; ++k) {
         if (dipolar)
             for (auto& mm : b->m)
@@ -227,11 +230,6 @@ int persist_prepare(llg_batch* b) {
 // predictor of its step, as in launch_chunk).  Batches with refreshes at the predicted spins
 // (every stage) take launch_chunk.
 int launch_chunk_persistent(llg_batch* b, uint32_t nsteps, bool dipolar) {
-    for (auto& m : b->m)
-        if (m.c) {
-            m.c->g3_valid = b->g3 != 0;
-            m.c->y_soa_valid = !b->g3 || batch_needs_y_soa(m.c);
-        }
     if (!b->bar.p) {
         SLLG_TRY(b->bar.alloc(sizeof(GridBar)));
         SLLG_HIP(hipMemsetAsync(b->bar.p, 0, sizeof(GridBar), b->stream));
@@ -467,7 +465,9 @@ int llg_batch_step(llg_batch* b, uint32_t nsteps) {
             dip_graph = dip_graph && dipolar_capturable(mm.c);
             dip_stage = dip_stage || mm.c->dip_every_stage;
         }
-    SLLG_TRY(upload_tables(b));
+    const bool small = small_chunk(b), g3 = b->g3 && !small;
+    SLLG_TRY(upload_tables(b, g3));
+    mark_current(b, g3);
     if (b->persist && !dip_stage) {
         bool replayed = false;
         if ((b->flags & LLG_BATCH_GRAPH) && dip_graph && b->persist_graph) {
@@ -515,10 +515,10 @@ int llg_batch_step(llg_batch* b, uint32_t nsteps) {
         }
     } else if ((b->flags & LLG_BATCH_GRAPH) && dip_graph) {
         std::vector<uint64_t> sig = refresh_signature(b);
-        if (!b->gexec || b->gpersist || b->gsteps != nsteps || sig != b->gsig) {
+        if (!b->gexec || b->gpersist || b->gsmall != small || b->gsteps != nsteps || sig != b->gsig) {
             drop_graph(b);
             SLLG_HIP(hipStreamBeginCapture(b->stream, hipStreamCaptureModeThreadLocal));
-            const int rc = launch_chunk(b, nsteps, dip);
+            const int rc = launch_chunk(b, nsteps, dip, small);
             hipGraph_t g = nullptr;
             const hipError_t e = hipStreamEndCapture(b->stream, &g);
             if (rc) {
@@ -530,11 +530,12 @@ int llg_batch_step(llg_batch* b, uint32_t nsteps) {
             SLLG_HIP(hipGraphInstantiate(&b->gexec, g, nullptr, nullptr, 0));
             b->gsteps = nsteps;
             b->gsig.swap(sig);
+            b->gsmall = small;
             b->graphs_built++;
         }
         SLLG_HIP(hipGraphLaunch(b->gexec, b->stream));
     } else {
-        SLLG_TRY(launch_chunk(b, nsteps, dip));
+        SLLG_TRY(launch_chunk(b, nsteps, dip, small));
     }
     for (auto& mm : b->m)
         if (mm.active()) mm.t += nsteps;
