@@ -285,8 +285,8 @@ int do_steps(llg_ctx* c, uint64_t t0, uint32_t nsteps) {
         c->y_soa_valid = true;
     }
     if (c->tune_small && small_applies(c, exec_fmt(c))) {
-        for (uint32_t k = 0; k < nsteps; k += kSmallSteps)
-            SLLG_TIMED("heun_steps", fused_heun_small(c, t0 + k, std::min(kSmallSteps, nsteps - k)));
+        for (uint64_t k = 0; k < nsteps; k += kSmallSteps)
+            SLLG_TIMED("heun_steps", fused_heun_small(c, t0 + k, std::min(kSmallSteps, nsteps - (uint32_t)k)));
         if (nsteps) c->det_valid = true;
         return 0;
     }

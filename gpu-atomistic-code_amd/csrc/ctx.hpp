@@ -29,8 +29,10 @@ constexpr int kDictLds = 2048;  // floats of coupling dictionary staged in LDS (
 // one whose rows are too long for registers (small_applies).
 constexpr uint32_t kSmallSpins = 2048;
 constexpr uint64_t kSmallEntries = 1024 * 42;
-// Steps of one such launch (some 20 ms at most).
-constexpr uint32_t kSmallSteps = 4096;
+// Steps of one such launch, for a handle and for a batch: some 14 ms at most (990 spins of 26 entries
+// with 9 components take 13.0 us a step), so other work on the GPU never waits long for it.  Cutting a
+// run here costs a launch, 0.2 % of the shortest steps (10^3 simple cubic, 2.2 us).
+constexpr uint32_t kSmallSteps = 1024;
 
 // Line-mode group records: line_group(nc) neighbour windows per record, line_words(nc) words
 // (the group's shift mask, its window starts, 3 shifts x nc couplings per window, the next

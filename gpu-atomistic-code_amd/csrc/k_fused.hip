@@ -970,11 +970,12 @@ __global__ __launch_bounds__(1024) void k_heun_small(FusedArgs a, float* S, floa
     small_run<NC, RPT, REG>(a, S, Y, a.t, nsteps);
 }
 
-// One block per member.
+// One block per member; steps step_off .. step_off + nsteps of the member's chunk.
 template <int NC, int RPT, bool REG>
-__global__ __launch_bounds__(1024) void k_heun_small_batch(const BatchMember* __restrict__ mem, uint32_t nsteps) {
+__global__ __launch_bounds__(1024) void k_heun_small_batch(const BatchMember* __restrict__ mem, uint32_t step_off,
+                                                           uint32_t nsteps) {
     const BatchMember& bm = mem[blockIdx.x];
-    small_run<NC, RPT, REG>(bm.a, bm.S, bm.Y, bm.t0, nsteps);
+    small_run<NC, RPT, REG>(bm.a, bm.S, bm.Y, bm.t0 + step_off, nsteps);
 }
 
 // RK4: stage m reads Yin (S for m = 0), k = rdt f(Yin);
@@ -1452,7 +1453,8 @@ int fused_heun_small(llg_ctx* c, uint64_t t0, uint32_t nsteps) {
     return 0;
 }
 
-// The same for the members of a batch group (its table built without gather copies).
+// The same for the members of a batch group (its table built without gather copies), in launches
+// of at most kSmallSteps.
 int batch_small_launch(hipStream_t s, const std::vector<llg_ctx*>& members, const void* dmem, uint32_t nsteps) {
     if (members.empty()) return 0;
     bool two = false, reg = true;
@@ -1461,10 +1463,13 @@ int batch_small_launch(hipStream_t s, const std::vector<llg_ctx*>& members, cons
         reg = reg && c->xs->len_max <= kSmallLen;
     }
     const BatchMember* m = static_cast<const BatchMember*>(dmem);
-#define SLLG_L(N, P, G) k_heun_small_batch<N, P, G><<<(unsigned)members.size(), 1024, 0, s>>>(m, nsteps)
-    SLLG_SMALL(small_nc(members[0]), two, reg, SLLG_L);
+    for (uint64_t k = 0; k < nsteps; k += kSmallSteps) {
+        const uint32_t off = (uint32_t)k, cnt = std::min(kSmallSteps, nsteps - off);
+#define SLLG_L(N, P, G) k_heun_small_batch<N, P, G><<<(unsigned)members.size(), 1024, 0, s>>>(m, off, cnt)
+        SLLG_SMALL(small_nc(members[0]), two, reg, SLLG_L);
 #undef SLLG_L
-    SLLG_HIP(hipGetLastError());
+        SLLG_HIP(hipGetLastError());
+    }
     return 0;
 }
 
