@@ -150,8 +150,18 @@ namespace {
 // entry; rows without an entry q (open boundaries) take the offset "none".  Every row meets its
 // own entries in CSR order, and the others load zeros, so the sums are the CSR's bit for bit.
 // Slices with equal records are stored once.  False (nothing kept) when the records would be
-// more than twice the entries of a row, as for couplings that differ from row to row, when the
-// offsets do not fit, or when the caller wants every slice stored.
+// more than twice the entries of a row, as for couplings that differ from row to row, when a
+// slice of a small system has more than kUniSlice times its entries, when the offsets do not
+// fit, or when the caller wants every slice stored.
+// The second bound: with few waves in flight a half step lasts as long as its longest slice, a
+// record about a third of a sliced-CSR entry.  us a step, records and sliced CSR, by the longest
+// slice's records an entry: bct 6^3 12.9 and 13.7 (3.75), fcc 10^3 37.2 and 33.5 (3.9), fcc 7^3 40.1
+// and 32.0 (4.1), fcc 100 x 9 x 5 37.8 and 32.2 (4.05), fcc 40 x 5 x 3 45.5 and 29.9 (5.3), bct 3^3 15.3
+// and 11.7 (6.75), a random chain of 64 with 4 neighbours 42.8 and 11.2 (64).  From 32,768 spins on
+// the waves share the SIMDs, and the sum of the records counts (fcc 30 x 30 x 20, longest 3.7, mean
+// 1.1: 43.7 and 65.4).
+constexpr uint32_t kUniSlice = 4;
+constexpr uint32_t kUniFew = 32768;
 bool build_uniform(llg_ctx* c, const HostExch& h, const Perm& P, std::vector<uint2>& table,
                    std::vector<uint32_t>& words, uint32_t& stored) {
     const uint32_t n = c->n, nc = (uint32_t)h.ncomp, nsl = (n + kSlice - 1) / kSlice, BW = uni_words((int)nc);
@@ -222,7 +232,7 @@ bool build_uniform(llg_ctx* c, const HostExch& h, const Perm& P, std::vector<uin
         }
         nrec += recs.size();
         nlen += most;
-        if (nrec > 2 * nlen + 256) return false;
+        if (nrec > 2 * nlen + 256 || (n < kUniFew && recs.size() > (size_t)kUniSlice * most)) return false;
         const uint32_t blocks = ((uint32_t)recs.size() + kUniBlock - 1) / kUniBlock;
         st.assign((size_t)blocks * BW, 0u);
         for (uint32_t r = 0; r < blocks * kUniBlock; ++r) {
