@@ -1201,7 +1201,8 @@ int build_sell(llg_ctx* c) {
                     X.encoding = buf;
                     done = true;
                 }
-        if (!x.tnw) (void)build_blocks(c, idx, tuples);
+        // read by a handle's own Heun steps only (RK and batches read lines or packed entries)
+        if (!x.tnw && c->scheme == LLG_HEUN && c->own_stream) (void)build_blocks(c, idx, tuples);
     }
     return 0;
 }
@@ -1230,7 +1231,8 @@ int encode_store(const llg_desc& d, std::shared_ptr<ExchStore>& out) {
     X->prec = d.precision;
     X->n = d.n;
     X->host_only = true;
-    llg_ctx c;  // what the encoder reads of a handle; no device state
+    llg_ctx c;  // what the encoder reads of a batch member; no device state
+    c.own_stream = false;
     c.n = d.n;
     c.prec = d.precision;
     c.flags = d.flags;
