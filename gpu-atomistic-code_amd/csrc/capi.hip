@@ -489,7 +489,7 @@ static int create_impl(const llg_desc* d, const std::shared_ptr<ExchStore>& shar
     c->ex32 = c->xs->ex32;
     c->ex64 = c->xs->ex64;
     c->perm = c->xs->perm;
-    if (c->xs->blk_wgs) c->tune_line = 2;
+    if (c->xs->blk_first) c->tune_line = 2;
     c->tune_thc = default_thermal_cache(c);
     // per-spin species / sublattice bytes in the device order chosen by the encoder
     {

@@ -224,6 +224,7 @@ struct ExchStore {
     std::string encoding;
     uint32_t len_max = 0;  // longest row of the packed entries
     uint32_t blk_wgs = 0, blk_waves = 0, blk_lds = 0;  // line blocks: workgroups (0: none), waves and LDS bytes of each
+    bool blk_first = false;  // a new handle reads them (blocks_pay)
     HostExch h;  // scalars kept; the large host vectors are released after upload
     // host_only: encoded away from the device; the buffers' contents wait in `pending` until
     // upload_store

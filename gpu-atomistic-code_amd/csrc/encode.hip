@@ -835,6 +835,44 @@ struct BlockLayout {
     }
 };
 
+// Whether a new handle reads line blocks (lines of Z cells) rather than what it has beside them.
+// The blocks stage every line of a workgroup and its neighbours, whole, so they gain with the
+// entries a row (read from LDS) and lose with the lines' length, which leaves fewer lines to a
+// workgroup and so more staged cells a row.  us a step at 300 K, untuned, blocks last.
+// Against packed entries:
+//   8 entries (bct): lines of 20 to 63 cells 0.85 to 1.03 of the packed time (64 x 65 x 63 cells 19.2
+//     and 18.5), but from 600,000 spins on and past 40 cells 1.01 to 1.13 (100 x 100 x 52 27.3 and 31.0);
+//     100 cells 1.02 to 1.24 (100^3 48.6 and 57.0), 200 cells 1.2 to 1.6
+//   12 (fcc) and 14 (bct): up to 63 cells 0.67 to 1.06; 80 to 127 cells 0.9 to 1.3 (fcc 64 x 65 x 80
+//     38.6 and 48.6); 200 cells 1.1 to 1.5
+//   18 (simple cubic): up to 52 cells 0.88 to 1.08, 63 cells 0.97 to 1.2, 80 and 100 cells 0.94 to 1.1
+//     and from 400,000 spins on 0.94 to 0.99, 127 cells 1.01 to 1.09
+//   26 and 32 (simple cubic): up to 127 cells 0.81 to 1.06; 200 cells 0.99 to 1.13
+//   42 (fcc): 0.64 to 0.92 at all lengths measured (7 to 127)
+// Against the line reader (encodings of 64- or 16-cell lines without tile streams), which also
+// loads a whole line at a time: one sublattice, 64 cells, 1.02 to 1.5 (18 and 26 entries, 8,000 to
+// 1,000,000 spins; 262,080 spins 12.9 and 15.8), 16 cells 0.93 to 0.97 at 65,536 spins and 1.05 to 1.09
+// at 262,144; bct, 14 entries, from 147,000 spins on 1.05 to 1.25, below 0.93 to 1.01, 8 entries 0.93
+// to 0.97 up to 508,000 spins and 1.09 at 991,000; fcc, 12 entries 0.75 to 0.95 throughout, 18 entries
+// up to 495,000 spins 0.83 to 0.98, 1,000,000 1.06, 42 entries up to 295,000 0.78 to 1.03, 495,000 and
+// more 1.07 to 1.18.
+bool blocks_pay(uint32_t n, uint32_t na, uint32_t Z, uint32_t entries, bool lines) {
+    if (lines) {
+        if (na == 1) return Z < 64 && n < 131072u;
+        if (na == 2) return n < (entries > 12 ? 131072u : 750000u);
+        return entries <= 12 || (uint64_t)n * entries < 17000000u;
+    }
+    if (entries >= 40) return true;
+    if (entries >= 24) return Z <= 128;
+    if (entries < 12 && Z > 40 && n >= 600000u) return false;
+    if (na == 1 && entries >= 16 && n >= 400000u) return Z <= 100;
+    return Z <= (na == 1 ? 56u : 64u);
+}
+
+// Up to this size blocks are built also where a new handle does not read them: a millisecond or
+// two of its creation, and the autotuner times them.
+constexpr uint32_t kBlockSmall = 16384;
+
 bool build_blocks(llg_ctx* c, const std::vector<uint32_t>& idx, const std::vector<TupleKey>& tuples) {
     ExchStore& X = *c->xs;
     const HostExch& h = X.h;
@@ -845,10 +883,12 @@ bool build_blocks(llg_ctx* c, const std::vector<uint32_t>& idx, const std::vecto
     std::vector<std::vector<BlockEnt>> lists;
     uint32_t Z = 0, nl = 0;
     std::vector<BlockEnt> e;
+    auto pays = [&](uint32_t z) { return blocks_pay(c->n, na, z, X.len_max, is_line_fmt(X.ex32.fmt)); };
     for (uint32_t z = 4; z <= zmax && z <= ncell && !Z; ++z) {
         if (ncell % z) continue;
         nl = ncell / z;
         if (!block_line(h, P, idx, z, 0, 0, e) || !block_line(h, P, idx, z, 0, nl / 2, e)) continue;
+        if (c->n > kBlockSmall && !pays(z)) continue;
         lists.assign((size_t)na * nl, {});
         bool ok = true;
         for (uint32_t k = 0; k < na * nl && ok; ++k) ok = block_line(h, P, idx, z, k / nl, k % nl, lists[k]);
@@ -988,6 +1028,7 @@ bool build_blocks(llg_ctx* c, const std::vector<uint32_t>& idx, const std::vecto
     X.blk_wgs = (uint32_t)(table.size() / 4);
     X.blk_waves = ws * na;
     X.blk_lds = umax * line_bytes;
+    X.blk_first = pays(Z);
     char buf[64];
     std::snprintf(buf, sizeof buf, "-blocks%ux%u", Z, m);
     X.encoding += buf;

@@ -1254,7 +1254,8 @@ static bool use_tile(const llg_ctx* c) {
     return c->tune_line == 2 && c->ex32.tnw && !c->xs->blk_wgs && (f == FMT_SELL_LINE || f == FMT_SELL_LINE_OPEN);
 }
 
-// The line-block reader likewise, on an encoding that has line blocks (a new handle's choice).
+// The line-block reader likewise, on an encoding that has line blocks (a new handle's choice where
+// blocks_pay, encode.hip).
 static bool use_block(const llg_ctx* c) { return c->tune_line == 2 && c->xs->blk_wgs; }
 
 // The AoS3 gather copy is used for the packed and line encodings when the tuner chose it.

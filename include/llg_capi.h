@@ -360,7 +360,7 @@ typedef struct llg_tune_result {
     int gather_copy;    /* 1: neighbours are gathered from an AoS3 copy of the spins */
     int line_mode;      /* 2 LDS-staged reader, where the encoding has tile streams or line blocks (else as
                            1); 1 the line reader of a line encoding, else the packed entries; 0 the
-                           packed entries.  A new handle has 2 with line blocks, else 1 */
+                           packed entries.  A new handle has 2 with line blocks where they measured faster, else 1 */
 } llg_tune_result;
 int llg_autotune(llg_ctx* ctx, uint32_t nsteps, llg_tune_result* out);
 int llg_set_launch(llg_ctx* ctx, int tpb, int xcd, int unroll, int thermal_cache, int gather_copy, int line_mode);
