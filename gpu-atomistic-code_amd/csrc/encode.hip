@@ -732,20 +732,35 @@ struct BlockEnt {
 };
 constexpr int32_t kBlockShift = 4;  // largest shift along a line
 
-// Entries of line L of sublattice t; false when its rows differ.
+// Entries of line L of sublattice t; false when its rows differ.  Away from the line's ends a
+// row's neighbours are the first row's, its distance further: whole rows are compared without a
+// branch.  at, id: scratch.
 bool block_line(const HostExch& h, const Perm& P, const std::vector<uint32_t>& idx, uint32_t Z, uint32_t t, uint32_t L,
-                std::vector<BlockEnt>& out) {
+                std::vector<BlockEnt>& out, std::vector<uint32_t>& at, std::vector<uint32_t>& id) {
     out.clear();
+    at.clear();
+    id.clear();
     const uint32_t r0 = P.to_ref(t * P.ncell + L * Z), q00 = h.xadj[r0], len = h.xadj[r0 + 1] - q00;
+    uint32_t reach = 0;  // largest shift along the line
     for (uint32_t q = 0; q < len; ++q) {
         const uint32_t j = P.to_dev(h.adj[q00 + q]), tj = j / P.ncell, cj = j - tj * P.ncell, zj = cj % Z;
         const int32_t dz = 2 * zj > Z ? (int32_t)zj - (int32_t)Z : (int32_t)zj;
         if (std::abs(dz) > kBlockShift || 2 * std::abs(dz) >= (int32_t)Z) return false;
+        reach = std::max(reach, (uint32_t)std::abs(dz));
         out.push_back(BlockEnt{tj, cj / Z, idx[q00 + q], dz});
+        at.push_back((uint32_t)((int32_t)(cj / Z * Z) + dz) * P.na + tj);  // modulo 2^32 where dz < 0
+        id.push_back(idx[q00 + q]);
     }
     for (uint32_t z = 1; z < Z; ++z) {  // reference rows of a line are na apart
         const uint32_t r = r0 + z * P.na, q0 = h.xadj[r];
         if (h.xadj[r + 1] - q0 != len) return false;
+        if (z >= reach && z + reach < Z) {  // nothing wraps
+            const uint32_t *pa = &h.adj[q0], *pi = &idx[q0];
+            uint32_t diff = 0;
+            for (uint32_t q = 0; q < len; ++q) diff |= (pa[q] - z * P.na - at[q]) | (pi[q] ^ id[q]);
+            if (diff) return false;
+            continue;
+        }
         for (uint32_t q = 0; q < len; ++q) {
             const BlockEnt& e = out[q];
             int32_t w = (int32_t)z + e.dz;
@@ -835,6 +850,28 @@ struct BlockLayout {
     }
 };
 
+// Groups of g lines whose entries lead, line by line, to the same lines relative to their own
+// first one (with the same couplings) have the same layout, moved along, and the same records:
+// both are built once a class of such groups.  Creating a handle, fcc 37 x 45 x 51 x 4 and 60 x 60 x
+// 20 x 4: 280 and 250 ms with a layout a group and rows compared entry by entry, 241 and 208 now, 230
+// and 189 without blocks.
+struct BlockClass {
+    uint32_t nst = 0;    // lines staged
+    uint32_t group = 0;  // of m lines: how many of them a group takes (group_at), once known
+    // of a class with stored records: staged lines {sublattice, line from the group's first}, per
+    // sublattice its own first line, first record word and records
+    std::vector<std::pair<uint32_t, uint32_t>> lines;
+    std::vector<uint32_t> own, where, nrec;
+};
+constexpr size_t kBlockClasses = 4096;  // remembered at a time
+struct BlockSigHash {
+    size_t operator()(const std::vector<uint32_t>& v) const {
+        uint64_t h = 1469598103934665603ull;
+        for (uint32_t w : v) h = (h ^ w) * 1099511628211ull;
+        return (size_t)h;
+    }
+};
+
 // Whether a new handle reads line blocks (lines of Z cells) rather than what it has beside them.
 // The blocks stage every line of a workgroup and its neighbours, whole, so they gain with the
 // entries a row (read from LDS) and lose with the lines' length, which leaves fewer lines to a
@@ -869,8 +906,8 @@ bool blocks_pay(uint32_t n, uint32_t na, uint32_t Z, uint32_t entries, bool line
     return Z <= (na == 1 ? 56u : 64u);
 }
 
-// Up to this size blocks are built also where a new handle does not read them: a millisecond or
-// two of its creation, and the autotuner times them.
+// Up to this size blocks are built also where a new handle does not read them: about a millisecond
+// of its creation, and the autotuner times them.
 constexpr uint32_t kBlockSmall = 16384;
 
 bool build_blocks(llg_ctx* c, const std::vector<uint32_t>& idx, const std::vector<TupleKey>& tuples) {
@@ -883,15 +920,16 @@ bool build_blocks(llg_ctx* c, const std::vector<uint32_t>& idx, const std::vecto
     std::vector<std::vector<BlockEnt>> lists;
     uint32_t Z = 0, nl = 0;
     std::vector<BlockEnt> e;
+    std::vector<uint32_t> at, id;
     auto pays = [&](uint32_t z) { return blocks_pay(c->n, na, z, X.len_max, is_line_fmt(X.ex32.fmt)); };
     for (uint32_t z = 4; z <= zmax && z <= ncell && !Z; ++z) {
         if (ncell % z) continue;
         nl = ncell / z;
-        if (!block_line(h, P, idx, z, 0, 0, e) || !block_line(h, P, idx, z, 0, nl / 2, e)) continue;
+        if (!block_line(h, P, idx, z, 0, 0, e, at, id) || !block_line(h, P, idx, z, 0, nl / 2, e, at, id)) continue;
         if (c->n > kBlockSmall && !pays(z)) continue;
         lists.assign((size_t)na * nl, {});
         bool ok = true;
-        for (uint32_t k = 0; k < na * nl && ok; ++k) ok = block_line(h, P, idx, z, k / nl, k % nl, lists[k]);
+        for (uint32_t k = 0; k < na * nl && ok; ++k) ok = block_line(h, P, idx, z, k / nl, k % nl, lists[k], at, id);
         if (ok) Z = z;
     }
     if (!Z) return false;
@@ -909,22 +947,44 @@ bool build_blocks(llg_ctx* c, const std::vector<uint32_t>& idx, const std::vecto
         }
         return true;
     };
+    std::unordered_map<std::vector<uint32_t>, BlockClass, BlockSigHash> classes;
+    std::vector<uint32_t> sig;
     BlockLayout lay;
+    auto class_of = [&](uint32_t L0, uint32_t g) -> BlockClass& {
+        sig.assign(1, g);
+        for (uint32_t t = 0; t < na; ++t) {
+            const size_t cnt = lists[(size_t)t * nl + L0].size();
+            sig.push_back((uint32_t)cnt);
+            for (size_t q = 0; q < cnt; ++q) {
+                const BlockEnt& a = lists[(size_t)t * nl + L0][q];
+                sig.insert(sig.end(), {a.t, a.id, (uint32_t)a.dz});
+                for (uint32_t j = 0; j < g; ++j) sig.push_back(lists[(size_t)t * nl + L0 + j][q].line - L0);
+            }
+        }
+        BlockClass& b = classes[sig];
+        if (b.nst == 0) {
+            lay.build(lists, na, nl, L0, g);
+            b.nst = lay.staged();
+        }
+        return b;
+    };
     // groups of at most m lines: one more line is taken while it does not stage more than half
     // as many lines as a line alone needs (a step over a lattice boundary does)
     auto group_at = [&](uint32_t L0, uint32_t m) -> uint32_t {
-        uint32_t g = 1, prev = 0, one = 0;
-        lay.build(lists, na, nl, L0, 1);
-        prev = one = lay.staged();
+        bool whole = L0 + m <= nl;
+        for (uint32_t j = 1; j < m && whole; ++j) whole = alike(L0, L0 + j);
+        uint32_t* const known = whole ? &class_of(L0, m).group : nullptr;
+        if (known && *known) return *known;
+        const uint32_t one = class_of(L0, 1).nst;
+        uint32_t g = 1, prev = one;
         while (g < m && L0 + g < nl && alike(L0, L0 + g)) {
-            lay.build(lists, na, nl, L0, g + 1);
-            const uint32_t s = lay.staged();
+            const uint32_t s = class_of(L0, g + 1).nst;
             if (g == 1 ? s > 2 * one : (s - prev) * 2 > one) break;
             if (s * line_bytes > kBlockLdsMax) break;
             prev = s;
             ++g;
         }
-        if (g < m) lay.build(lists, na, nl, L0, g);
+        if (known) *known = g;
         return g;
     };
     // Lines of a workgroup: the least estimated time of a cell, from the cycles of a wave (the row
@@ -943,8 +1003,7 @@ bool build_blocks(llg_ctx* c, const std::vector<uint32_t>& idx, const std::vecto
             bool same = true;
             for (uint32_t j = 1; j < k && same; ++j) same = alike(L0, L0 + j);
             if (!same) continue;
-            lay.build(lists, na, nl, L0, k);
-            nst = std::min(nst, lay.staged());
+            nst = std::min(nst, class_of(L0, k).nst);
         }
         if (nst == 0xFFFFFFFFu || nst * line_bytes > kBlockLdsMax) continue;
         const uint32_t wv = (k * Z + 63) / 64;
@@ -965,8 +1024,10 @@ bool build_blocks(llg_ctx* c, const std::vector<uint32_t>& idx, const std::vecto
     const uint32_t RW = (uint32_t)block_words((int)nc);
     std::vector<uint32_t> key, recs;
     for (uint32_t L0 = 0, g; L0 < nl; L0 += g) {
+        if (classes.size() > kBlockClasses) classes.clear();
         g = group_at(L0, m);
-        const uint32_t nst = lay.staged();
+        BlockClass& cl = class_of(L0, g);
+        const uint32_t nst = cl.nst;
         if (nst * line_bytes > kBlockLdsMax) return false;
         umax = std::max(umax, nst);
         const uint32_t base = (uint32_t)tw.size();
@@ -976,15 +1037,19 @@ bool build_blocks(llg_ctx* c, const std::vector<uint32_t>& idx, const std::vecto
         tw[base] = ((1u << 20) + Z - 1) / Z;
         tw[base + 1] = ((1u << 20) + len - 1) / len;
         tw[base + 2] = 64u / len;
-        for (const auto& tr : lay.tracks)
-            for (uint32_t L : tr.lines) tw.push_back(tr.t * ncell + L * Z);
+        const bool first = cl.own.empty();
+        if (first) {
+            lay.build(lists, na, nl, L0, g);
+            for (const auto& tr : lay.tracks)
+                for (uint32_t L : tr.lines) cl.lines.emplace_back(tr.t, L - L0);
+        }
+        for (const auto& q : cl.lines) tw.push_back(q.first * ncell + (L0 + q.second) * Z);
         while (tw.size() % 4) tw.push_back(0u);
         key.assign(g + 1, 0u);
-        for (uint32_t t = 0; t < na; ++t) {
+        for (uint32_t t = 0; first && t < na; ++t) {
             key[0] = t;
             for (uint32_t j = 0; j < g; ++j) key[j + 1] = L0 + j;
             const uint32_t own = lay.at.at(key).second;
-            tw[base + 4 + t] = own * line_bytes + H * 12u;
             const auto& l0 = lists[(size_t)t * nl + L0];
             const uint32_t nrec = ((uint32_t)l0.size() + 3) / 4;
             recs.assign((size_t)nrec * RW, 0u);  // unused entries: the row itself, zero couplings
@@ -1014,8 +1079,14 @@ bool build_blocks(llg_ctx* c, const std::vector<uint32_t>& idx, const std::vecto
                 tw.insert(tw.end(), recs.begin(), recs.end());
                 seen[hsh].emplace_back(where, (uint32_t)recs.size());
             }
-            tw[base + 12 + t] = where - base;  // modulo 2^32: lists of earlier workgroups lie before
-            tw[base + 20 + t] = nrec;
+            cl.own.push_back(own);
+            cl.where.push_back(where);
+            cl.nrec.push_back(nrec);
+        }
+        for (uint32_t t = 0; t < na; ++t) {
+            tw[base + 4 + t] = cl.own[t] * line_bytes + H * 12u;
+            tw[base + 12 + t] = cl.where[t] - base;  // modulo 2^32: lists of earlier workgroups lie before
+            tw[base + 20 + t] = cl.nrec[t];
         }
     }
     tw.insert(tw.end(), 2 * (size_t)RW, 0u);  // the reader fetches a record or two past a list
