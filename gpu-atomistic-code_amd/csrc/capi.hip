@@ -918,13 +918,19 @@ std::string tune_key(const llg_ctx* c) {
     char buf[256];
     // what changes the kernels that run: the thermal field (drawn only at T > 0 with counter
     // noise), the dipolar field operand, the four-spin term, a per-spin species index, and a
-    // reader pinned by the caller
+    // reader pinned by the caller, and line blocks (systems of one size may differ in them, and a
+    // choice made without them says nothing about their reader)
     const int thermal = c->T > 0.0 && c->noise_mode == LLG_NOISE_COUNTER;
     std::snprintf(buf, sizeof buf, "%s|%d|%d|%u|%llu|%u|T%d|D%d|F%d|M%d|R%d", p.gcnArchName, c->ex32.fmt,
                   c->ex32.ncomp, c->n, (unsigned long long)c->ex32.nent, c->perm.na, thermal, c->dip ? 1 : 0,
                   c->ex32.fs_xadj ? 1 : 0, c->multi_species ? 1 : 0,
                   (c->flags & LLG_FLAG_TUNE_FIXED_READER) ? 1 + c->tune_line : 0);
-    return buf;
+    std::string key = buf;
+    if (c->xs->blk_wgs) {
+        std::snprintf(buf, sizeof buf, "|B%u.%u.%u", c->ex32.tlps, c->xs->blk_waves, c->xs->blk_wgs);
+        key += buf;
+    }
+    return key;
 }
 
 void tune_file_load() {
@@ -932,9 +938,9 @@ void tune_file_load() {
     if (!f) return;
     FILE* fp = std::fopen(f, "r");
     if (!fp) return;
-    char key[256];
+    char key[320];
     TuneChoice t{};
-    while (std::fscanf(fp, "%255s %d %d %d %d %d %d", key, &t.tpb, &t.xcd, &t.unr, &t.thc, &t.g3, &t.line) == 7)
+    while (std::fscanf(fp, "%319s %d %d %d %d %d %d", key, &t.tpb, &t.xcd, &t.unr, &t.thc, &t.g3, &t.line) == 7)
         g_tune_cache[key] = t;
     std::fclose(fp);
 }
