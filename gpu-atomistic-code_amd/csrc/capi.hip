@@ -1032,7 +1032,8 @@ extern "C" int llg_autotune(llg_ctx* c, uint32_t nsteps, llg_tune_result* out) {
     const int nthc = (c->T > 0.0 && c->noise_mode == LLG_NOISE_COUNTER) ? 2 : 1;
     // the AoS3 gather copy applies to the packed and line encodings
     const int ng3 = (c->ex32.fmt == FMT_SELL_PACK || lfmt) ? 2 : 1;
-    const int rd_default = lfmt || readers.size() > 1 ? 1 : c->tune_line;
+    // the reader of a new handle (of this one, where the caller pinned it)
+    const int rd_default = readers.size() == 1 ? readers[0] : (c->xs->blk_first ? 2 : 1);
     double best = 1e300;
     TuneChoice b{256, 1, 2, c->tune_thc, c->tune_g3, c->tune_line};
     std::vector<std::pair<double, TuneChoice>> timed;  // every candidate's first timing
@@ -1114,6 +1115,25 @@ extern "C" int llg_autotune(llg_ctx* c, uint32_t nsteps, llg_tune_result* out) {
                 if (acc[k] < acc[kb]) kb = k;
             b = timed[kb].second;
             best = acc[kb] / 2.0;
+        }
+    }
+    // a system of one workgroup's size steps there whatever the shape: that is what both times say
+    if (!rc && noise == LLG_NOISE_COUNTER) {
+        const int fmt = c->ex32.fmt;
+        const bool small0 = small_applies(c, lfmt && !rd_default ? (int)FMT_SELL_PACK : fmt);
+        const bool small1 = small_applies(c, lfmt && !b.line ? (int)FMT_SELL_PACK : fmt);
+        if (small0 || small1) {
+            c->tune_small = 1;
+            c->tune_line = small1 ? b.line : rd_default;
+            rc = do_steps(c, 0, 2);
+            (void)hipEventRecord(e0, c->stream);
+            if (!rc) rc = do_steps(c, 2, 2 * nsteps);
+            (void)hipEventRecord(e1, c->stream);
+            (void)hipEventSynchronize(e1);
+            float ms = 0.f;
+            (void)hipEventElapsedTime(&ms, e0, e1);
+            if (small0) out->ms_per_step_default = ms / (2.0 * nsteps);
+            if (small1) best = ms / (2.0 * nsteps);
         }
     }
     c->noise_mode = noise;

@@ -352,8 +352,9 @@ int llg_profile_kernels(llg_ctx* ctx, uint64_t t0, uint32_t nsteps, int max_kind
  * across processes.  Other paths return LLG_OK with the defaults. */
 typedef struct llg_tune_result {
     int tpb, xcd;
-    double ms_per_step;     /* chosen */
-    double ms_per_step_default; /* 256 threads, remap on, 2 chunks ahead, hand-off on, gather copy on, line reader */
+    double ms_per_step;     /* chosen (one-workgroup steps where the system takes them) */
+    double ms_per_step_default; /* a new handle's: 256 threads, remap on, 2 chunks ahead, gather copy on, hand-off
+                                   and reader as a new handle has them, or one-workgroup steps */
     int candidates, from_cache;
     int unroll;
     int thermal_cache;  /* 1: the predictor hands its thermal field to the corrector */
