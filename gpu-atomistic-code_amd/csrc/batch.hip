@@ -691,6 +691,25 @@ int llg_batch_autotune(llg_batch* b, uint32_t nsteps, llg_batch_tune* out) {
             best = acc[kb] / 2.0;
         }
     }
+    // members of one workgroup's size step there whatever the shape: that is what the times say
+    if (!rc) {
+        rc = llg_batch_set_launch(b, btpb, bxcd, bline, bg3);
+        b->small = 1;
+        if (!rc && b->dirty) rc = regroup(b);
+        if (!rc && small_chunk(b)) {
+            rewind();
+            rc = llg_batch_step(b, 2);
+            if (!rc) rc = llg_batch_step(b, 2 * nsteps);
+            if (!rc && hipEventRecord(e0, b->stream) != hipSuccess) rc = LLG_E_DEVICE;
+            if (!rc) rc = llg_batch_step(b, 2 * nsteps);
+            if (!rc && hipEventRecord(e1, b->stream) != hipSuccess) rc = LLG_E_DEVICE;
+            if (!rc && hipEventSynchronize(e1) != hipSuccess) rc = LLG_E_DEVICE;
+            float ms = 0.f;
+            if (!rc && hipEventElapsedTime(&ms, e0, e1) != hipSuccess) rc = LLG_E_DEVICE;
+            best = (double)ms / (2.0 * nsteps);
+            if (bline || !any_line) out->ms_per_step_default = best;  // a new batch runs them too
+        }
+    }
     (void)hipEventDestroy(e0);
     (void)hipEventDestroy(e1);
     // restore the members' spins and step counters

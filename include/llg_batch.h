@@ -101,8 +101,8 @@ int llg_batch_set_persistent(llg_batch* b, int on, uint32_t spin_limit);
  * keeps the fastest, and restores every member's spins and step counter. */
 typedef struct llg_batch_tune {
     int tpb, xcd;
-    double ms_per_step;          /* chosen */
-    double ms_per_step_default;  /* 256 threads, XCD order, line reader */
+    double ms_per_step;          /* chosen (one-workgroup steps where every member takes them) */
+    double ms_per_step_default;  /* a new batch's: 256 threads, XCD order, line reader, or one-workgroup steps */
     int candidates;
     int line_mode;
     int gather_copy;
