@@ -166,9 +166,11 @@ int upload_tables(llg_batch* b, bool g3) {
 // per group and chunk instead of two a step.
 bool small_chunk(const llg_batch* b) {
     if (!b->small || b->persist || b->groups.empty()) return false;
+    size_t members = 0;
+    for (const auto& g : b->groups) members += g->idx.size();
     for (const auto& g : b->groups)
         for (int k : g->idx)
-            if (!small_applies(b->m[k].c, g->fmt)) return false;
+            if (!small_applies(b->m[k].c, g->fmt, members)) return false;
     return true;
 }
 

@@ -29,9 +29,12 @@ constexpr int kDictLds = 2048;  // floats of coupling dictionary staged in LDS (
 // one whose rows are too long for registers (small_applies).
 constexpr uint32_t kSmallSpins = 2048;
 constexpr uint64_t kSmallEntries = 1024 * 42;
-// Steps of one such launch, for a handle and for a batch: some 14 ms at most (990 spins of 26 entries
-// with 9 components take 13.0 us a step), so other work on the GPU never waits long for it.  Cutting a
-// run here costs a launch, 0.2 % of the shortest steps (10^3 simple cubic, 2.2 us).
+constexpr uint64_t kSmallCouplings = 200000;  // entries times components
+constexpr size_t kSmallMembers = 96;          // members of a batch from which the latter bound is left out
+// Steps of one such launch, for a handle and for a batch, so that other work on the GPU does not wait
+// long for it: some 12 ms at most for a handle (400 fcc spins of 9 components 11 us a step), as long as
+// the members' steps take for a batch (256 members of 1,008 such spins 24 ms, 1,024 members 92).
+// Cutting a run here costs a launch, 0.2 % of the shortest steps (10^3 simple cubic, 2.2 us).
 constexpr uint32_t kSmallSteps = 1024;
 
 // Line-mode group records: line_group(nc) neighbour windows per record, line_words(nc) words

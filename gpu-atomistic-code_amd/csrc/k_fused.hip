@@ -1421,22 +1421,28 @@ int fused_heun_corr(llg_ctx* c, const StepSched& s) {
         }                                                                                \
     } while (0)
 
+static int small_nc(const llg_ctx* c) { return c->ex32.fmt == FMT_NONE ? 1 : c->ex32.ncomp; }
+
 // What the one-workgroup steps cover, for a reader of format fmt: no dipolar refresh (other
 // kernels in the step), no four-spin term, counter noise.
 // One CU computes what the launches spread over the GPU, so the work is bounded: rows whose
 // entries stay in registers up to kSmallSpins (two a thread; simple cubic, 300 K: 10^3 spins
 // 2.2 us a step against 9.2 with two launches, 12^3 4.4 against 9.3), longer ones up to one row
 // a thread and kSmallEntries in all (fcc, 42 entries: 840 spins 9.3 us against 12.4, but 2,048
-// spins 16.8 against 13.2).
-bool small_applies(const llg_ctx* c, int fmt) {
+// spins 16.8 against 13.2).  Entries of 9 components cost that CU nine times the couplings: up to
+// kSmallCouplings in all (500 fcc spins of 42 entries 11.1 us against 13.8, 990 simple cubic spins of
+// 26 13.0 against 12.4, 1,008 of 42 20.0 against 14.7), unless a batch of `members` fills the GPU
+// anyway (256 members of 1,008 fcc spins: 23.9 us against 38.1; 16: 20.6 against 14.9).
+bool small_applies(const llg_ctx* c, int fmt, size_t members) {
     if (c->prec != LLG_FP32 || c->scheme != LLG_HEUN || c->dip || c->ex32.fs_xadj ||
         c->noise_mode != LLG_NOISE_COUNTER || (fmt != FMT_SELL_PACK && fmt != FMT_NONE))
         return false;
     const uint32_t len = c->xs->len_max;
-    return len <= kSmallLen ? c->n <= kSmallSpins : c->n <= 1024u && (uint64_t)c->n * len <= kSmallEntries;
+    if (len <= kSmallLen) return c->n <= kSmallSpins;
+    const uint64_t entries = (uint64_t)c->n * len;
+    return c->n <= 1024u && entries <= kSmallEntries &&
+           (members >= kSmallMembers || entries * (uint64_t)small_nc(c) <= kSmallCouplings);
 }
-
-static int small_nc(const llg_ctx* c) { return c->ex32.fmt == FMT_NONE ? 1 : c->ex32.ncomp; }
 
 // nsteps Heun steps from step t0; the spins are left in S, the last predictor output in Y.
 int fused_heun_small(llg_ctx* c, uint64_t t0, uint32_t nsteps) {

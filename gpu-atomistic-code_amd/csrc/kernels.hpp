@@ -20,7 +20,8 @@ struct StepSched {
 };
 int fused_heun_pred(llg_ctx* c, const StepSched& s);
 int fused_heun_corr(llg_ctx* c, const StepSched& s);
-bool small_applies(const llg_ctx* c, int fmt);  // one-workgroup steps cover the handle (reader of format fmt)
+// one-workgroup steps cover the handle (reader of format fmt), alone or as one of a batch's members
+bool small_applies(const llg_ctx* c, int fmt, size_t members = 1);
 int fused_heun_small(llg_ctx* c, uint64_t t0, uint32_t nsteps);
 int batch_small_launch(hipStream_t s, const std::vector<llg_ctx*>& members, const void* dmem, uint32_t nsteps);
 int fused_y_soa(llg_ctx* c);  // rebuild the SoA predictor output from its AoS3 copy
