@@ -295,7 +295,8 @@ struct llg_ctx {
     sllg::DevBuf bin_idx, bin_w, bin_cs, bin_cb, bin_part;
     uint32_t nbins = 0, nbin_chunks = 0;
     // transverse structure factor (llg_set_sq): per listed spin its device row, mesh coordinates
-    // along the projected axes and weights (ua, ub); chunk tables; projections, wave-vectors
+    // along the projected axes and weights (ua, ub); chunk tables; projections, wave-vectors.  The
+    // direct sum (no projections: sq_np 0) has {row, mesh coordinates} in sq_row
     sllg::DevBuf sq_row, sq_uv, sq_w, sq_cs, sq_cx, sq_cg, sq_proj, sq_k, sq_part, sq_out;
     uint32_t sq_nk = 0, sq_np = 0, sq_ngroups = 0, sq_nch = 0;
     uint32_t sq_grid[3] = {0, 0, 0};  // mesh extents: plane axis, projected axes

@@ -296,6 +296,8 @@ __global__ __launch_bounds__(kTPB) void k_bin_finish(uint32_t nbins, const uint3
 // block each (4 spins a thread, kept in registers over the projections); partial sums are
 // combined in a fixed order.  Phases: (k x mod N) / N exactly in FP64 (products below 2^53),
 // then sincospi.
+// Wave-vector lists with many projections, or spins in many groups (few to a plane), are summed
+// directly instead (k_sq_direct) where that is estimated faster (set_sq).
 // Bound by latency (262,144 spins read 1 MB of rows and 2 MB of spins).  64^3 spins, 33
 // wave-vectors (q, 0, 0), trace durations: 90 + 125 us for the two passes with one sincospi per
 // (spin, k) and one thread per k in the second; 5.1 + 3.8 us here.
@@ -382,6 +384,75 @@ __global__ __launch_bounds__(kTPB) void k_sq_partial(SqArgs a, const SpinT* __re
         }
         __syncthreads();
     }
+}
+
+// The direct sum: the spins of each group in chunks of kSqDirect, staged in LDS; each thread takes
+// one wave-vector over a chunk.  Phases as above, the residue of k x by a reciprocal: k x and q N are
+// exact, and a quotient off by one only moves the phase by a whole turn.
+constexpr uint32_t kSqDirect = 512;
+
+struct SqDirect {
+    uint32_t n, nk, axis;
+    double N[3], inv[3];   // mesh extents, 1 / N
+    const uint4* spin;     // {device row, x, y, z} per listed spin
+    const double2* w;      // (ua, ub) or null
+    const uint32_t* cs;    // chunk starts [nch + 1]
+    const uint32_t* cg;    // first chunk of each group [ngroups + 1]
+    const uint32_t* kp;    // [nk][3]
+};
+
+// k x modulo N, in [-N, 2 N)
+__device__ __forceinline__ double sq_residue(double k, double x, double N, double inv) {
+    const double t = k * x;
+    return fma(-floor(t * inv), N, t);
+}
+
+template <class SpinT>
+__global__ __launch_bounds__(kTPB) void k_sq_direct(SqDirect a, const SpinT* __restrict__ S, double2* __restrict__ part) {
+    __shared__ double sre[kSqDirect], sim[kSqDirect], px[kSqDirect], py[kSqDirect], pz[kSqDirect];
+    const uint32_t ch = blockIdx.x, b = a.cs[ch], e = a.cs[ch + 1];
+    const uint32_t ca = a.axis == 0 ? 1u : 0u, cb = a.axis == 2 ? 1u : 2u;
+    for (uint32_t q = b + threadIdx.x; q < e; q += kTPB) {
+        const uint4 sp = a.spin[q];
+        const double2 w = a.w ? a.w[q] : make_double2(1.0, 1.0);
+        const uint32_t l = q - b;
+        sre[l] = (double)S[(size_t)ca * a.n + sp.x] * w.x;
+        sim[l] = (double)S[(size_t)cb * a.n + sp.x] * w.y;
+        px[l] = (double)sp.y;
+        py[l] = (double)sp.z;
+        pz[l] = (double)sp.w;
+    }
+    __syncthreads();
+    for (uint32_t k = blockIdx.y * kTPB + threadIdx.x; k < a.nk; k += gridDim.y * kTPB) {
+        const double kx = a.kp[3 * (size_t)k], ky = a.kp[3 * (size_t)k + 1], kz = a.kp[3 * (size_t)k + 2];
+        double re = 0.0, im = 0.0;
+#pragma unroll 2
+        for (uint32_t l = 0; l < e - b; ++l) {
+            double t = sq_residue(kx, px[l], a.N[0], a.inv[0]) * a.inv[0];
+            t = fma(sq_residue(ky, py[l], a.N[1], a.inv[1]), a.inv[1], t);
+            t = fma(sq_residue(kz, pz[l], a.N[2], a.inv[2]), a.inv[2], t);
+            double sn, cn;
+            sincospi(2.0 * (t - floor(t)), &sn, &cn);
+            re = fma(sre[l], cn, fma(sim[l], sn, re));
+            im = fma(sim[l], cn, fma(-sre[l], sn, im));
+        }
+        part[(size_t)ch * a.nk + k] = make_double2(re, im);
+    }
+}
+
+__global__ __launch_bounds__(kTPB) void k_sq_direct_finish(SqDirect a, uint32_t ngroups, const double2* __restrict__ part,
+                                                           double* __restrict__ out) {
+    const uint32_t v = blockIdx.x * kTPB + threadIdx.x;
+    if (v >= ngroups * a.nk) return;
+    const uint32_t g = v / a.nk, k = v % a.nk;
+    double2 s = make_double2(0.0, 0.0);
+    for (uint32_t ch = a.cg[g]; ch < a.cg[g + 1]; ++ch) {
+        const double2 c = part[(size_t)ch * a.nk + k];
+        s.x += c.x;
+        s.y += c.y;
+    }
+    out[(size_t)v * 2] = s.x;
+    out[(size_t)v * 2 + 1] = s.y;
 }
 
 // One wave per (group, wave-vector): its lanes take the group's chunks in a stride.
@@ -721,15 +792,103 @@ int set_sq(llg_ctx* c, const uint32_t grid[3], const uint32_t* mesh, uint32_t nk
             proj.swap(pr);
         }
     }
-    // listed spins by (group, plane), ascending device row within a plane
-    std::vector<std::pair<uint64_t, uint32_t>> list;
-    list.reserve(n);
-    for (uint32_t r = 0; r < n; ++r) {
-        const uint32_t i = c->perm.to_ref(r), g = group ? group[i] : 0u;
-        if (g < ngroups) list.emplace_back(((uint64_t)g << 32) | mesh[3 * (size_t)i + ax[d][0]], r);
+    // Spins of each group, and of each of its planes: counted where there are not many more
+    // (group, plane) pairs than spins, else from a sorted list.
+    const uint64_t D = grid[ax[d][0]], pairs = (uint64_t)ngroups * D;
+    const bool counted = pairs <= 4ull * n + 1024;
+    std::vector<std::pair<uint64_t, uint32_t>> list;  // (group, plane), device row
+    std::vector<uint32_t> at(counted ? pairs + 1 : 0, 0), first(ngroups + 1, 0);
+    auto each = [&](auto&& take) {
+        for (uint32_t r = 0; r < n; ++r) {
+            const uint32_t i = c->perm.to_ref(r), g = group ? group[i] : 0u;
+            if (g < ngroups) take(g, mesh[3 * (size_t)i + ax[d][0]], r, i);
+        }
+    };
+    uint64_t planes = 0;  // chunks of planes
+    if (counted) {
+        each([&](uint32_t g, uint32_t x, uint32_t, uint32_t) { ++at[g * D + x + 1]; });
+        for (uint64_t k = 0; k < pairs; ++k) {
+            planes += (at[k + 1] + kSqChunk - 1) / kSqChunk;
+            first[k / D + 1] += at[k + 1];
+            at[k + 1] += at[k];
+        }
+    } else {
+        list.reserve(n);
+        each([&](uint32_t g, uint32_t x, uint32_t r, uint32_t) { list.emplace_back(((uint64_t)g << 32) | x, r); });
+        std::sort(list.begin(), list.end());
+        for (size_t q = 0, from = 0; q < list.size(); ++q) {
+            ++first[(list[q].first >> 32) + 1];
+            if (q + 1 < list.size() && list[q + 1].first == list[q].first) continue;
+            planes += (q + 1 - from + kSqChunk - 1) / kSqChunk;
+            from = q + 1;
+        }
     }
-    if (!std::is_sorted(list.begin(), list.end())) std::sort(list.begin(), list.end());
+    uint32_t longest = 0;  // spins of the longest direct chunk
+    for (uint32_t g = 0; g < ngroups; ++g) {
+        longest = std::max(longest, std::min(kSqDirect, first[g + 1]));
+        first[g + 1] += first[g];
+    }
+    const uint32_t listed = first[ngroups];
     const bool weighted = ua || ub;
+    auto up = [&](DevBuf& b, const void* h, size_t bytes) -> int {
+        SLLG_TRY(b.alloc(std::max<size_t>(bytes, 8)));
+        if (bytes) SLLG_HIP(hipMemcpyAsync(b.p, h, bytes, hipMemcpyHostToDevice, c->stream));
+        return 0;
+    };
+    // Two passes or the direct sum, by an estimate of their times in us: a chunk of a plane and a
+    // projection take 4.0 ns with the chip full (0.5 without a phase), whatever the spins in the
+    // chunk, and a block 1.5 us for each of its projections; a spin and 256 wave-vectors take 0.65 ns
+    // with the chip full, and a direct chunk of 512 spins 100 us.  us a sample, two passes and direct:
+    // 64^3 spins, 1,000 wave-vectors 974 and 691; 500 in 16 groups 1,990 and 429; 48^3, 300 in 300
+    // groups 15,575 and 386; 14 x 5 x 4, 1,202 in 2 groups 75 and 58; 32^3, 50 wave-vectors 72 and 126; a
+    // line of 33 of 64^3 29 and 215.
+    double phases = 0.0;
+    for (const uint2& p : proj) phases += (p.x | p.y) ? 4.0e-3 : 0.5e-3;
+    const double tile = 1.5 / 4.0e-3 * std::min(phases, kSqTile * 4.0e-3);
+    const double two_pass = std::max((double)planes * phases, tile);
+    const double direct = std::max(100.0 / kSqDirect * (double)longest, 0.65e-3 * (double)listed * ((nk + 255) / 256));
+    if (direct < two_pass) {
+        std::vector<uint4> sp(std::max<uint32_t>(1, listed));
+        std::vector<double2> w(weighted ? sp.size() : 0);
+        std::vector<uint32_t> fill(first.begin(), first.end() - 1), cs(1, 0), cg(ngroups + 1, 0);
+        each([&](uint32_t g, uint32_t, uint32_t r, uint32_t i) {
+            const uint32_t q = fill[g]++;
+            sp[q] = make_uint4(r, mesh[3 * (size_t)i], mesh[3 * (size_t)i + 1], mesh[3 * (size_t)i + 2]);
+            if (weighted) w[q] = make_double2(ua ? ua[i] : 1.0, ub ? ub[i] : 1.0);
+        });
+        for (uint32_t g = 0; g < ngroups; ++g) {
+            cg[g] = (uint32_t)cs.size() - 1;
+            for (uint32_t q = first[g]; q < first[g + 1]; q += std::min(kSqDirect, first[g + 1] - q))
+                cs.push_back(q + std::min(kSqDirect, first[g + 1] - q));
+        }
+        const uint32_t dchunks = cg[ngroups] = (uint32_t)cs.size() - 1;
+        SLLG_TRY(up(c->sq_row, sp.data(), sp.size() * sizeof(uint4)));
+        c->sq_uv.release();
+        c->sq_cx.release();
+        c->sq_proj.release();
+        if (weighted)
+            SLLG_TRY(up(c->sq_w, w.data(), w.size() * sizeof(double2)));
+        else
+            c->sq_w.release();
+        SLLG_TRY(up(c->sq_cs, cs.data(), cs.size() * 4));
+        SLLG_TRY(up(c->sq_cg, cg.data(), cg.size() * 4));
+        SLLG_TRY(up(c->sq_k, kpts, (size_t)nk * 3 * 4));
+        SLLG_TRY(c->sq_part.alloc(std::max<size_t>(1, (size_t)dchunks * nk) * 2 * sizeof(double)));
+        SLLG_TRY(c->sq_out.alloc(std::max<size_t>(1, (size_t)ngroups * nk) * 2 * sizeof(double)));
+        SLLG_HIP(hipStreamSynchronize(c->stream));
+        c->sq_nk = nk;
+        c->sq_np = 0;
+        c->sq_ngroups = ngroups;
+        c->sq_nch = dchunks;
+        c->sq_axis = axis;
+        for (int a = 0; a < 3; ++a) c->sq_grid[a] = grid[a];
+        return 0;
+    }
+    // listed spins by (group, plane), ascending device row within a plane
+    if (counted) {
+        list.resize(listed);
+        each([&](uint32_t g, uint32_t x, uint32_t r, uint32_t) { list[at[g * D + x]++] = {((uint64_t)g << 32) | x, r}; });
+    }
     std::vector<uint32_t> row(std::max<size_t>(1, list.size()));
     std::vector<uint2> uv(row.size());
     std::vector<double2> w(weighted ? row.size() : 0);
@@ -747,11 +906,6 @@ int set_sq(llg_ctx* c, const uint32_t grid[3], const uint32_t* mesh, uint32_t nk
     }
     for (uint32_t g = 0; g < ngroups; ++g) cg[g + 1] = std::max(cg[g + 1], cg[g]);  // groups without spins
     const uint32_t nch = (uint32_t)cx.size();
-    auto up = [&](DevBuf& b, const void* h, size_t bytes) -> int {
-        SLLG_TRY(b.alloc(std::max<size_t>(bytes, 8)));
-        if (bytes) SLLG_HIP(hipMemcpyAsync(b.p, h, bytes, hipMemcpyHostToDevice, c->stream));
-        return 0;
-    };
     SLLG_TRY(up(c->sq_row, row.data(), row.size() * 4));
     SLLG_TRY(up(c->sq_uv, uv.data(), uv.size() * sizeof(uint2)));
     if (weighted)
@@ -778,6 +932,34 @@ int set_sq(llg_ctx* c, const uint32_t grid[3], const uint32_t* mesh, uint32_t nk
 int sample_sq(llg_ctx* c, double* dev_out) {
     SLLG_TRY(sync_spins(c));
     if (c->sq_nk == 0 || c->sq_ngroups == 0) return 0;
+    if (c->sq_np == 0) {  // the direct sum
+        SqDirect a{};
+        a.n = c->n;
+        a.nk = c->sq_nk;
+        a.axis = (uint32_t)c->sq_axis;
+        for (int k = 0; k < 3; ++k) {
+            a.N[k] = (double)c->sq_grid[k];
+            a.inv[k] = 1.0 / a.N[k];
+        }
+        a.spin = c->sq_row.as<uint4>();
+        a.w = c->sq_w.as<double2>();
+        a.cs = c->sq_cs.as<uint32_t>();
+        a.cg = c->sq_cg.as<uint32_t>();
+        a.kp = c->sq_k.as<uint32_t>();
+        double2* const part = c->sq_part.as<double2>();
+        if (c->sq_nch) {
+            const dim3 grid(c->sq_nch, std::min(blocks_for(a.nk, kTPB), 65535u));
+            if (c->prec == LLG_FP64_PLAIN)
+                k_sq_direct<double><<<grid, kTPB, 0, c->stream>>>(a, c->S.as<double>(), part);
+            else
+                k_sq_direct<float><<<grid, kTPB, 0, c->stream>>>(a, c->S.as<float>(), part);
+            SLLG_HIP(hipGetLastError());
+        }
+        k_sq_direct_finish<<<blocks_for((size_t)c->sq_ngroups * c->sq_nk, kTPB), kTPB, 0, c->stream>>>(
+            a, c->sq_ngroups, part, dev_out);
+        SLLG_HIP(hipGetLastError());
+        return 0;
+    }
     SqArgs a{};
     a.n = c->n;
     a.nk = c->sq_nk;
