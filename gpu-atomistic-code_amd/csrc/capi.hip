@@ -74,19 +74,21 @@ struct Scope {
 
 size_t prec_bytes(const llg_ctx* c) { return c->prec == LLG_FP64_PLAIN ? sizeof(double) : sizeof(float); }
 
-// One component between the reference spin order in FP64 (host side) and the device order in
-// the path's precision.
+// Components (one a block row) between the reference spin order in FP64 (host side) and the device
+// order in the path's precision.
 template <class T>
 __global__ __launch_bounds__(kTPB) void k_from_ref(uint32_t n, Perm perm, const double* __restrict__ ref,
                                                    T* __restrict__ dev) {
     const uint32_t i = blockIdx.x * kTPB + threadIdx.x;
-    if (i < n) dev[perm.to_dev(i)] = (T)ref[i];
+    const size_t o = (size_t)blockIdx.y * n;
+    if (i < n) dev[o + perm.to_dev(i)] = (T)ref[o + i];
 }
 template <class T>
 __global__ __launch_bounds__(kTPB) void k_to_ref(uint32_t n, Perm perm, const T* __restrict__ dev,
                                                  double* __restrict__ ref) {
     const uint32_t i = blockIdx.x * kTPB + threadIdx.x;
-    if (i < n) ref[i] = (double)dev[perm.to_dev(i)];
+    const size_t o = (size_t)blockIdx.y * n;
+    if (i < n) ref[o + i] = (double)dev[o + perm.to_dev(i)];
 }
 
 // A new handle's state: spins along +z (predicted spins too), no staggered field.
@@ -106,6 +108,10 @@ __global__ __launch_bounds__(kTPB) void k_init_state(uint32_t n, T* __restrict__
 // loop, an FP64 field fetched in 2.0 instead of 8.8); below it three kernels and copies take
 // longer than the loop (10^3 spins: 58 us against 28).
 constexpr uint32_t kIoDevice = 65536;
+// The same for FP64 handles in another order than the caller's, all components in one launch (us, host
+// loop and device, set and get: 16,384 spins 70, 54 and 66, 60; 23,328 84, 71 and 78, 67; 62,500 211, 225
+// and 144, 113).
+constexpr uint32_t kIoDevice64 = 20000;
 // Largest <M> series of llg_run_sampled whose device buffer the handle keeps (1365 samples of one
 // sublattice): an allocation and its release cost a short run some 30 us.
 constexpr size_t kSeriesKeep = 32768;
@@ -116,9 +122,25 @@ constexpr size_t kSeriesKeep = 32768;
 // and 19.2, 64^3 x 4 31.5 and 30.6).  The same values either way.
 constexpr uint32_t kDrawTwice = 300000;
 int default_thermal_cache(const llg_ctx* c) { return c->n < kDrawTwice ? 1 : 0; }
-// n doubles of device memory that are free between steps: the FP32 path's A, the FP64 path's H
-// (both only carry values within a step).
+// Device memory that is free between steps: the FP32 path's A (n doubles, one component), the
+// FP64 path's H (3 n, all three; both only carry values within a step).
 double* io_scratch(const llg_ctx* c) { return c->prec == LLG_FP64_PLAIN ? c->H.as<double>() : c->A.as<double>(); }
+bool io_on_device(const llg_ctx* c) { return c->n >= (c->prec == LLG_FP64_PLAIN ? kIoDevice64 : kIoDevice); }
+
+// Host components in the reference order to the device (SoA, device order, precision T) through
+// the scratch memory: as many components at a time as it holds.  Enqueued, not waited for.
+template <class T>
+int from_ref(llg_ctx* c, const double* const src[3], T* dst) {
+    const uint32_t n = c->n, per = c->prec == LLG_FP64_PLAIN ? 3 : 1;
+    double* const tmp = io_scratch(c);
+    for (uint32_t a = 0; a < 3; a += per) {
+        for (uint32_t k = 0; k < per; ++k)
+            SLLG_HIP(hipMemcpyAsync(tmp + (size_t)k * n, src[a + k], (size_t)n * 8, hipMemcpyHostToDevice, c->stream));
+        k_from_ref<T><<<dim3(blocks_for(n, kTPB), per), kTPB, 0, c->stream>>>(n, c->perm, tmp, dst + (size_t)a * n);
+        SLLG_HIP(hipGetLastError());
+    }
+    return 0;
+}
 
 // Upload a host SoA double[3n] (reference spin order) into a state buffer of the path's
 // precision, in the device order.
@@ -131,7 +153,7 @@ int upload_state(llg_ctx* c, DevBuf& dst, const double* x, const double* y, cons
     }
     if (&dst == &c->Y) c->y_soa_valid = true;
     const bool f64 = c->prec == LLG_FP64_PLAIN, direct = f64 && !c->permuted();
-    if (!direct && n < kIoDevice) {
+    if (!direct && !io_on_device(c)) {
         std::vector<double> t64(f64 ? 3 * (size_t)n : 0);
         std::vector<float> t32(f64 ? 0 : 3 * (size_t)n);
         for (uint32_t i = 0; i < n; ++i) {
@@ -146,17 +168,13 @@ int upload_state(llg_ctx* c, DevBuf& dst, const double* x, const double* y, cons
         SLLG_HIP(hipStreamSynchronize(c->stream));
         return 0;
     }
-    double* const tmp = io_scratch(c);
-    for (int a = 0; a < 3; ++a) {
-        double* const to = direct ? dst.as<double>() + (size_t)a * n : tmp;
-        SLLG_HIP(hipMemcpyAsync(to, src[a], (size_t)n * 8, hipMemcpyHostToDevice, c->stream));
-        if (direct) continue;
-        if (f64)
-            k_from_ref<double><<<blocks_for(n, kTPB), kTPB, 0, c->stream>>>(n, c->perm, tmp, dst.as<double>() + (size_t)a * n);
-        else
-            k_from_ref<float><<<blocks_for(n, kTPB), kTPB, 0, c->stream>>>(n, c->perm, tmp, dst.as<float>() + (size_t)a * n);
-        SLLG_HIP(hipGetLastError());
-    }
+    if (direct)
+        for (int a = 0; a < 3; ++a)
+            SLLG_HIP(hipMemcpyAsync(dst.as<double>() + (size_t)a * n, src[a], (size_t)n * 8, hipMemcpyHostToDevice, c->stream));
+    else if (f64)
+        SLLG_TRY(from_ref<double>(c, src, dst.as<double>()));
+    else
+        SLLG_TRY(from_ref<float>(c, src, dst.as<float>()));
     SLLG_HIP(hipStreamSynchronize(c->stream));
     return 0;
 }
@@ -167,7 +185,7 @@ int download_state(llg_ctx* c, const void* src_dev, bool src_f64, double* x, dou
     const uint32_t n = c->n;
     double* dst[3] = {x, y, z};
     const bool direct = src_f64 && !c->permuted();
-    if (!direct && n < kIoDevice) {
+    if (!direct && !io_on_device(c)) {
         const size_t eb = src_f64 ? 8 : 4;
         std::vector<unsigned char> raw(3 * (size_t)n * eb);
         SLLG_HIP(hipMemcpyAsync(raw.data(), src_dev, raw.size(), hipMemcpyDeviceToHost, c->stream));
@@ -181,17 +199,21 @@ int download_state(llg_ctx* c, const void* src_dev, bool src_f64, double* x, dou
         return 0;
     }
     double* const tmp = io_scratch(c);
-    for (int a = 0; a < 3; ++a) {
+    const uint32_t per = c->prec == LLG_FP64_PLAIN ? 3 : 1;
+    const dim3 grid(blocks_for(n, kTPB), per);
+    for (uint32_t a = 0; a < 3; a += per) {
         const double* const s64 = (const double*)src_dev + (size_t)a * n;
         const float* const s32 = (const float*)src_dev + (size_t)a * n;
         if (!direct) {
             if (src_f64)
-                k_to_ref<double><<<blocks_for(n, kTPB), kTPB, 0, c->stream>>>(n, c->perm, s64, tmp);
+                k_to_ref<double><<<grid, kTPB, 0, c->stream>>>(n, c->perm, s64, tmp);
             else
-                k_to_ref<float><<<blocks_for(n, kTPB), kTPB, 0, c->stream>>>(n, c->perm, s32, tmp);
+                k_to_ref<float><<<grid, kTPB, 0, c->stream>>>(n, c->perm, s32, tmp);
             SLLG_HIP(hipGetLastError());
         }
-        SLLG_HIP(hipMemcpyAsync(dst[a], direct ? s64 : tmp, (size_t)n * 8, hipMemcpyDeviceToHost, c->stream));
+        for (uint32_t k = 0; k < per; ++k)
+            SLLG_HIP(hipMemcpyAsync(dst[a + k], (direct ? s64 : tmp) + (size_t)k * n, (size_t)n * 8, hipMemcpyDeviceToHost,
+                                    c->stream));
     }
     SLLG_HIP(hipStreamSynchronize(c->stream));
     return 0;
@@ -603,13 +625,18 @@ int llg_set_staggered(llg_ctx* c, const double* hx, const double* hy, const doub
     if (!hx || !hy || !hz) SLLG_FAIL(LLG_E_INVALID, "staggered field: give all three components or none");
     // H0 stays on the device in FP64 (device order) for llg_scale_staggered; H = 1 * H0
     const double* src[3] = {hx, hy, hz};
-    std::vector<double> h0(3 * (size_t)n);
-    for (uint32_t i = 0; i < n; ++i) {
-        const size_t d = c->perm.to_dev(i);
-        for (int a = 0; a < 3; ++a) h0[(size_t)a * n + d] = src[a][i];
+    if (c->STG0.bytes != 3 * (size_t)n * 8) SLLG_TRY(c->STG0.alloc(3 * (size_t)n * 8));
+    std::vector<double> h0;
+    if (io_on_device(c)) {
+        SLLG_TRY(from_ref<double>(c, src, c->STG0.as<double>()));
+    } else {
+        h0.resize(3 * (size_t)n);
+        for (uint32_t i = 0; i < n; ++i) {
+            const size_t d = c->perm.to_dev(i);
+            for (int a = 0; a < 3; ++a) h0[(size_t)a * n + d] = src[a][i];
+        }
+        SLLG_HIP(hipMemcpyAsync(c->STG0.p, h0.data(), h0.size() * 8, hipMemcpyHostToDevice, c->stream));
     }
-    if (c->STG0.bytes != h0.size() * 8) SLLG_TRY(c->STG0.alloc(h0.size() * 8));
-    SLLG_HIP(hipMemcpyAsync(c->STG0.p, h0.data(), h0.size() * 8, hipMemcpyHostToDevice, c->stream));
     SLLG_TRY(stag_scale(c, 1.0));
     SLLG_HIP(hipStreamSynchronize(c->stream));
     c->stag_set = true;
