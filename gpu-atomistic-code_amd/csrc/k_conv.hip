@@ -295,15 +295,46 @@ __global__ __launch_bounds__(64 * kConvWaves) void k_conv_fwd(ConvArgs a, const 
     }
 }
 
+// Real inverse DFT along z of LY rows, h(z) = dot(X_0, zt_0(z)) + 2 sum_s dot(X_s, zt_s(z)), Z
+// values of z a thread.
+template <int LY, uint32_t Z>
+__device__ __forceinline__ void conv_z(const c2* X, const c2* zt, float* P, uint32_t lz, float scale) {
+    const uint32_t ls = lz + 1u, nz = (lz + Z - 1u) / Z;
+    for (uint32_t e = threadIdx.x; e < LY * nz; e += blockDim.x) {
+        const uint32_t y = e % LY, z0 = e / LY * Z;
+        float h0[Z], h[Z];
+        const c2 x0 = X[y];
+#pragma unroll
+        for (uint32_t q = 0; q < Z; ++q) {
+            h0[q] = x0.x + (((z0 + q) & 1u) ? -x0.y : x0.y);
+            h[q] = 0.f;
+        }
+        for (uint32_t s = 1; s < lz; ++s) {
+            const c2 v = X[s * LY + y];
+#pragma unroll
+            for (uint32_t q = 0; q < Z; ++q) {
+                const c2 u = zt[s * lz + (z0 + q < lz ? z0 + q : lz - 1u)];
+                h[q] += v.x * u.x + v.y * u.y;
+            }
+        }
+#pragma unroll
+        for (uint32_t q = 0; q < Z; ++q)
+            if (z0 + q < lz) P[y * ls + z0 + q] = (h0[q] + 2.f * h[q]) * scale;
+    }
+}
+
 // Inverse plane: the y transforms of the lz sequences (row 0: H_0 + i H_{Gz/2}, whose results
-// are real) into LDS, then per mesh point the real inverse DFT along z,
-// h(z) = dot(X_0, zt_0(z)) + 2 sum_s dot(X_s, zt_s(z)), eight z a thread.
-constexpr uint32_t kConvZ = 8;
+// are real) into LDS by the block's first nw waves, then the z transforms by all of them: eight z
+// a thread, fewer where that would leave threads without any.  With only the nw waves and always
+// eight z a thread, 64 of the 128 threads of a 16 x 16 x 32 mesh carried the serial z sums (13.0
+// us a kernel).  A step with the dipolar field of a 16 x 16 x 32 mesh takes 27.7 us (31.7 before),
+// 64 x 8 x 24 27.3 (31.7), 128 x 128 x 32 78.3 (88.8); with FFT exchange 40.2 (53.1), 40.5 (53.8)
+// and 136 (159); flat meshes stay as they were.
 template <int GY>
-__global__ __launch_bounds__(64 * kConvWaves) void k_conv_inv(ConvArgs a, float scale, float* __restrict__ H) {
+__global__ __launch_bounds__(64 * kConvWaves) void k_conv_inv(ConvArgs a, uint32_t nw, float scale, float* __restrict__ H) {
     constexpr int R = fft_r(GY), T = fft_t(GY), C = fft_cols(GY), LY = GY / 2;
     extern __shared__ c2 conv_lds[];
-    const uint32_t nt = blockDim.x, nw = nt / 64u, lz = a.lz, ls = lz + 1u;
+    const uint32_t nt = blockDim.x, lz = a.lz;
     c2* const zt = conv_lds;                          // lz lz
     c2* const X = zt + lz * lz;                       // lz sequences of LY
     c2* const exch = X + lz * LY;                     // nw C sequences, then the plane's field
@@ -315,7 +346,7 @@ __global__ __launch_bounds__(64 * kConvWaves) void k_conv_inv(ConvArgs a, float 
     load_tw<GY>(w, a.twy, t);
     c2* const ex = exch + (wave * C + col) * fft_lds(GY);
     const c2* const in = a.spec + ((size_t)c * a.lx + x) * lz * GY;
-    for (uint32_t s0 = wave * C; s0 < lz; s0 += nw * C) {
+    for (uint32_t s0 = wave < nw ? wave * C : lz; s0 < lz; s0 += nw * C) {
         const bool on = s0 + col < lz;
         const uint32_t s = on ? s0 + col : lz - 1u;
         const c2* const row = in + (size_t)s * GY;
@@ -334,28 +365,14 @@ __global__ __launch_bounds__(64 * kConvWaves) void k_conv_inv(ConvArgs a, float 
         }
     }
     __syncthreads();
-    const uint32_t nz = (lz + kConvZ - 1) / kConvZ;
-    for (uint32_t e = threadIdx.x; e < LY * nz; e += nt) {
-        const uint32_t y = e % LY, z0 = e / LY * kConvZ;
-        float h0[kConvZ], h[kConvZ];
-        const c2 x0 = X[y];
-#pragma unroll
-        for (uint32_t q = 0; q < kConvZ; ++q) {
-            h0[q] = x0.x + (((z0 + q) & 1u) ? -x0.y : x0.y);
-            h[q] = 0.f;
-        }
-        for (uint32_t s = 1; s < lz; ++s) {
-            const c2 v = X[s * LY + y];
-#pragma unroll
-            for (uint32_t q = 0; q < kConvZ; ++q) {
-                const c2 u = zt[s * lz + (z0 + q < lz ? z0 + q : lz - 1u)];
-                h[q] += v.x * u.x + v.y * u.y;
-            }
-        }
-#pragma unroll
-        for (uint32_t q = 0; q < kConvZ; ++q)
-            if (z0 + q < lz) P[y * ls + z0 + q] = (h0[q] + 2.f * h[q]) * scale;
-    }
+    if (LY * ((lz + 7u) / 8u) >= nt)
+        conv_z<LY, 8>(X, zt, P, lz, scale);
+    else if (LY * ((lz + 3u) / 4u) >= nt)
+        conv_z<LY, 4>(X, zt, P, lz, scale);
+    else if (LY * ((lz + 1u) / 2u) >= nt)
+        conv_z<LY, 2>(X, zt, P, lz, scale);
+    else
+        conv_z<LY, 1>(X, zt, P, lz, scale);
     __syncthreads();
     const uint32_t i0 = x * pts;
     for (uint32_t e = threadIdx.x; e < pts; e += nt) {
@@ -653,7 +670,7 @@ void launch_plane(bool fwd, const ConvArgs& a, const float* S, float scale, floa
     if (fwd)
         k_conv_fwd<GY><<<3 * a.lx, nw * 64, lds, s>>>(a, S);
     else
-        k_conv_inv<GY><<<3 * a.lx, nw * 64, lds, s>>>(a, scale, H);
+        k_conv_inv<GY><<<3 * a.lx, kConvWaves * 64, lds, s>>>(a, nw, scale, H);
 }
 
 template <int GX>
