@@ -5,7 +5,7 @@
 // cycles whatever its addresses: 42 of them a row are half of its time.  Here a workgroup takes
 // a few consecutive lines of every sublattice (build_blocks, encode.hip), stages the lines they
 // couple to once in LDS, each with the cells that wrap around its ends, and reads neighbours
-// from there.  In the staged layout an entry's neighbour is the same number of bytes away from
+// from there (which of the readers a new handle takes: blocks_pay, encode.hip).  In the staged layout an entry's neighbour is the same number of bytes away from
 // every row of the workgroup's sublattice, so the entry stream is lane-uniform (scalar loads:
 // offset and couplings of four entries a record) where the packed reader loads a word a lane.
 // Rows keep their entries' order, so the sums have the packed reader's bits.

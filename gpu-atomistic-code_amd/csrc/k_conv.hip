@@ -5,9 +5,11 @@
 //
 //   N_ab(r) = N_ba(r),  N_ab(.., -r_d, ..) = s N_ab(.., r_d, ..),  s = -1 if exactly one of a, b is d.
 //
-// Its transform is then real with the same mirror symmetry in k, so 6 components on one octant
-// (kx <= Gx/2, ky <= Gy/2, kz <= Gz/2) hold all of it: 6.8 MB for the 128 x 128 x 16 film instead
-// of 26.7 MB (the whole x range) or 80 MB (nine complex components).  Gx and Gy are the powers
+// Its transform is then real with the same mirror symmetry in k, so one octant (kx <= Gx/2, ky <=
+// Gy/2, kz <= Gz/2) holds all of it.  It is stored as [kx][kz][ky][3][3], both triangles, so that
+// the wave of one component reads its row as three neighbouring floats: 10.2 MB for the 128 x
+// 128 x 16 film (six components would be 6.8) instead of 26.7 MB (six real components over the whole
+// kx range) or 80 MB (nine complex ones).  Gx and Gy are the powers
 // of two of at least twice the extents: a linear convolution may be padded further, so extents
 // that are no powers of two take this path too.  Gz is twice the extent: z is transformed
 // directly.
@@ -27,9 +29,11 @@
 // The radix-2 form they replaced made four LDS passes and a block barrier a pass per transform
 // and was bound by them (about 20 LDS accesses a point and x transform against 4 here).
 // 128 x 128 x 16 film (trace durations): forward planes 16.1 -> 9.3 us, x 25.4 -> 15.8 us (26.3
-// with the complex FFT-exchange kernel), inverse planes 13.4 -> 9.6 us.  The three move 55 MB
-// (11 us at copy rate); a film's 1,024 to 1,536 waves of work give each SIMD one or two, so load
-// latency and the last wave are what is left.  100 x 84 x 12 (padded to 256 x 256 x 24, 200 x
+// with the complex FFT-exchange kernel), inverse planes 13.4 -> 9.6 us.  The three move 67 MB,
+// the kernel's 10 included (13 us at copy rate).  A film's 1,024 to 1,536 waves of work are 1.5 a
+// SIMD in the plane kernels and 2.6 in the x kernel, and busy CUs issue VALU work 44, 58 and 44 %
+// of their time (forward, x, inverse): waves wait for data (about 40 % of their lives), and in the
+// x kernel a third of the CUs' time goes to LDS bank conflicts of the exchange.  100 x 84 x 12 (padded to 256 x 256 x 24, 200 x
 // 168 x 24 with hipFFT and the scatter, product and gather kernels): 102 -> 35 us a
 // refresh.
 #include <algorithm>

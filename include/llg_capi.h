@@ -334,7 +334,8 @@ void* llg_stream(llg_ctx* ctx);
 
 /* Per-kernel timing: runs nsteps steps with HIP events around every launch and
  * returns the mean duration (ms) of each kernel kind.  names receives up to
- * max_kinds NUL-terminated names of up to 47 chars (48 bytes each). */
+ * max_kinds NUL-terminated names of up to 47 chars (48 bytes each).  Systems small enough
+ * for one workgroup report "heun_steps", one launch of up to 1,024 steps. */
 int llg_profile_kernels(llg_ctx* ctx, uint64_t t0, uint32_t nsteps, int max_kinds,
                         char* names, double* mean_ms, int* n_kinds);
 
@@ -345,11 +346,11 @@ int llg_profile_kernels(llg_ctx* ctx, uint64_t t0, uint32_t nsteps, int max_kind
  * (packed and line encodings) with neighbours gathered from the SoA spins or from an AoS3
  * copy the kernels keep beside them (bit-identical either way), and (line encodings) with
  * the line reader or the packed entries kept beside the line stream (same couplings, sums
- * in another order), on this handle's own couplings, for nsteps steps each; keeps the
- * fastest.
+ * in another order), and with line blocks where the encoding has them (the packed entries'
+ * bits), on this handle's own couplings, for nsteps steps each; keeps the fastest.
  * The spin state is restored afterwards.  Results are cached per (device, encoding, n,
- * entries) in the process and, if the environment variable SLLG_TUNE_FILE names a file,
- * across processes.  Other paths return LLG_OK with the defaults. */
+ * entries, shape of the line blocks and what else a step holds) in the process and, if the
+ * environment variable SLLG_TUNE_FILE names a file, across processes.  Other paths return LLG_OK with the defaults. */
 typedef struct llg_tune_result {
     int tpb, xcd;
     double ms_per_step;     /* chosen (one-workgroup steps where the system takes them) */
